@@ -41,17 +41,20 @@
 //   - Split-K (the core-template entry point with splitK > 1): each split writes fp32 partials
 //     to the library workspace; a second kernel sums them in split order and applies
 //     alpha/beta (deterministic; the reference accumulates with lossy bf16 atomics).
-// Shapes the tiled kernel does not take (a contiguous extent or leading dimension that is not
-// a multiple of 8, pointers not 16-byte aligned) run on a simple fp32-accumulating kernel.
+// Products of few such tiles and operands whose rows are no whole 16-byte vectors run on the tiles of
+// bgemm_flex.hip (make_plan); leading dimensions those do not take either, and K == 0, on a simple
+// fp32-accumulating kernel.
 #include <mutex>
 #include <type_traits>
 
-#include "hk_device.h"
-#include "hk_host.h"
+#include "bgemm_flex.h"
+#include "bgemm_tile.h"
 
 namespace {
 
-constexpr int BM = 256, BN = 256, BK = 64;             // BN: the full tile width
+using namespace hk::gemm;
+
+constexpr int BM = 256, BN = 256;                      // BN: the full tile width
 constexpr int kStages = 2;                             // LDS ring depth (k-tiles)
 constexpr int kWaves = 8;                              // 2 x 4 over the tile, 2 per SIMD
 constexpr int kThreads = kWaves * 64;
@@ -78,244 +81,6 @@ struct TileN {
   static constexpr int kLoadsB = kStageBytesB / 1024 / kWaves;
   static constexpr size_t kLdsBytes =
       static_cast<size_t>(kStages) * (TileM<BMT>::kStageBytes + kStageBytesB);
-};
-
-typedef short bf16x8_t __attribute__((ext_vector_type(8)));
-typedef short bf16x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-#define HK_LDS __attribute__((address_space(3)))
-
-// 16-byte global -> LDS copy of one lane (global_load_lds_dwordx4): the wave's 64 lanes write
-// 1 KiB of LDS at m0 + 16 * lane. Written as inline asm on purpose: for the builtin, the
-// compiler assumes every later LDS read may alias the copy and waits for ALL of them to land
-// before any LDS read, which would serialise the load pipeline against the MFMA loop. Here the
-// kernel waits for the copies itself (vmcnt) before the barrier that publishes a stage.
-// Address = sbase (wave-uniform 64-bit, SGPRs) + voff (per-lane byte offset).
-__device__ __forceinline__ void copy16_to_lds(const void* sbase, int voff, unsigned lds_addr) {
-  // m0 (the LDS destination) is an input operand, so the compiler knows the asm sets it. Its
-  // hazard checks do not see inside the asm, so the asm supplies the wait states itself: an
-  // SALU write of m0 needs 1 before an LDS-DMA load, and an SGPR of sbase written by a VALU
-  // (v_readlane, when the compiler reloads a spilled SGPR) needs 5 before a VMEM read of it.
-  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase),
-               "{m0}"(lds_addr));
-}
-
-// One operand of a k-tile in LDS: 256 rows of M (or N) by BK = 64 k, bf16, 32 KiB.
-//
-// gfx950's LDS has 64 banks of 4 bytes: a ds_read_b128 is served 16 lanes (256 bytes) per
-// cycle and a ds_read_b64(_tr) 32 lanes per cycle, so each such lane group must cover all 64
-// banks once (a 2-way conflict halves the read rate; measured 134 against 222 B/clk/CU).
-//
-// K-major operands (element (row, k) at base[row * ld + k]) are stored [row][64 k]: 128-byte
-// rows whose eight 16-byte chunks sit at chunk ^ ((row >> 1) & 7). A wave's copy instruction
-// moves 8 rows (lane l: row l / 8, stored chunk l % 8, which is global chunk
-// (l % 8) ^ ((row >> 1) & 7), so each row's 128 contiguous bytes are read by 8 lanes). The
-// MFMA operand of a lane is 8 consecutive k of one row, one ds_read_b128; the 16 lanes of one
-// read cycle take 16 consecutive rows at one logical chunk: the even rows fill one 128-byte
-// bank half at 8 distinct chunk positions and the odd rows the other.
-//
-// M/N-major operands (element at base[k * ld + row]) are stored as in HBM, [64 k][256 rows]:
-// 512-byte k-rows (256 bytes for a 128-wide B tile) whose 16-byte chunk c sits at
-// c ^ (2 * (krow & 3)) ^ (8 * ((c >> 1) & 1)). Both row pitches are whole multiples of the 64
-// banks, so a chunk's banks depend on its stored position mod 16 alone and the placement below
-// holds for both. A copy instruction moves 2 k-rows (4 for 256-byte rows; 32 or 16 lanes read
-// one contiguous row segment). The
-// MFMA operand (8 consecutive k of one row/column) is gathered with two ds_read_b64_tr_b16:
-// within each 16-lane group, lane j reads 4 bf16 of k-row kb + j / 4 at columns
-// c0 + 4 (j % 4) and the hardware transposes the 16 x 4 block so lane i receives column
-// c0 + i, k = kb .. kb + 3. One group covers 4 k-rows x 32 bytes, which the (krow & 3) term
-// spreads over 32 banks; the two groups of a read cycle sit 16 columns (2 chunks) apart and
-// the (c >> 1) term places them in opposite bank halves.
-template <bool KMAJOR, int ROWS = 256>
-struct TileOperand {
-  // M/N-major: a copy instruction (1 KiB) covers kRowsPerCopy k-rows of ROWS * 2 bytes.
-  static constexpr int kKRowBytes = ROWS * 2;
-  static constexpr int kRowsPerCopy = 1024 / kKRowBytes;
-  static constexpr int kLanesPerRow = 64 / kRowsPerCopy;
-  // M/N-major: stored position of logical 16-byte chunk c of k-row krow, and its inverse.
-  __device__ static int stored_chunk(int c, int krow) {
-    return c ^ (2 * (krow & 3)) ^ (8 * ((c >> 1) & 1));
-  }
-  __device__ static int logical_chunk(int p, int krow) {
-    return p ^ (8 * (((p >> 1) ^ krow) & 1)) ^ (2 * (krow & 3));
-  }
-  // Byte offset of lane `lane`'s 16 bytes of copy instruction ii (0 .. 31) from the tile's
-  // global base at k = 0, and the (row, k) of its first element.
-  __device__ static void source(int ii, int lane, int& row, int& k) {
-    if (KMAJOR) {
-      row = ii * 8 + (lane >> 3);
-      k = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
-    } else {
-      k = ii * kRowsPerCopy + lane / kLanesPerRow;
-      row = logical_chunk(lane % kLanesPerRow, k) * 8;
-    }
-  }
-  __device__ static int64_t byte_offset(int row, int k, int64_t ld) {
-    return KMAJOR ? 2 * (static_cast<int64_t>(row) * ld + k)
-                  : 2 * (static_cast<int64_t>(k) * ld + row);
-  }
-  // Global step of one k-tile (elements).
-  __device__ static int64_t ktile_step(int64_t ld) { return KMAJOR ? BK : BK * ld; }
-  // LDS byte offset of the MFMA operand of MFMA block b (32 rows at wave offset wo),
-  // 16-deep k step s; `half` selects the second 4-k read of an M/N-major operand.
-  __device__ static int frag(int wo, int b, int s, int half, int lane) {
-    if (KMAJOR) {
-      const int row = wo + b * 32 + (lane & 31);
-      const int c = 2 * s + (lane >> 5);
-      return row * 128 + ((c ^ ((row >> 1) & 7)) * 16);
-    } else {
-      const int g = lane >> 4, j = lane & 15;
-      const int col = wo + b * 32 + 16 * (g & 1) + 4 * (j & 3);
-      const int krow = 16 * s + 8 * (g >> 1) + (j >> 2) + 4 * half;
-      return krow * kKRowBytes + stored_chunk(col >> 3, krow) * 16 + (col & 7) * 2;
-    }
-  }
-  __device__ static bf16x8_t read(const unsigned char HK_LDS* st, int wo, int b, int s,
-                                  int lane) {
-    if (KMAJOR) {
-      return *reinterpret_cast<const bf16x8_t HK_LDS*>(st + frag(wo, b, s, 0, lane));
-    } else {
-      const bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (bf16x4_t HK_LDS*)(st + frag(wo, b, s, 0, lane)));
-      const bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (bf16x4_t HK_LDS*)(st + frag(wo, b, s, 1, lane)));
-      return bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    }
-  }
-};
-
-// Linear tile id t -> (tile_m, tile_n): consecutive ids to one XCD, grouped 8 tile-rows. The
-// hardware deals workgroups to the 8 XCDs round-robin, so t % 8 is the XCD when t is a
-// workgroup id or one offset by a multiple of 8.
-__device__ __forceinline__ void tile_coords(int t, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  if ((total & 7) == 0) t = (t & 7) * (total >> 3) + (t >> 3);
-  constexpr int G = 8;
-  const int per_group = G * tiles_n;
-  const int group = t / per_group;
-  const int first_m = group * G;
-  const int gsz = min(tiles_m - first_m, G);
-  const int in_group = t - group * per_group;
-  tm = first_m + in_group % gsz;
-  tn = in_group / gsz;
-}
-
-// Output transform: C = alpha * acc + beta * C, or, with a bias (bias != NULL),
-// C = alpha * acc + beta * bias and C is written without being read. The bias element of
-// output (row, col) is bias[row * brow + col * bcol]: (brow, bcol) = (0, 1) for a per-column
-// bias (numel N), (1, 0) per row (numel M), (0, 0) scalar (numel 1), (N, 1) full (numel M*N,
-// the same for every batch).
-struct Epi {
-  float alpha, beta;
-  const uint16_t* bias;
-  int64_t brow, bcol;
-};
-
-__device__ __forceinline__ float bias_at(const Epi& ep, int row, int col) {
-  return hk::bf16_to_f32(ep.bias[row * ep.brow + col * ep.bcol]);
-}
-
-// Bias element of column col of batch b for an fp32 output (hk::F32Out).
-__device__ __forceinline__ float f32out_bias(const hk::F32Out& fo, int M, int N, int b, int col) {
-  if (fo.bias_stride == N) return fo.bias[col];
-  if (fo.bias_stride == static_cast<int64_t>(M) * N)
-    return fo.bias[static_cast<int64_t>(b % M) * N + col];
-  if (fo.bias_stride == 1) return fo.bias[0];
-  return 0.f;
-}
-
-// Scheduling hint: NR LDS reads spread over NM MFMAs (reads first in each pair), so the
-// operands of the next k step are fetched while the current one multiplies.
-template <int NM, int NR, int Q = 0>
-__device__ __forceinline__ void interleave_reads() {
-  if constexpr (Q < NM) {
-    constexpr int per = (NR + NM - 1) / NM;
-    constexpr int left = NR - Q * per;
-    constexpr int n = left <= 0 ? 0 : (left < per ? left : per);
-    if constexpr (n > 0) __builtin_amdgcn_sched_group_barrier(0x100, n, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    interleave_reads<NM, NR, Q + 1>();
-  }
-}
-
-// Hands the accumulators of a wave to `out` through LDS, one 32-row MFMA block row at a time:
-// the wave stores its block row into its own fp32 staging area (32 rows, pitch kWaveN * 4 + 16
-// bytes, so the 16 lanes of one 16-byte write cycle start 4 banks apart) and reads it back as 8
-// consecutive columns per lane: out(row, col, a, b) gets the wave-relative row and column of
-// values a[0..3], b[0..3], and kWaveN / 8 consecutive lanes hold one row segment, so the
-// outputs can be written 16 (bf16) or 32 (fp32) bytes per lane in whole lines. Stored straight
-// from the MFMA layout instead, every store touched 32 rows and each 128-byte line of C was
-// assembled from 8 stores (bf16): 23% of the BASELINE product. The area is the wave's own, so
-// it needs no barrier beyond the one that ends the main loop.
-template <int kWaveN, int kBlkM, typename Out>
-__device__ __forceinline__ void staged_rows(const f32x16_t (&acc)[kBlkM][kWaveN / 32],
-                                            unsigned char HK_LDS* area, int lane, Out&& out) {
-  constexpr int kBlkN = kWaveN / 32;
-  constexpr int P = kWaveN * 4 + 16;        // staging pitch (bytes)
-  constexpr int LPR = kWaveN / 8;           // lanes per row
-  constexpr int RPP = 64 / LPR;             // rows per pass
-  const int r = lane & 31, h = lane >> 5;
-  const int rr0 = lane / LPR, cc = (lane % LPR) * 8;
-#pragma unroll
-  for (int i = 0; i < kBlkM; ++i) {
-#pragma unroll
-    for (int j = 0; j < kBlkN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<f32x4_t HK_LDS*>(area + r * P + (32 * j + 8 * q + 4 * h) * 4) =
-            f32x4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                    acc[i][j][4 * q + 3]};
-#pragma unroll
-    for (int p = 0; p < 32 / RPP; ++p) {
-      const int rr = p * RPP + rr0;
-      const f32x4_t a = *reinterpret_cast<const f32x4_t HK_LDS*>(area + rr * P + cc * 4);
-      const f32x4_t b = *reinterpret_cast<const f32x4_t HK_LDS*>(area + rr * P + cc * 4 + 16);
-      out(32 * i + rr, cc, a, b);
-    }
-  }
-}
-
-// The bf16 epilogue on staged rows: C = alpha * acc + beta * C (or + beta * bias) in fp32,
-// one rounding to bf16 (v_cvt_pk_bf16_f32, round to nearest even), 16-byte stores.
-template <bool BIAS>
-struct Bf16RowOut {
-  const Epi& ep;
-  uint16_t* Cb;
-  int64_t ldc;
-  int M, N, wrow0, wcol0;
-  __device__ void operator()(int rr, int cc, const f32x4_t& a, const f32x4_t& b) const {
-    const int row = wrow0 + rr, col = wcol0 + cc;
-    if (row >= M || col >= N) return;  // N % 8 == 0: the 8 columns are all in or all out
-    f32x2_t v[4] = {f32x2_t{a[0], a[1]} * ep.alpha, f32x2_t{a[2], a[3]} * ep.alpha,
-                    f32x2_t{b[0], b[1]} * ep.alpha, f32x2_t{b[2], b[3]} * ep.alpha};
-    uint4* dst = reinterpret_cast<uint4*>(Cb + static_cast<int64_t>(row) * ldc + col);
-    if (BIAS) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] += ep.beta * f32x2_t{bias_at(ep, row, col + 2 * e), bias_at(ep, row, col + 2 * e + 1)};
-    } else if (ep.beta != 0.0f) {
-      const uint4 old = *dst;
-      const uint32_t o[4] = {old.x, old.y, old.z, old.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] += ep.beta * f32x2_t{__uint_as_float(o[e] << 16), __uint_as_float(o[e] & 0xffff0000u)};
-    }
-    uint32_t w[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bf16x2_t bv = __builtin_convertvector(v[e], bf16x2_t);
-      __builtin_memcpy(&w[e], &bv, 4);
-    }
-    // non-temporal: C is not read again by this product, and keeping it out of the caches
-    // leaves them to the operands (8192^3 NN: 742 -> 714 us on MI355X). The fp32 split-K
-    // partials below are read back by the finalize kernel and keep ordinary stores (with
-    // non-temporal ones the 8192 x 1280 x 5120 dA product went from 130 to 149 us).
-    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(u32x4_t{w[0], w[1], w[2], w[3]}, reinterpret_cast<u32x4_t*>(dst));
-  }
 };
 
 // Main loop per k-tile kt (ring slot kt % 2), 4 k steps of 16 MFMAs each:
@@ -536,45 +301,18 @@ __device__ __forceinline__ void tile_body(
   const int wrow0 = m0 + wm * kWaveM, wcol0 = n0 + wn * kWaveN;
   if (PARTIAL && fo.C) {
     // one split: fp32 C with alpha, beta and the bias applied here
-    float* cb = fo.C + static_cast<int64_t>(batch) * fo.sC;
-    staged_rows<kWaveN, kBlkM>(acc, area, lane, [&](int rr, int cc, const f32x4_t& a, const f32x4_t& b) {
-      const int row = wrow0 + rr, col = wcol0 + cc;
-      if (row >= M || col >= N) return;  // N % 8 == 0
-      f32x4_t* dst = reinterpret_cast<f32x4_t*>(cb + static_cast<int64_t>(row) * fo.ldc + col);
-      f32x4_t v0 = fo.alpha * a, v1 = fo.alpha * b;
-      if (fo.beta != 0.0f) {
-        v0 += fo.beta * dst[0];
-        v1 += fo.beta * dst[1];
-      }
-      if (fo.bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v0[e] += fo.bias_scale * f32out_bias(fo, M, N, batch, col + e);
-          v1[e] += fo.bias_scale * f32out_bias(fo, M, N, batch, col + 4 + e);
-        }
-      }
-      dst[0] = v0;
-      dst[1] = v1;
-    });
+    store_f32<kWaveN, kBlkM>(acc, area, lane, fo, batch, M, N, wrow0, wcol0);
     return;
   }
   if (PARTIAL) {
-    float* out = part + (static_cast<int64_t>(split) * (gridDim.z / split_k) + batch) *
-                            static_cast<int64_t>(M) * N;
-    staged_rows<kWaveN, kBlkM>(acc, area, lane, [&](int rr, int cc, const f32x4_t& a, const f32x4_t& b) {
-      const int row = wrow0 + rr, col = wcol0 + cc;
-      if (row >= M || col >= N) return;
-      f32x4_t* dst = reinterpret_cast<f32x4_t*>(out + static_cast<int64_t>(row) * N + col);
-      dst[0] = a;
-      dst[1] = b;
-    });
+    store_partial<kWaveN, kBlkM>(
+        acc, area, lane,
+        part + (static_cast<int64_t>(split) * (gridDim.z / split_k) + batch) * M * part_pitch(N), M,
+        N, wrow0, wcol0);
     return;
   }
   uint16_t* Cb = C + static_cast<int64_t>(batch) * sC;
-  if (ep.bias)
-    staged_rows<kWaveN, kBlkM>(acc, area, lane, Bf16RowOut<true>{ep, Cb, ldc, M, N, wrow0, wcol0});
-  else
-    staged_rows<kWaveN, kBlkM>(acc, area, lane, Bf16RowOut<false>{ep, Cb, ldc, M, N, wrow0, wcol0});
+  store_bf16<kWaveN, kBlkM>(acc, area, lane, ep, Cb, ldc, M, N, wrow0, wcol0);
 }
 
 // One column region: workgroup x takes tile x.
@@ -815,27 +553,34 @@ __global__ __launch_bounds__(kThreads, 1) void bgemm_nt_w160(
       }
     }
   };
-  if (ep.bias)
+  if (ep.ragged) {
+    if (ep.bias)
+      emit(Bf16RowOut<true, true>{ep, Cb, ldc, M, N, wrow0, wcol0});
+    else
+      emit(Bf16RowOut<false, true>{ep, Cb, ldc, M, N, wrow0, wcol0});
+  } else if (ep.bias) {
     emit(Bf16RowOut<true>{ep, Cb, ldc, M, N, wrow0, wcol0});
-  else
+  } else {
     emit(Bf16RowOut<false>{ep, Cb, ldc, M, N, wrow0, wcol0});
+  }
 }
 
-// C = alpha * sum_s part[s] + beta * C (split order), fp32 -> bf16.
-// I: the index type, uint32_t when every index of the launch fits in 31 bits (a 64-bit
-// division costs several times a 32-bit one).
+// C = alpha * sum_s part[s] + beta * C or + beta * bias (split order), fp32 -> bf16, four
+// consecutive outputs per thread. I: the index type, uint32_t when every index of the launch fits
+// in 31 bits (a 64-bit division costs several times a 32-bit one).
 template <typename I>
 __global__ __launch_bounds__(256) void bgemm_splitk_finalize(const float* __restrict__ part,
                                                              int split_k, int batch, int M, int N,
                                                              Epi ep, uint16_t* __restrict__ C,
                                                              int64_t ldc, int64_t sC) {
-  // 4 consecutive outputs per thread (N is a multiple of 8 on the tiled path)
   const I idx = (static_cast<I>(blockIdx.x) * 256 + threadIdx.x) * 4;
-  const I mn = static_cast<I>(M) * N;
+  const I pitch = part_pitch(N), mn = static_cast<I>(M) * pitch;
   if (idx >= mn * batch) return;
   const I b = idx / mn;
   const I e = idx - b * mn;
-  const int row = static_cast<int>(e / N), col = static_cast<int>(e - static_cast<I>(row) * N);
+  const int row = static_cast<int>(e / pitch);
+  const int col = static_cast<int>(e - static_cast<I>(row) * pitch);
+  if (col >= N) return;
   f32x2_t lo = f32x2_t{0.f, 0.f}, hi = f32x2_t{0.f, 0.f};
   for (int k = 0; k < split_k; ++k) {
     const float4 v = *reinterpret_cast<const float4*>(part + (static_cast<int64_t>(k) * batch + b) * mn + e);
@@ -844,7 +589,20 @@ __global__ __launch_bounds__(256) void bgemm_splitk_finalize(const float* __rest
   }
   lo *= ep.alpha;
   hi *= ep.alpha;
-  uint2* dst = reinterpret_cast<uint2*>(C + b * sC + static_cast<int64_t>(row) * ldc + col);
+  uint16_t* cp = C + b * sC + static_cast<int64_t>(row) * ldc + col;
+  if (ep.ragged) {  // rows of C at any 2-byte address, columns past N not stored
+    const float f[4] = {lo[0], lo[1], hi[0], hi[1]};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (col + i >= N) break;
+      float v = f[i];
+      if (ep.bias) v += ep.beta * bias_at(ep, row, col + i);
+      else if (ep.beta != 0.0f) v += ep.beta * hk::bf16_to_f32(cp[i]);
+      cp[i] = hk::f32_to_bf16(v);
+    }
+    return;
+  }
+  uint2* dst = reinterpret_cast<uint2*>(cp);
   if (ep.bias) {
     lo += ep.beta * f32x2_t{bias_at(ep, row, col), bias_at(ep, row, col + 1)};
     hi += ep.beta * f32x2_t{bias_at(ep, row, col + 2), bias_at(ep, row, col + 3)};
@@ -860,6 +618,20 @@ __global__ __launch_bounds__(256) void bgemm_splitk_finalize(const float* __rest
   __builtin_memcpy(&v.x, &blo, 4);
   __builtin_memcpy(&v.y, &bhi, 4);
   *dst = v;
+}
+
+hipError_t launch_splitk_finalize(hipStream_t stream, const float* part, int used, int batch,
+                                         int M, int N, const Epi& ep, uint16_t* C, int64_t ldc,
+                                         int64_t sC) {
+  const int64_t total = static_cast<int64_t>(M) * part_pitch(N) * batch;
+  const dim3 grid(static_cast<unsigned>(hk::ceil_div(total, 1024)));
+  if (total < (int64_t{1} << 31))
+    hipLaunchKernelGGL(bgemm_splitk_finalize<uint32_t>, grid, dim3(256), 0, stream, part, used,
+                       batch, M, N, ep, C, ldc, sC);
+  else
+    hipLaunchKernelGGL(bgemm_splitk_finalize<int64_t>, grid, dim3(256), 0, stream, part, used,
+                       batch, M, N, ep, C, ldc, sC);
+  return hk::launch_status();
 }
 
 // Fallback: one thread per output, fp32 accumulation in k order.
@@ -1073,7 +845,7 @@ hipError_t run_regions(bool ta, bool tb, int grid_z, hipStream_t stream, int M, 
 // Calibrated on the 8192 x 1280 x 5120 and 1280 x 5120 x 8192 products (160 and 100 tiles):
 // measured 123 / 149 / 131 us at 1 / 2 / 3 splits for the first, 120 / 115 / 151 / 137 / 135
 // us at 1 to 5 for the second; the model picks 1 and 2.
-int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs) {
+int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs, double* best_cost) {
   const int64_t cus = hk::device_cu_count();
   auto t_kt = [&](int64_t busy) {
     const double f = static_cast<double>(busy) / static_cast<double>(cus);
@@ -1097,25 +869,66 @@ int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs) {
       best_s = s;
     }
   }
+  if (best_cost) *best_cost = best;
   return best_s;
 }
 
-// Whether a product takes the 256 x 256 MFMA tiles (else the fp32-accumulating bgemm_simple):
-// 8-element multiples for every contiguous extent, leading dimension and batch stride, 16-byte
-// aligned bases, and leading dimensions whose per-lane 32-bit byte offsets fit.
-bool tiled_path(bool ta, bool tb, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-                int64_t sA, int64_t sB, int64_t sC, bool aligned) {
+// What the rows of a product's matrices are, as the kernels see them.
+enum class Rows {
+  kAligned,  // whole 16-byte vectors: 8-element multiples for every contiguous extent, leading
+             // dimension and batch stride, 16-byte aligned bases
+  kRaggedC,  // A and B like that, C at any 2-byte address and any N
+  kRagged,   // any 2-byte address, any extent
+  kNone      // no MFMA path: no k, a leading dimension whose per-lane 32-bit byte offsets do not
+             // fit, or one under 8 (a vector could leave the matrix)
+};
+Rows row_kind(bool ta, bool tb, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+              int64_t sA, int64_t sB, int64_t sC, bool a16, bool b16, bool c16) {
+  if (K <= 0 || lda >= (1 << 22) || ldb >= (1 << 22)) return Rows::kNone;
   const int contig_a = ta ? M : K, contig_b = tb ? K : N;
-  return (contig_a % 8 == 0) && (contig_b % 8 == 0) && (N % 8 == 0) && (lda % 8 == 0) &&
-         (ldb % 8 == 0) && (ldc % 8 == 0) && (sA % 8 == 0) && (sB % 8 == 0) &&
-         (sC % 8 == 0) && aligned && K > 0 && lda < (1 << 22) && ldb < (1 << 22);
+  const bool ab = contig_a % 8 == 0 && contig_b % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
+                  sA % 8 == 0 && sB % 8 == 0 && a16 && b16;
+  if (!ab) return lda >= 8 && ldb >= 8 ? Rows::kRagged : Rows::kNone;
+  return N % 8 == 0 && ldc % 8 == 0 && sC % 8 == 0 && c16 ? Rows::kAligned : Rows::kRaggedC;
+}
+// The same for contiguous, 16-byte aligned operands (the planning queries).
+Rows packed_rows(bool ta, bool tb, int M, int N, int K) {
+  const int64_t lda = ta ? M : K, ldb = tb ? K : N;
+  return row_kind(ta, tb, M, N, K, lda, ldb, N, lda * (ta ? K : M), ldb * (tb ? N : K),
+                  static_cast<int64_t>(M) * N, true, true, true);
 }
 
-// Number of k splits the tiled path runs for a product (split_k == 0: the library's choice).
-int tiled_splits(int M, int N, int K, int batch, int split_k) {
-  int used = 1, kps = 0;
-  hk::bgemm_split_plan(M, N, K, batch, split_k, &used, &kps);
-  return used;
+// How a product runs: on the 256-wide tiles (flex == 0) or on tile shape `flex` of
+// bgemm_flex.hip, in `used` k splits of kps.
+struct Plan {
+  int flex, used, kps;
+};
+
+// Modelled time (us) of the 256-wide tiles' plan for one k split (auto_split_k covers the others),
+// with the tile shape run_regions picks.
+double wide_cost(bool ta, bool tb, int M, int N, int K, int batch, int splits, double split_cost) {
+  if (splits > 1) return split_cost;
+  const double kt = static_cast<double>(hk::ceil_div(K, BK));
+  if (w160_plan(ta, tb, M, N, K, batch, 1)) return 8.0 + 0.99 * kt;
+  if (row_tile(ta, M, N, batch, 1) == 192) return 8.0 + (split_cost - 8.0) * 0.85;
+  return split_cost;
+}
+
+// The library's choice between the two families (split_k == 0): the smaller modelled time, the
+// 256-wide tiles kept unless the other is 5% faster. An explicit split keeps the 256-wide tiles
+// where they take the operands.
+Plan make_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_k, Rows rows) {
+  const bool ragged = rows == Rows::kRagged;
+  Plan wide{0, 1, K};
+  double cost = 0.0;
+  if (!ragged) {
+    hk::bgemm_split_plan(M, N, K, batch, split_k, &wide.used, &wide.kps, &cost);
+    if (split_k > 0) return wide;
+    cost = wide_cost(ta, tb, M, N, K, batch, wide.used, cost);
+  }
+  const hk::FlexPlan f = hk::bgemm_flex_plan(M, N, K, batch, split_k, ragged);
+  if (!ragged && f.cost > 0.95 * cost) return wide;
+  return Plan{f.tile, f.used, f.kps};
 }
 
 // bias == NULL: C = alpha * op(A) op(B) + beta * C. Otherwise C = alpha * op(A) op(B) +
@@ -1143,7 +956,7 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
     return hk::bgemv_run(!ta, M, K, alpha_bits, beta_bits, A, lda, strideA, B, tb ? 1 : ldb,
                          strideB, C, ldc, strideC, batchCount, stream);
   }
-  Epi ep{bf16_bits_to_float(alpha_bits), bf16_bits_to_float(beta_bits), bias, 0, 0};
+  Epi ep{bf16_bits_to_float(alpha_bits), bf16_bits_to_float(beta_bits), bias, 0, 0, false};
   if (bias) {
     if (bias_numel == N) ep.bcol = 1;
     else if (bias_numel == M) ep.brow = 1;
@@ -1152,10 +965,9 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
     else return hipErrorInvalidValue;
   }
 
-  const bool tiled_ok = tiled_path(ta, tb, M, N, K, lda, ldb, ldc, strideA, strideB, strideC,
-                                   hk::aligned16(A) && hk::aligned16(B) && hk::aligned16(C));
-  if (!tiled_ok) {
-    if (K == 0) splitK = 1;
+  const Rows rows = row_kind(ta, tb, M, N, K, lda, ldb, ldc, strideA, strideB, strideC,
+                             hk::aligned16(A), hk::aligned16(B), hk::aligned16(C));
+  if (rows == Rows::kNone) {
     dim3 grid((N + 15) / 16, (M + 15) / 16, batchCount);
     hipLaunchKernelGGL(bgemm_simple, grid, dim3(256), 0, stream, ta ? 1 : 0, tb ? 1 : 0, M, N,
                        K, ep, A, static_cast<int64_t>(lda), static_cast<int64_t>(strideA), B,
@@ -1163,43 +975,53 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
                        static_cast<int64_t>(ldc), static_cast<int64_t>(strideC));
     return hk::launch_status();
   }
+  ep.ragged = rows != Rows::kAligned;
+  Plan plan = make_plan(ta, tb, M, N, K, batchCount, splitK, rows);
+  // A captured graph would keep the address of the stream's workspace, which a later call may
+  // grow: under capture the small and any-alignment tiles run unsplit and need none.
+  if (plan.flex && plan.used > 1 && hk::stream_capturing(stream)) {
+    const hk::FlexPlan f =
+        hk::bgemm_flex_plan(M, N, K, batchCount, 1, rows == Rows::kRagged);
+    plan = Plan{f.tile, 1, K};
+  }
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  // k range per split rounded to the k-tile; `used` splits are not empty
-  int used = 1, kps = K;
-  hk::bgemm_split_plan(M, N, K, batchCount, splitK, &used, &kps);
-  HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batchCount) * used <= 65535);
-  if (used == 1)
+  HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batchCount) * plan.used <= 65535);
+  float* part = nullptr;
+  if (plan.used > 1) {
+    void* ws = nullptr;
+    const size_t part_bytes =
+        static_cast<size_t>(plan.used) * batchCount * M * part_pitch(N) * sizeof(float);
+    HK_RETURN_IF_ERROR(hk::device_workspace(part_bytes, stream, &ws));
+    part = static_cast<float*>(ws);
+  }
+  if (plan.flex) {
+    HK_RETURN_IF_ERROR(hk::bgemm_flex_run(
+        plan.flex, hk::FlexCall{ta, tb, M, N, K, batchCount, A, lda, strideA, B, ldb, strideB, C,
+                                ldc, strideC, &ep, plan.used, plan.kps, part, nullptr},
+        stream));
+  } else if (plan.used == 1) {
     return run_regions<false>(ta, tb, batchCount, stream, M, N, K, ep, A, lda, strideA, B, ldb,
                               strideB, C, ldc, strideC, 1, K, nullptr, hk::F32Out{});
-  void* ws = nullptr;
-  const size_t part_bytes = static_cast<size_t>(used) * batchCount * M * N * sizeof(float);
-  HK_RETURN_IF_ERROR(hk::device_workspace(part_bytes, stream, &ws));
-  float* part = static_cast<float*>(ws);
-  HK_RETURN_IF_ERROR(run_regions<true>(ta, tb, batchCount * used, stream, M, N, K, ep, A, lda,
-                                       strideA, B, ldb, strideB, C, ldc, strideC, used, kps,
-                                       part, hk::F32Out{}));
-  const int64_t total = static_cast<int64_t>(M) * N * batchCount;
-  const dim3 fgrid(static_cast<unsigned>(hk::ceil_div(total, 1024)));
-  if (total < (int64_t{1} << 31))
-    hipLaunchKernelGGL(bgemm_splitk_finalize<uint32_t>, fgrid, dim3(256), 0, stream, part, used,
-                       batchCount, M, N, ep, C, static_cast<int64_t>(ldc),
-                       static_cast<int64_t>(strideC));
-  else
-    hipLaunchKernelGGL(bgemm_splitk_finalize<int64_t>, fgrid, dim3(256), 0, stream, part, used,
-                       batchCount, M, N, ep, C, static_cast<int64_t>(ldc),
-                       static_cast<int64_t>(strideC));
-  return hk::launch_status();
+  } else {
+    HK_RETURN_IF_ERROR(run_regions<true>(ta, tb, batchCount * plan.used, stream, M, N, K, ep, A,
+                                         lda, strideA, B, ldb, strideB, C, ldc, strideC,
+                                         plan.used, plan.kps, part, hk::F32Out{}));
+  }
+  if (plan.used == 1) return hipSuccess;
+  return launch_splitk_finalize(stream, part, plan.used, batchCount, M, N, ep, C,
+                                static_cast<int64_t>(ldc), static_cast<int64_t>(strideC));
 }
 
 }  // namespace
 
 namespace hk {
 
-void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, int* kps) {
+void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, int* kps,
+                      double* cost) {
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   const int s = split_k > 0 ? split_k
                             : auto_split_k(tiles * batch, hk::ceil_div(K, BK),
-                                           static_cast<int64_t>(M) * N * batch);
+                                           static_cast<int64_t>(M) * N * batch, cost);
   *kps = static_cast<int>(hk::ceil_div(hk::ceil_div(K, s), BK) * BK);
   *used = static_cast<int>(hk::ceil_div(K, *kps));
 }
@@ -1215,7 +1037,7 @@ hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* 
                hk::aligned16(B) && lda < (1 << 22) && ldb < (1 << 22));
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batch) * used <= 65535);
-  const Epi ep{1.0f, 0.0f, nullptr, 0, 0};
+  const Epi ep{1.0f, 0.0f, nullptr, 0, 0, false};
   const F32Out fo = used == 1 && out ? *out : F32Out{};
   return run_regions<true>(ta, tb, batch * used, stream, M, N, K, ep, A, lda, sA, B, ldb, sB,
                            nullptr, 0, 0, used, kps, part, fo);
@@ -1223,43 +1045,54 @@ hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* 
 
 }  // namespace hk
 
-extern "C" int hk_bgemm_split_count(int transA, int transB, int M, int N, int K, int batchCount,
-                                    int splitK) {
+// 0: empty, -1: invalid, 1: the GEMV kernels or the fallback, 2: the MFMA tiles.
+static int query_kind(int transA, int transB, int M, int N, int K, int batchCount, int splitK) {
   if (transA < 0 || transA > 2 || transB < 0 || transB > 2 || M < 0 || N < 0 || K < 0 ||
       batchCount < 0 || splitK < 0)
     return -1;
   if (M == 0 || N == 0 || batchCount == 0) return 0;
+  if (splitK == 0 && (M == 1 || N == 1)) return 1;
+  return packed_rows(transA != 0, transB != 0, M, N, K) == Rows::kNone ? 1 : 2;
+}
+
+extern "C" int hk_bgemm_split_count(int transA, int transB, int M, int N, int K, int batchCount,
+                                    int splitK) {
+  const int kind = query_kind(transA, transB, M, N, K, batchCount, splitK);
+  if (kind < 2) return kind;
   const bool ta = transA != 0, tb = transB != 0;
-  if (splitK == 0 && (M == 1 || N == 1)) return 1;  // the GEMV kernels
-  const int64_t lda = ta ? M : K, ldb = tb ? K : N;
-  if (!tiled_path(ta, tb, M, N, K, lda, ldb, N, lda * (ta ? K : M), ldb * (tb ? N : K),
-                  static_cast<int64_t>(M) * N, true))
-    return 1;
-  return tiled_splits(M, N, K, batchCount, splitK);
+  return make_plan(ta, tb, M, N, K, batchCount, splitK, packed_rows(ta, tb, M, N, K)).used;
+}
+
+extern "C" int hk_bgemm_small_tile(int transA, int transB, int M, int N, int K, int batchCount,
+                                   int splitK) {
+  const int kind = query_kind(transA, transB, M, N, K, batchCount, splitK);
+  if (kind < 2) return kind < 0 ? -1 : 0;
+  const bool ta = transA != 0, tb = transB != 0;
+  return hk::bgemm_flex_tile_rows(
+      make_plan(ta, tb, M, N, K, batchCount, splitK, packed_rows(ta, tb, M, N, K)).flex);
+}
+
+// The 256-wide tiles' own plan for a product whose operands they take; splits: its k splits.
+static int wide_tile(int transA, int transB, int M, int N, int K, int batchCount, int splitK,
+                     bool cols) {
+  const int kind = query_kind(transA, transB, M, N, K, batchCount, splitK);
+  if (kind <= 0) return kind;
+  const bool ta = transA != 0, tb = transB != 0;
+  if (kind == 1 || packed_rows(ta, tb, M, N, K) == Rows::kRagged) return 0;
+  int used = 1, kps = 0;
+  hk::bgemm_split_plan(M, N, K, batchCount, splitK, &used, &kps);
+  if (w160_plan(ta, tb, M, N, K, batchCount * used, used)) return cols ? w160::kBN : w160::kBM;
+  return cols ? BN : row_tile(ta, M, N, batchCount * used, used);
 }
 
 extern "C" int hk_bgemm_tile_rows(int transA, int transB, int M, int N, int K, int batchCount,
                                   int splitK) {
-  const int splits = hk_bgemm_split_count(transA, transB, M, N, K, batchCount, splitK);
-  if (splits < 0) return -1;
-  if (splits == 0) return 0;
-  const bool ta = transA != 0, tb = transB != 0;
-  const int64_t lda = ta ? M : K, ldb = tb ? K : N;
-  if ((splitK == 0 && (M == 1 || N == 1)) ||
-      !tiled_path(ta, tb, M, N, K, lda, ldb, N, lda * (ta ? K : M), ldb * (tb ? N : K),
-                  static_cast<int64_t>(M) * N, true))
-    return 0;
-  if (w160_plan(ta, tb, M, N, K, batchCount * splits, splits)) return w160::kBM;
-  return row_tile(ta, M, N, batchCount * splits, splits);
+  return wide_tile(transA, transB, M, N, K, batchCount, splitK, false);
 }
 
 extern "C" int hk_bgemm_tile_cols(int transA, int transB, int M, int N, int K, int batchCount,
                                   int splitK) {
-  const int rows = hk_bgemm_tile_rows(transA, transB, M, N, K, batchCount, splitK);
-  if (rows <= 0) return rows;
-  const int splits = hk_bgemm_split_count(transA, transB, M, N, K, batchCount, splitK);
-  return w160_plan(transA != 0, transB != 0, M, N, K, batchCount * splits, splits) ? w160::kBN
-                                                                                   : BN;
+  return wide_tile(transA, transB, M, N, K, batchCount, splitK, true);
 }
 
 extern "C" hipError_t hk_bgemm(int transA, int transB, int M, int N, int K, hk_bf16 alpha,

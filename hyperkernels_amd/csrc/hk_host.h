@@ -30,6 +30,9 @@ int device_cu_count();
 // it once per call; growing it first waits for the work queued on that stream.
 hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out);
 
+// Whether the stream is being captured into a graph.
+bool stream_capturing(hipStream_t stream);
+
 // Batched BF16 matrix-vector product (bgemv.hip), shared by the hk_bgemv_* entry points and
 // hk_bgemm's M == 1 / N == 1 products. Per batch b (element strides sm, sx, sy):
 //   dot_form:  y[r*incy] = alpha sum_k mtx[r*ld + k] x[k*incx] + beta y[r*incy]
@@ -59,7 +62,8 @@ struct F32Out {
 // its epilogue instead (part is not touched). Needs the tiled path's alignment: 8-element
 // multiples and 16-byte aligned bases. bgemm_split_plan picks (used, kps) for a shape: split_k
 // ranges of kps k each (split_k == 0: the library's choice), `used` of them non-empty.
-void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, int* kps);
+void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, int* kps,
+                      double* cost = nullptr);  // cost: the modelled time (us) of split_k == 0
 hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* A, int64_t lda,
                           int64_t sA, const hk_bf16* B, int64_t ldb, int64_t sB, int batch,
                           int used, int kps, float* part, const F32Out* out,

@@ -53,6 +53,15 @@ int device_cu_count() {
   return s->cu_count;
 }
 
+bool stream_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();  // the status is unknown, the call's own launch will tell
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out) {
   std::lock_guard<std::mutex> lk(g_mu);
   int dev = 0;

@@ -289,14 +289,17 @@ HK_API hipError_t hk_reduce_generic_f32(const float* src, float* dst, int out_nd
  *   the output has too few 256 x 256 tiles to fill the device the library may split K itself,
  *   where its cost model expects that to pay (same fp32 partials and split-order sum as
  *   hk_bgemm_core).
+ * Products too small for 256-wide output tiles run on smaller ones, and so do those whose rows
+ *   are no whole 16-byte vectors (extents, leading dimensions or strides that are no multiple of 8,
+ *   pointers at any 2-byte address): the same sums in fp32, in a fixed order.
  * hk_bgemm_split_count (no counterpart in the reference: a host-only planning query for callers
  *   and tests that check which plan runs) returns the number of k splits a product of this
  *   shape runs with (contiguous operands, 16-byte aligned): splitK = 0 for hk_bgemm and the
  *   backward entry points (the library's choice), the hk_bgemm_core argument otherwise. 1 for
  *   the GEMV and fallback kernels, 0 for an empty product, -1 for an invalid argument.
- * Any M, N, K; the MFMA path needs the contiguous extents, leading dimensions and strides to
- * be multiples of 8 and 16-byte aligned pointers (the reference's own precondition,
- * bgemm_test.cu:252-256); other shapes run on a slower fp32-accumulating kernel.
+ * Any M, N, K, leading dimension, stride and 2-byte aligned pointer (the reference needs multiples
+ *   of 8, bgemm_test.cu:252-256); leading dimensions under 8 or from 2^22 on run on a slower
+ *   fp32-accumulating kernel unless the rows are aligned.
  * ---------------------------------------------------------------------------------------- */
 #define HK_LAYOUT_NT 0
 #define HK_LAYOUT_TN 1
@@ -319,15 +322,22 @@ HK_API hipError_t hk_bgemm_tn_backward(int M, int N, int K, hk_bf16 alpha, const
                                        long long strideC, int batchCount, hipStream_t stream);
 HK_API int hk_bgemm_split_count(int transA, int transB, int M, int N, int K, int batchCount,
                                 int splitK);
-/* hk_bgemm_tile_rows (no counterpart in the reference: a host-only planning query, like
- * hk_bgemm_split_count) returns the rows per output tile the MFMA path runs a product of this
- * shape with: 256, or 192 when 256-row tiles would leave most CUs idle and A is k-major
- * (transA == 0); 0 for the GEMV and fallback kernels or an empty product, -1 for an invalid
- * argument. hk_bgemm_tile_cols (likewise a host-only query) returns the columns per output
- * tile: 160 when both operands are k-major (transA == 0, transB != 0), the product runs in one
- * k split, M, N and K are multiples of 256, 160 and 64, and 256 x 256 tiles would leave CUs
- * idle while 256 x 160 tiles fit one round (the 8192 x 1280 x 5120 dA product); otherwise 256
- * (the last tile columns may run 128 wide); 0 / -1 as hk_bgemm_tile_rows. */
+/* hk_bgemm_small_tile (no counterpart in the reference: a host-only planning query, like
+ * hk_bgemm_split_count) returns the rows per output tile, 64 to 256, when a product of this shape
+ * runs on the small or any-alignment tiles, 0 when it runs on the 256-wide ones, the GEMV or the
+ * fallback kernels, -1 for an invalid argument. An explicit splitK keeps the 256-wide tiles for
+ * rows they take. hk_bgemm_tile_rows and hk_bgemm_tile_cols describe the 256-wide tiles' plan of a
+ * shape, whether or not its product runs on them.
+ * hk_bgemm_tile_rows returns the rows per output tile of that plan: 256, or 192 when 256-row tiles
+ * would leave most CUs idle and A is k-major (transA == 0); 0 for rows these tiles do not take, the
+ * GEMV and fallback kernels or an empty product, -1 for an invalid argument. hk_bgemm_tile_cols
+ * (likewise a host-only query) returns the columns per output tile: 160 when both operands are
+ * k-major (transA == 0, transB != 0), the product runs in one k split, M, N and K are multiples of
+ * 256, 160 and 64, and 256 x 256 tiles would leave CUs idle while 256 x 160 tiles fit one round (the
+ * 8192 x 1280 x 5120 dA product); otherwise 256 (the last tile columns may run 128 wide); 0 / -1 as
+ * hk_bgemm_tile_rows. */
+HK_API int hk_bgemm_small_tile(int transA, int transB, int M, int N, int K, int batchCount,
+                               int splitK);
 HK_API int hk_bgemm_tile_rows(int transA, int transB, int M, int N, int K, int batchCount,
                               int splitK);
 HK_API int hk_bgemm_tile_cols(int transA, int transB, int M, int N, int K, int batchCount,
