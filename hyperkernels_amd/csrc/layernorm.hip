@@ -10,14 +10,17 @@
 //   backward (g, b)    kernels/layernorm/ln_backward_gamma_beta_sm89_kernel.cu:15-49
 //                      dgamma += sum_r dy xhat, dbeta += sum_r dy
 //
-// Design (gfx950): one 64-lane wave owns one row; when a row is a whole number of 16-byte
-// vectors (cols % 4 == 0 for fp32, % 8 for 16-bit) of at most 16 per lane (cols <= 4096 fp32,
-// 8192 16-bit) the row is held in VGPRs in its storage format, so x is read from HBM once
-// and mean/variance are computed in two exact passes over registers (no Welford merge). The
+// Design (gfx950): one 64-lane wave owns one row; a row of at most 16 16-byte vectors per lane
+// (cols <= 4096 fp32, 8192 16-bit) is held in VGPRs in its storage format, so x is read from HBM
+// once and mean/variance are computed in two exact passes over registers (no Welford merge). Rows
+// of any length and alignment take this path (Vec): gfx950 serves unaligned 16-byte accesses, and a
+// row that is no whole number of vectors ends with one that overlaps the vector before it. The
 // gamma/beta gradient is accumulated per lane in registers across the rows a wave visits,
-// reduced across the workgroup's waves in LDS, written as one partial per workgroup, and summed over the
-// workgroups in a fixed order by a second small kernel: the result is deterministic, unlike
-// the reference's atomics. Shapes outside the register path use a workgroup-per-row fallback.
+// reduced across the workgroup's waves in LDS, written as one partial per workgroup, and summed over
+// the workgroups in a fixed order by a second small kernel: the result is deterministic, unlike
+// the reference's atomics. Rows of 2049 to 4096 columns are shared by two waves there; few rows
+// take one launch for both gradients (ln_bwd_few_rows). Longer rows use a workgroup-per-row
+// fallback and a column-slab reduction.
 #include <initializer_list>
 #include <mutex>
 #include <type_traits>
@@ -36,11 +39,58 @@ using St = typename T::storage;
 
 __device__ __forceinline__ uint4 u4_zero() { return make_uint4(0u, 0u, 0u, 0u); }
 
+// Vector c of a row of `cols` elements. RAGGED: rows start at any element, and when cols is no
+// multiple of the vector length (and at least one vector) the last vector starts early and
+// repeats `skip` elements of the one before it, which its lane leaves out.
+typedef uint32_t any_t __attribute__((ext_vector_type(4), aligned(2)));  // 16 bytes anywhere
+template <typename T, bool RAGGED>
+struct Vec {
+  using S = typename T::storage;
+  static constexpr int P = T::kPerVec;
+  __device__ static int start(int c, int cols) { return RAGGED ? min(c * P, cols - P) : c * P; }
+  __device__ static int skip(int c, int cols) { return RAGGED ? c * P - start(c, cols) : 0; }
+  __device__ static uint4 load_nt(const S* row, int c, int cols) {
+    if (!RAGGED) return hk::ld_nt(reinterpret_cast<const uint4*>(row) + c);
+    const any_t v =
+        __builtin_nontemporal_load(reinterpret_cast<const any_t*>(row + start(c, cols)));
+    return make_uint4(v.x, v.y, v.z, v.w);
+  }
+  __device__ static uint4 load(const S* row, int c, int cols) {
+    if (!RAGGED) return reinterpret_cast<const uint4*>(row)[c];
+    const any_t v = *reinterpret_cast<const any_t*>(row + start(c, cols));
+    return make_uint4(v.x, v.y, v.z, v.w);
+  }
+  __device__ static void unpack(const uint4& v, int c, int cols, float* f) {
+    T::unpack(v, f);
+    if (RAGGED) {
+      const int n = skip(c, cols);
+#pragma unroll
+      for (int k = 0; k < P; ++k) f[k] = k < n ? 0.f : f[k];
+    }
+  }
+  __device__ static void store_nt(S* row, int c, int cols, const float* f) {
+    const uint4 v = T::pack(f);
+    if (!RAGGED) {
+      hk::st_nt(reinterpret_cast<uint4*>(row) + c, v);
+      return;
+    }
+    S* p = row + start(c, cols);
+    const int n = skip(c, cols);
+    if (n == 0) {
+      __builtin_nontemporal_store(any_t{v.x, v.y, v.z, v.w}, reinterpret_cast<any_t*>(p));
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+      if (k >= n) T::store(p, k, f[k]);
+  }
+};
+
 // One 16-byte vector of gamma (or beta) as fp32, or `dflt` everywhere when the pointer is NULL.
-template <typename T>
-__device__ __forceinline__ void affine(const uint4* p, int c, float dflt, float* f) {
+template <typename T, bool RAGGED>
+__device__ __forceinline__ void affine(const St<T>* p, int c, int cols, float dflt, float* f) {
   if (p) {
-    T::unpack(p[c], f);
+    T::unpack(Vec<T, RAGGED>::load(p, c, cols), f);
   } else {
 #pragma unroll
     for (int k = 0; k < T::kPerVec; ++k) f[k] = dflt;
@@ -50,27 +100,29 @@ __device__ __forceinline__ void affine(const uint4* p, int c, float dflt, float*
 // ------------------------------------------------------------------------------------------
 // Forward, register-resident rows: VPL 16-byte vectors per lane, nvec vectors per row.
 // ------------------------------------------------------------------------------------------
-template <typename T, int VPL>
-__global__ __launch_bounds__(kThreads) void ln_fwd_reg(const uint4* __restrict__ x,
-                                                       const uint4* __restrict__ gamma,
-                                                       const uint4* __restrict__ beta,
-                                                       uint4* __restrict__ y,
+template <typename T, int VPL, bool RAGGED>
+__global__ __launch_bounds__(kThreads) void ln_fwd_reg(const St<T>* __restrict__ x,
+                                                       const St<T>* __restrict__ gamma,
+                                                       const St<T>* __restrict__ beta,
+                                                       St<T>* __restrict__ y,
                                                        float* __restrict__ mean_out,
                                                        float* __restrict__ rstd_out, int rows,
-                                                       int nvec, float inv_cols, float eps) {
+                                                       int cols, float inv_cols, float eps) {
+  using V = Vec<T, RAGGED>;
   constexpr int P = T::kPerVec;
+  const int nvec = (cols + P - 1) / P;
   const int lane = threadIdx.x & (HK_WAVE - 1);
   const int row = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const uint4* xr = x + static_cast<int64_t>(row) * nvec;
+  const St<T>* xr = x + static_cast<int64_t>(row) * cols;
   uint4 v[VPL];
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int c = lane + i * HK_WAVE;
-    v[i] = (c < nvec) ? hk::ld_nt(xr + c) : u4_zero();
+    v[i] = (c < nvec) ? V::load_nt(xr, c, cols) : u4_zero();
     float f[P];
-    T::unpack(v[i], f);
+    V::unpack(v[i], c < nvec ? c : 0, cols, f);
     s += hk::tree_sum<P>(f);
   }
   const float mu = hk::wave_sum(s) * inv_cols;
@@ -82,7 +134,8 @@ __global__ __launch_bounds__(kThreads) void ln_fwd_reg(const uint4* __restrict__
       float f[P];
       T::unpack(v[i], f);
 #pragma unroll
-      for (int k = 0; k < P; ++k) f[k] = (f[k] - mu) * (f[k] - mu);
+      for (int k = 0; k < P; ++k)
+        f[k] = RAGGED && k < V::skip(c, cols) ? 0.f : (f[k] - mu) * (f[k] - mu);
       q += hk::tree_sum<P>(f);
     }
   }
@@ -92,18 +145,18 @@ __global__ __launch_bounds__(kThreads) void ln_fwd_reg(const uint4* __restrict__
     if (mean_out) mean_out[row] = mu;
     if (rstd_out) rstd_out[row] = rs;
   }
-  uint4* yr = y + static_cast<int64_t>(row) * nvec;
+  St<T>* yr = y + static_cast<int64_t>(row) * cols;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int c = lane + i * HK_WAVE;
     if (c < nvec) {
       float f[P], g[P], b[P];
       T::unpack(v[i], f);
-      affine<T>(gamma, c, 1.f, g);
-      affine<T>(beta, c, 0.f, b);
+      affine<T, RAGGED>(gamma, c, cols, 1.f, g);
+      affine<T, RAGGED>(beta, c, cols, 0.f, b);
 #pragma unroll
       for (int k = 0; k < P; ++k) f[k] = (f[k] - mu) * rs * g[k] + b[k];
-      hk::st_nt(yr + c, T::pack(f));
+      V::store_nt(yr, c, cols, f);
     }
   }
 }
@@ -136,67 +189,85 @@ constexpr int kOneRowMaxCols = T::kPerVec == 4 ? 768 : 1024;
 // so the two wave reductions of one row overlap the loads of the next; ONE_ROW drops the
 // prefetch (each row is loaded at the top of its iteration) for grids where each wave has one
 // row. dy, x and gamma stay in registers in their storage format and are widened to fp32
-// where they are used.
+// where they are used. NW > 1: NW waves share a row (vectors dealt to them 64 by 64) and
+// exchange their two sums through LDS, so rows of up to 4096 columns keep their gamma/beta sums
+// in registers; every wave of the workgroup then makes the same number of iterations.
 // ------------------------------------------------------------------------------------------
-template <typename T, int VPL, bool WRITE_DX, bool DO_GB, int WAVES, bool ONE_ROW = false>
-__global__ __launch_bounds__(WAVES * HK_WAVE, ONE_ROW ? 4 : 1) void ln_bwd_reg(
-    const uint4* __restrict__ dy, const uint4* __restrict__ x, const float* __restrict__ mean,
-    const float* __restrict__ rstd, const uint4* __restrict__ gamma, uint4* __restrict__ dx,
-    float* __restrict__ part, int rows, int nvec, float inv_cols) {
+template <typename T, int VPL, bool WRITE_DX, bool DO_GB, int WAVES, bool ONE_ROW = false,
+          bool RAGGED = false, int NW = 1>
+__global__ __launch_bounds__(WAVES * HK_WAVE, ONE_ROW && WAVES == 16 ? 4 : 1) void ln_bwd_reg(
+    const St<T>* __restrict__ dy, const St<T>* __restrict__ x, const float* __restrict__ mean,
+    const float* __restrict__ rstd, const St<T>* __restrict__ gamma, St<T>* __restrict__ dx,
+    float* __restrict__ part, int rows, int cols, float inv_cols) {
   // Every product below is rounded on its own (as the reference formula is written), so a
   // row whose terms cancel exactly (cols == 1) gives exactly zero.
 #pragma clang fp contract(off)
+  using V = Vec<T, RAGGED>;
   constexpr int P = T::kPerVec;
-  extern __shared__ float4 lds4[];  // [WAVES][2][cols] floats when DO_GB
+  constexpr int SLOTS = WAVES / NW;  // rows in flight per workgroup
+  extern __shared__ float4 lds4[];   // [SLOTS][2][cols] floats when DO_GB
+  __shared__ float2 row_sums[2][NW > 1 ? WAVES : 1];
+  const int nvec = (cols + P - 1) / P;
   const int lane = threadIdx.x & (HK_WAVE - 1);
   const int wave = threadIdx.x >> 6;
+  const int slot = wave / NW, share = wave % NW;
+  auto col = [&](int i) { return lane + (share + NW * i) * HK_WAVE; };  // vector i of this lane
   uint4 graw[VPL];
   float acc_g[VPL][P], acc_b[VPL][P];
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
-    const int c = lane + i * HK_WAVE;
-    graw[i] = (gamma && c < nvec) ? gamma[c] : u4_zero();
+    const int c = col(i);
+    // NW > 1 reads gamma where it is used (from cache): held here, 4096 columns would spill
+    if (NW == 1) graw[i] = (gamma && c < nvec) ? V::load(gamma, c, cols) : u4_zero();
 #pragma unroll
     for (int k = 0; k < P; ++k) acc_g[i][k] = acc_b[i][k] = 0.f;
   }
-  const int stride = gridDim.x * WAVES;
-  int row = blockIdx.x * WAVES + wave;
+  const int stride = gridDim.x * SLOTS;
+  int row = blockIdx.x * SLOTS + slot;
   uint4 dn[VPL], xn[VPL];
   float mn = 0.f, rn = 0.f;
   auto fetch = [&](int r) {
-    const uint4* dyr = dy + static_cast<int64_t>(r) * nvec;
-    const uint4* xr = x + static_cast<int64_t>(r) * nvec;
+    const St<T>* dyr = dy + static_cast<int64_t>(r) * cols;
+    const St<T>* xr = x + static_cast<int64_t>(r) * cols;
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int c = lane + i * HK_WAVE;
-      dn[i] = (c < nvec) ? hk::ld_nt(dyr + c) : u4_zero();
-      xn[i] = (c < nvec) ? hk::ld_nt(xr + c) : u4_zero();
+      const int c = col(i);
+      dn[i] = (c < nvec) ? V::load_nt(dyr, c, cols) : u4_zero();
+      xn[i] = (c < nvec) ? V::load_nt(xr, c, cols) : u4_zero();
     }
     mn = mean[r];
     rn = rstd[r];
   };
-  // dy, x-hat and dy * gamma of vector i of the current row (x-hat is zero past the row end).
+  // dy, x-hat and dy * gamma of vector i of the current row (zero past the row end and for the
+  // repeated elements of a ragged row's last vector).
   auto widen = [&](const uint4& draw, const uint4& xraw, int i, float m, float rs, float* d,
                    float* n, float* a) {
-    const bool in = lane + i * HK_WAVE < nvec;
+    const int c = col(i);
+    const bool in = c < nvec;
+    const int skip = RAGGED && in ? V::skip(c, cols) : 0;
     float g[P];
     T::unpack(draw, d);
     T::unpack(xraw, n);
     if (gamma) {
-      T::unpack(graw[i], g);
+      T::unpack(NW == 1 ? graw[i] : V::load(gamma, in ? c : 0, cols), g);
     } else {
 #pragma unroll
       for (int k = 0; k < P; ++k) g[k] = 1.f;
     }
 #pragma unroll
     for (int k = 0; k < P; ++k) {
-      n[k] = in ? (n[k] - m) * rs : 0.f;
+      const bool own = in && (!RAGGED || k >= skip);
+      n[k] = own ? (n[k] - m) * rs : 0.f;
+      if (RAGGED) d[k] = own ? d[k] : 0.f;
       a[k] = d[k] * g[k];
     }
   };
   if (!ONE_ROW && row < rows) fetch(row);
-  for (; row < rows; row += stride) {
-    if (ONE_ROW) fetch(row);
+  int parity = 0;
+  // NW > 1: `row - slot` is the same for the whole workgroup, which iterates together
+  for (; (NW > 1 ? row - slot : row) < rows; row += stride) {
+    const bool live = NW == 1 || row < rows;
+    if (ONE_ROW && live) fetch(row);
     uint4 dcur[VPL], xcur[VPL];
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
@@ -206,68 +277,106 @@ __global__ __launch_bounds__(WAVES * HK_WAVE, ONE_ROW ? 4 : 1) void ln_bwd_reg(
     const float m = mn, rs = rn;
     if (!ONE_ROW && row + stride < rows) fetch(row + stride);
     float s1 = 0.f, s2 = 0.f;
+    if (live) {
 #pragma unroll
-    for (int i = 0; i < VPL; ++i) {
-      float d[P], n[P], a[P];
-      widen(dcur[i], xcur[i], i, m, rs, d, n, a);
-      if (DO_GB) {
+      for (int i = 0; i < VPL; ++i) {
+        float d[P], n[P], a[P];
+        widen(dcur[i], xcur[i], i, m, rs, d, n, a);
+        if (DO_GB) {
 #pragma unroll
-        for (int k = 0; k < P; ++k) {
-          acc_g[i][k] += d[k] * n[k];
-          acc_b[i][k] += d[k];
+          for (int k = 0; k < P; ++k) {
+            acc_g[i][k] += d[k] * n[k];
+            acc_b[i][k] += d[k];
+          }
         }
-      }
-      if (WRITE_DX) {
-        s1 += hk::tree_sum<P>(a);
+        if (WRITE_DX) {
+          s1 += hk::tree_sum<P>(a);
 #pragma unroll
-        for (int k = 0; k < P; ++k) n[k] = a[k] * n[k];
-        s2 += hk::tree_sum<P>(n);
+          for (int k = 0; k < P; ++k) n[k] = a[k] * n[k];
+          s2 += hk::tree_sum<P>(n);
+        }
       }
     }
     if (WRITE_DX) {
-      const float t1 = hk::wave_sum(s1), t2 = hk::wave_sum(s2);
-      uint4* dxr = dx + static_cast<int64_t>(row) * nvec;
+      float t1 = hk::wave_sum(s1), t2 = hk::wave_sum(s2);
+      if constexpr (NW > 1) {
+        // two buffers: the next row's sums are written while a slower wave still reads these
+        if (lane == 0) row_sums[parity][wave] = make_float2(t1, t2);
+        __syncthreads();
+        t1 = t2 = 0.f;
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) {
-        const int c = lane + i * HK_WAVE;
-        if (c < nvec) {
-          float d[P], n[P], a[P], o[P];
-          widen(dcur[i], xcur[i], i, m, rs, d, n, a);
+        for (int w = 0; w < NW; ++w) {
+          const float2 v = row_sums[parity][slot * NW + w];
+          t1 += v.x;
+          t2 += v.y;
+        }
+        parity ^= 1;
+      }
+      if (live) {
+        St<T>* dxr = dx + static_cast<int64_t>(row) * cols;
 #pragma unroll
-          for (int k = 0; k < P; ++k) o[k] = rs * (a[k] - (t1 + n[k] * t2) * inv_cols);
-          hk::st_nt(dxr + c, T::pack(o));
+        for (int i = 0; i < VPL; ++i) {
+          const int c = col(i);
+          if (c < nvec) {
+            float d[P], n[P], a[P], o[P];
+            widen(dcur[i], xcur[i], i, m, rs, d, n, a);
+#pragma unroll
+            for (int k = 0; k < P; ++k) o[k] = rs * (a[k] - (t1 + n[k] * t2) * inv_cols);
+            V::store_nt(dxr, c, cols, o);
+          }
         }
       }
     }
   }
-  if (DO_GB) {
-    // LDS holds [wave][gamma | beta][cols] floats; vector c covers columns c*P .. c*P+P-1.
-    constexpr int Q = P / 4;  // float4s per vector
-    const int cols4 = nvec * Q;
-    float4* my = lds4 + static_cast<int64_t>(wave) * 2 * cols4;
+  if constexpr (DO_GB) {
+    // LDS holds [slot][gamma | beta][cols] floats
+    float* ldsf = reinterpret_cast<float*>(lds4);
+    float* my = ldsf + static_cast<int64_t>(slot) * 2 * cols;
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-      const int c = lane + i * HK_WAVE;
-      if (c < nvec) {
+      const int c = col(i);
+      if (c >= nvec) continue;
+      float* g = my + V::start(c, cols);
+      float* b = g + cols;
+      if constexpr (RAGGED) {
+        const int skip = V::skip(c, cols);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          my[c * Q + q] = make_float4(acc_g[i][4 * q], acc_g[i][4 * q + 1], acc_g[i][4 * q + 2],
-                                      acc_g[i][4 * q + 3]);
-          my[cols4 + c * Q + q] = make_float4(acc_b[i][4 * q], acc_b[i][4 * q + 1],
-                                              acc_b[i][4 * q + 2], acc_b[i][4 * q + 3]);
+        for (int k = 0; k < P; ++k)
+          if (k >= skip) {
+            g[k] = acc_g[i][k];
+            b[k] = acc_b[i][k];
+          }
+      } else {
+#pragma unroll
+        for (int q = 0; q < P; q += 4) {
+          *reinterpret_cast<float4*>(g + q) =
+              make_float4(acc_g[i][q], acc_g[i][q + 1], acc_g[i][q + 2], acc_g[i][q + 3]);
+          *reinterpret_cast<float4*>(b + q) =
+              make_float4(acc_b[i][q], acc_b[i][q + 1], acc_b[i][q + 2], acc_b[i][q + 3]);
         }
       }
     }
     __syncthreads();
-    float4* out = reinterpret_cast<float4*>(part) + static_cast<int64_t>(blockIdx.x) * 2 * cols4;
-    for (int c = threadIdx.x; c < 2 * cols4; c += WAVES * HK_WAVE) {
-      float4 s = lds4[c];
+    if constexpr (RAGGED) {
+      float* out = part + static_cast<int64_t>(blockIdx.x) * 2 * cols;
+      for (int c = threadIdx.x; c < 2 * cols; c += WAVES * HK_WAVE) {
+        float t = ldsf[c];
 #pragma unroll
-      for (int w = 1; w < WAVES; ++w) {
-        const float4 t = lds4[static_cast<int64_t>(w) * 2 * cols4 + c];
-        s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+        for (int w = 1; w < SLOTS; ++w) t += ldsf[static_cast<int64_t>(w) * 2 * cols + c];
+        out[c] = t;
       }
-      out[c] = s;
+    } else {
+      const int cols4 = cols / 4;
+      float4* out = reinterpret_cast<float4*>(part) + static_cast<int64_t>(blockIdx.x) * 2 * cols4;
+      for (int c = threadIdx.x; c < 2 * cols4; c += WAVES * HK_WAVE) {
+        float4 s = lds4[c];
+#pragma unroll
+        for (int w = 1; w < SLOTS; ++w) {
+          const float4 t = lds4[static_cast<int64_t>(w) * 2 * cols4 + c];
+          s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+        }
+        out[c] = s;
+      }
     }
   }
 }
@@ -311,6 +420,101 @@ __global__ __launch_bounds__(kFinCols * kFinGroups) void ln_gb_finalize(
 #pragma unroll
     for (int g = 1; g < kFinGroups; ++g) s += red[g][col];
     if (dst) *dst = prev + s;
+  }
+}
+
+// Few rows: grad_x and the gamma/beta gradients in one launch. The first `row_groups` workgroups
+// take one row per wave; each of the others owns kFinCols columns and sums them over every row (32
+// row groups, added pairwise), reading dy and x a second time, from cache. Saves the partials'
+// round trip and the finalize launch, which at 64 x 768 cost more than the second read.
+template <typename T, int VPL, bool RAGGED>
+__global__ __launch_bounds__(kFinCols * kFinGroups) void ln_bwd_few_rows(
+    const St<T>* __restrict__ dy, const St<T>* __restrict__ x, const float* __restrict__ mean,
+    const float* __restrict__ rstd, const St<T>* __restrict__ gamma, St<T>* __restrict__ dx,
+    float* __restrict__ grad_gamma, float* __restrict__ grad_beta, int rows, int cols,
+    float inv_cols, int row_groups) {
+#pragma clang fp contract(off)
+  using V = Vec<T, RAGGED>;
+  constexpr int P = T::kPerVec;
+  if (static_cast<int>(blockIdx.x) < row_groups) {
+    const int nvec = (cols + P - 1) / P;
+    const int lane = threadIdx.x & (HK_WAVE - 1);
+    const int row = blockIdx.x * (kFinCols * kFinGroups / HK_WAVE) + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const St<T>* dyr = dy + static_cast<int64_t>(row) * cols;
+    const St<T>* xr = x + static_cast<int64_t>(row) * cols;
+    uint4 dv[VPL], xv[VPL];
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = lane + i * HK_WAVE;
+      dv[i] = c < nvec ? V::load(dyr, c, cols) : u4_zero();
+      xv[i] = c < nvec ? V::load(xr, c, cols) : u4_zero();
+    }
+    const float m = mean[row], rs = rstd[row];
+    auto widen = [&](int i, float* n, float* a) {
+      const int c = lane + i * HK_WAVE;
+      const int skip = RAGGED && c < nvec ? V::skip(c, cols) : 0;
+      float d[P], g[P];
+      T::unpack(dv[i], d);
+      T::unpack(xv[i], n);
+      affine<T, RAGGED>(gamma, c < nvec ? c : 0, cols, 1.f, g);
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        const bool own = c < nvec && (!RAGGED || k >= skip);
+        n[k] = own ? (n[k] - m) * rs : 0.f;
+        a[k] = own ? d[k] * g[k] : 0.f;
+      }
+    };
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      float n[P], a[P];
+      widen(i, n, a);
+      s1 += hk::tree_sum<P>(a);
+#pragma unroll
+      for (int k = 0; k < P; ++k) n[k] = a[k] * n[k];
+      s2 += hk::tree_sum<P>(n);
+    }
+    const float t1 = hk::wave_sum(s1), t2 = hk::wave_sum(s2);
+    St<T>* dxr = dx + static_cast<int64_t>(row) * cols;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int c = lane + i * HK_WAVE;
+      if (c < nvec) {
+        float n[P], a[P], o[P];
+        widen(i, n, a);
+#pragma unroll
+        for (int k = 0; k < P; ++k) o[k] = rs * (a[k] - (t1 + n[k] * t2) * inv_cols);
+        V::store_nt(dxr, c, cols, o);
+      }
+    }
+    return;
+  }
+  __shared__ float red[2][kFinGroups][kFinCols];
+  const int col = threadIdx.x % kFinCols, grp = threadIdx.x / kFinCols;
+  const int c = (blockIdx.x - row_groups) * kFinCols + col;
+  // the values added into are loaded first, as in the finalize above
+  const float* into = grp == 0 ? grad_gamma : grp == 1 ? grad_beta : nullptr;
+  const float prev = into && c < cols ? into[c] : 0.f;
+  float sg = 0.f, sb = 0.f;
+  if (c < cols) {
+#pragma unroll 4
+    for (int r = grp; r < rows; r += kFinGroups) {
+      const int64_t o = static_cast<int64_t>(r) * cols + c;
+      const float d = T::load(dy, o);
+      sg = __builtin_fmaf(d, (T::load(x, o) - mean[r]) * rstd[r], sg);
+      sb += d;
+    }
+  }
+  red[0][grp][col] = sg;
+  red[1][grp][col] = sb;
+  __syncthreads();
+  if (grp < 2 && c < cols) {  // group 0: gamma, group 1: beta, each a pairwise sum of the groups
+    float v[kFinGroups];
+#pragma unroll
+    for (int g = 0; g < kFinGroups; ++g) v[g] = red[grp][g][col];
+    float* dst = grp == 0 ? grad_gamma : grad_beta;
+    if (dst) dst[c] = prev + hk::tree_sum<kFinGroups>(v);
   }
 }
 
@@ -387,24 +591,34 @@ __global__ __launch_bounds__(kThreads) void ln_bwd_input_rowblock(
   }
 }
 
-// Column-parallel gamma/beta gradient for the fallback path: one thread per column, rows
-// summed in order (deterministic).
+// Gamma/beta gradient of rows that the register path does not hold: a lane per column, the rows in
+// gridDim.y slabs of `slab` rows, each summed in row order into part[slab][2 * cols] (gamma then
+// beta) for ln_gb_finalize. One slab (gridDim.y == 1) adds into the gradients itself.
 template <typename T, typename S = typename T::storage>
-__global__ __launch_bounds__(kThreads) void ln_gb_columns(const S* __restrict__ dy,
-                                                          const S* __restrict__ x,
-                                                          const float* __restrict__ mean,
-                                                          const float* __restrict__ rstd,
-                                                          float* __restrict__ grad_gamma,
-                                                          float* __restrict__ grad_beta,
-                                                          int rows, int cols) {
+__global__ __launch_bounds__(kThreads) void ln_gb_slab(const S* __restrict__ dy,
+                                                       const S* __restrict__ x,
+                                                       const float* __restrict__ mean,
+                                                       const float* __restrict__ rstd,
+                                                       float* __restrict__ part,
+                                                       float* __restrict__ grad_gamma,
+                                                       float* __restrict__ grad_beta, int rows,
+                                                       int cols, int slab) {
   const int c = blockIdx.x * kThreads + threadIdx.x;
   if (c >= cols) return;
+  const int r0 = blockIdx.y * slab, r1 = min(rows, r0 + slab);
   float sg = 0.f, sb = 0.f;
-  for (int r = 0; r < rows; ++r) {
+#pragma unroll 8
+  for (int r = r0; r < r1; ++r) {
     const int64_t o = static_cast<int64_t>(r) * cols + c;
     const float d = T::load(dy, o);
     sg += d * ((T::load(x, o) - mean[r]) * rstd[r]);
     sb += d;
+  }
+  if (gridDim.y > 1) {
+    float* out = part + static_cast<int64_t>(blockIdx.y) * 2 * cols;
+    out[c] = sg;
+    out[cols + c] = sb;
+    return;
   }
   if (grad_gamma) grad_gamma[c] += sg;
   if (grad_beta) grad_beta[c] += sb;
@@ -435,30 +649,43 @@ hipError_t with_vpl(int vpl, F&& f) {
   }
 }
 
+// Rows of whole, 16-byte aligned vectors (else the RAGGED forms).
 template <typename T>
-bool reg_path_ok(int cols, std::initializer_list<const void*> ptrs) {
-  constexpr int P = T::kPerVec;
-  if (cols % P != 0 || pick_vpl(cols / P) == 0) return false;
+bool vec_rows(int cols, std::initializer_list<const void*> ptrs) {
+  if (cols % T::kPerVec != 0) return false;
   for (const void* p : ptrs)
     if (p && !hk::aligned16(p)) return false;
   return true;
 }
 
-constexpr int kMaxGbCols = 2048;
+// 16-byte vectors per lane of a row over `waves` waves; 0: no register path (longer than 16 per
+// lane, or shorter than one vector).
+template <typename T>
+int row_vpl(int cols, int waves = 1) {
+  if (cols < T::kPerVec) return 0;
+  return pick_vpl(static_cast<int>(hk::ceil_div(hk::ceil_div(cols, T::kPerVec), waves)));
+}
+
+constexpr int kMaxGbCols = 2048;      // one wave per row with gamma/beta sums in registers
+constexpr int kMaxWideCols = 4096;    // four waves per row
+// Rows up to which both gradients come from one launch (ln_bwd_few_rows). Fused backward on MI355X,
+// one launch against two, us per call back to back (a call costs its caller 3.4): 64 x 768 fp32 3.4
+// against 6.9, 512 x 768 4.1 against 7.0, 300 x 4096 bf16 7.6 against 11.3.
+constexpr int kFewRows = 512;
+template <typename T>
+constexpr int kMaxFewVpl = T::kPerVec == 4 ? 12 : 8;  // fp32 rows of 16 vectors per lane spill
 template <typename T>
 constexpr int kMaxBwdVpl = 4096 / (HK_WAVE * T::kPerVec);
 
-// Lets a ONE_ROW gamma/beta backward form use its up to 128 KiB of dynamic LDS (set once per
-// kernel, before its first launch).
-template <typename T, int V, bool WRITE_DX>
-hipError_t one_row_lds_limit() {
+// Lets a kernel use `bytes` of dynamic LDS (set once per kernel, before its first launch).
+template <auto Kernel>
+hipError_t lds_limit(size_t bytes) {
   static std::once_flag once;
   static hipError_t status = hipSuccess;
-  std::call_once(once, [] {
-    status = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&ln_bwd_reg<T, V, WRITE_DX, true, kOneRowWaves, true>),
-        hipFuncAttributeMaxDynamicSharedMemorySize,
-        static_cast<int>(kOneRowWaves * 2 * kOneRowMaxCols<T> * sizeof(float)));
+  std::call_once(once, [bytes] {
+    status = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 static_cast<int>(bytes));
   });
   return status;
 }
@@ -477,22 +704,129 @@ hipError_t launch_fwd(const St<T>* x, const St<T>* gamma, const St<T>* beta, St<
   HK_CHECK_ARG(rows >= 0 && cols >= 0);
   if (rows == 0 || cols == 0) return hipSuccess;
   HK_CHECK_ARG(x && y);
-  if (reg_path_ok<T>(cols, {x, gamma, beta, y})) {
-    const int nvec = cols / T::kPerVec;
+  if (const int vpl = row_vpl<T>(cols)) {
+    const bool vec = vec_rows<T>(cols, {x, gamma, beta, y});
     const unsigned grid = static_cast<unsigned>(hk::ceil_div(rows, kWavesPerBlock));
     const float inv_cols = 1.0f / static_cast<float>(cols);
-    return with_vpl(pick_vpl(nvec), [&](auto vpl_c) -> hipError_t {
+    return with_vpl(vpl, [&](auto vpl_c) -> hipError_t {
       constexpr int V = decltype(vpl_c)::value;
-      hipLaunchKernelGGL((ln_fwd_reg<T, V>), dim3(grid), dim3(kThreads), 0, stream,
-                         reinterpret_cast<const uint4*>(x), reinterpret_cast<const uint4*>(gamma),
-                         reinterpret_cast<const uint4*>(beta), reinterpret_cast<uint4*>(y),
-                         mean_out, rstd_out, rows, nvec, inv_cols, eps);
+      hipLaunchKernelGGL((vec ? ln_fwd_reg<T, V, false> : ln_fwd_reg<T, V, true>), dim3(grid),
+                         dim3(kThreads), 0, stream, x, gamma, beta, y, mean_out, rstd_out, rows,
+                         cols, inv_cols, eps);
       return hk::launch_status();
     });
   }
   hipLaunchKernelGGL(ln_fwd_rowblock<T>, dim3(rows), dim3(kThreads), 0, stream, x, gamma, beta, y,
                      mean_out, rstd_out, cols, eps);
   return hk::launch_status();
+}
+
+template <typename T>
+using BwdKernel = void (*)(const St<T>*, const St<T>*, const float*, const float*, const St<T>*,
+                           St<T>*, float*, int, int, float);
+
+// The fused gamma/beta forms of the register path: kernel, workgroup and grid of a shape.
+template <typename T>
+struct GbForm {
+  BwdKernel<T> kernel = nullptr;
+  int waves = 0, grid = 0;
+  size_t lds = 0;
+};
+
+template <typename T, bool RAGGED>
+hipError_t gb_form(int rows, int cols, bool write_dx, GbForm<T>* out) {
+  const int64_t cus = hk::device_cu_count();
+  if (cols > kMaxGbCols) {
+    // Four waves per row, four rows in flight per workgroup, one workgroup per CU, LDS for 4 x 2 x
+    // cols floats (128 KiB at most). Fused backward on MI355X: 4096 x 2560 bf16 23.6 us (two waves
+    // per row and 8 per workgroup 23.6, too: 34.4 against 31.0 at 4096 columns), fp32 29.3 us (31.4).
+    // These rows ran a workgroup per row for grad_x and one lane per column over all rows for the
+    // gradients, 1,278 and 1,235 us.
+    return with_vpl(row_vpl<T>(cols, 4), [&](auto vpl_c) -> hipError_t {
+      constexpr int V = decltype(vpl_c)::value;
+      if constexpr (V * T::kPerVec > kMaxWideCols / (4 * HK_WAVE)) {
+        return hipErrorInvalidValue;
+      } else {
+        constexpr int W = 16, kSlots = W / 4;
+        constexpr size_t kLds = kSlots * 2 * kMaxWideCols * sizeof(float);
+        const int64_t want = hk::ceil_div(rows, kSlots);
+        constexpr auto dx_gb = ln_bwd_reg<T, V, true, true, W, true, RAGGED, 4>;
+        constexpr auto gb = ln_bwd_reg<T, V, false, true, W, true, RAGGED, 4>;
+        HK_RETURN_IF_ERROR(write_dx ? lds_limit<dx_gb>(kLds) : lds_limit<gb>(kLds));
+        *out = GbForm<T>{write_dx ? dx_gb : gb, W, static_cast<int>(want < cus ? want : cus),
+                         static_cast<size_t>(kSlots) * 2 * cols * sizeof(float)};
+        return hipSuccess;
+      }
+    });
+  }
+  // The gamma/beta partials of one workgroup live in LDS: 8 (cols <= 1024) or 4 waves x 2 x
+  // cols floats, kept within 64 KiB (cols <= kMaxGbCols); the one-row form's 16 waves take up
+  // to 128 KiB (cols <= kOneRowMaxCols<T>).
+  const bool one_row = !RAGGED && cols <= kOneRowMaxCols<T> && rows <= cus * kOneRowWaves;
+  return with_vpl(row_vpl<T>(cols), [&](auto vpl_c) -> hipError_t {
+    constexpr int V = decltype(vpl_c)::value;
+    constexpr int kCols = V * HK_WAVE * T::kPerVec;  // the widest row of this VPL
+    if constexpr (kCols > kMaxGbCols) {
+      return hipErrorInvalidValue;
+    } else {
+      if constexpr (!RAGGED && kCols <= kOneRowMaxCols<T>) {
+        if (one_row) {
+          constexpr int W = kOneRowWaves;
+          constexpr size_t kLds = W * 2 * kOneRowMaxCols<T> * sizeof(float);
+          constexpr auto dx_gb = ln_bwd_reg<T, V, true, true, W, true>;
+          constexpr auto gb = ln_bwd_reg<T, V, false, true, W, true>;
+          HK_RETURN_IF_ERROR(write_dx ? lds_limit<dx_gb>(kLds) : lds_limit<gb>(kLds));
+          *out = GbForm<T>{write_dx ? dx_gb : gb, W, static_cast<int>(hk::ceil_div(rows, W)),
+                           static_cast<size_t>(W) * 2 * cols * sizeof(float)};
+          return hipSuccess;
+        }
+      }
+      // row_vpl takes the smallest VPL that holds the row, so cols <= 1024 exactly when
+      // kCols <= 1024: the wave count is fixed by V
+      constexpr int W = gb_waves(kCols);
+      *out = GbForm<T>{write_dx ? ln_bwd_reg<T, V, true, true, W, false, RAGGED>
+                                : ln_bwd_reg<T, V, false, true, W, false, RAGGED>,
+                       W, bwd_gb_grid(rows, W), static_cast<size_t>(W) * 2 * cols * sizeof(float)};
+      return hipSuccess;
+    }
+  });
+}
+
+template <typename T>
+hipError_t launch_finalize(const float* part, int nparts, int cols, float* dgamma, float* dbeta,
+                           hipStream_t stream) {
+  hipLaunchKernelGGL(ln_gb_finalize, dim3(static_cast<unsigned>(hk::ceil_div(2 * cols, kFinCols))),
+                     dim3(kFinCols * kFinGroups), 0, stream, part, nparts, cols, dgamma, dbeta);
+  return hk::launch_status();
+}
+
+// grad_x alone.
+template <typename T>
+hipError_t launch_dx(const St<T>* dy, const St<T>* x, const float* mean, const float* rstd,
+                     const St<T>* gamma, St<T>* dx, int rows, int cols, bool vec,
+                     hipStream_t stream) {
+  // The backward keeps dy, x and their prefetch in registers; past kMaxBwdVpl vectors per lane
+  // (4096 columns for every storage type) it would spill, so wider rows take a workgroup per row.
+  const int vpl = row_vpl<T>(cols);
+  if (vpl == 0 || vpl > kMaxBwdVpl<T>) {
+    hipLaunchKernelGGL(ln_bwd_input_rowblock<T>, dim3(rows), dim3(kThreads), 0, stream, dy, x,
+                       mean, rstd, gamma, dx, cols);
+    return hk::launch_status();
+  }
+  return with_vpl(vpl, [&](auto vpl_c) -> hipError_t {
+    constexpr int V = decltype(vpl_c)::value;
+    if constexpr (V > kMaxBwdVpl<T>) {
+      return hipErrorInvalidValue;
+    } else {
+      constexpr int W = kWavesPerBlock;
+      hipLaunchKernelGGL((vec ? ln_bwd_reg<T, V, true, false, W>
+                              : ln_bwd_reg<T, V, true, false, W, false, true>),
+                         dim3(static_cast<unsigned>(hk::ceil_div(rows, W))), dim3(W * HK_WAVE), 0,
+                         stream, dy, x, mean, rstd, gamma, dx, static_cast<float*>(nullptr), rows,
+                         cols, 1.0f / static_cast<float>(cols));
+      return hk::launch_status();
+    }
+  });
 }
 
 template <typename T>
@@ -503,85 +837,65 @@ hipError_t launch_bwd(const St<T>* dy, const St<T>* x, const float* mean, const 
   if (rows == 0 || cols == 0) return hipSuccess;
   HK_CHECK_ARG(dy && x && mean && rstd);
   HK_CHECK_ARG(!write_dx || dx);
-  // The gamma/beta partials of one workgroup live in LDS: 8 (cols <= 1024) or 4 waves x 2 x
-  // cols floats, kept within 64 KiB (cols <= kMaxGbCols); the one-row form's 16 waves take up
-  // to 128 KiB (cols <= kOneRowMaxCols<T>). The backward keeps dy, x and their prefetch in
-  // registers; past kMaxBwdVpl vectors per lane (4096 columns for every storage type) it would
-  // spill, so wider rows take the workgroup-per-row kernels.
-  if (reg_path_ok<T>(cols, {dy, x, gamma, dx}) && pick_vpl(cols / T::kPerVec) <= kMaxBwdVpl<T> &&
-      (!do_gb || cols <= kMaxGbCols)) {
-    const int nvec = cols / T::kPerVec;
-    const bool one_row = do_gb && cols <= kOneRowMaxCols<T> &&
-                         rows <= static_cast<int64_t>(hk::device_cu_count()) * kOneRowWaves;
-    const int waves = one_row ? kOneRowWaves : do_gb ? gb_waves(cols) : kWavesPerBlock;
-    const int grid = one_row ? static_cast<int>(hk::ceil_div(rows, kOneRowWaves))
-                     : do_gb ? bwd_gb_grid(rows, waves)
-                             : static_cast<int>(hk::ceil_div(rows, kWavesPerBlock));
-    float* part = nullptr;
-    if (do_gb) {
-      void* ws = nullptr;
-      HK_RETURN_IF_ERROR(
-          hk::device_workspace(static_cast<size_t>(grid) * 2 * cols * sizeof(float), stream, &ws));
-      part = static_cast<float*>(ws);
-    }
-    const size_t lds = do_gb ? static_cast<size_t>(waves) * 2 * cols * sizeof(float) : 0;
-    const float inv_cols = 1.0f / static_cast<float>(cols);
-    HK_RETURN_IF_ERROR(with_vpl(pick_vpl(nvec), [&](auto vpl_c) -> hipError_t {
+  const bool vec = vec_rows<T>(cols, {dy, x, gamma, dx});
+  if (!do_gb) return launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream);
+  const int vpl = row_vpl<T>(cols);
+  const float inv_cols = 1.0f / static_cast<float>(cols);
+  if (rows <= kFewRows && vpl > 0 && vpl <= kMaxFewVpl<T>) {
+    const int row_groups =
+        write_dx ? static_cast<int>(hk::ceil_div(rows, kFinCols * kFinGroups / HK_WAVE)) : 0;
+    const unsigned grid = static_cast<unsigned>(row_groups + hk::ceil_div(cols, kFinCols));
+    return with_vpl(vpl, [&](auto vpl_c) -> hipError_t {
       constexpr int V = decltype(vpl_c)::value;
-      // only the forms the conditions above can select are instantiated
-      if constexpr (V > kMaxBwdVpl<T>) {
+      if constexpr (V > kMaxFewVpl<T>) {
         return hipErrorInvalidValue;
       } else {
-        constexpr int kCols = V * HK_WAVE * T::kPerVec;  // the widest row of this VPL
-        constexpr bool kGb = kCols <= kMaxGbCols;
-        using Kernel = void (*)(const uint4*, const uint4*, const float*, const float*,
-                                const uint4*, uint4*, float*, int, int, float);
-        Kernel k = ln_bwd_reg<T, V, true, false, kWavesPerBlock>;
-        // pick_vpl takes the smallest VPL that holds the row, so cols <= 1024 exactly when
-        // kCols <= 1024: the wave count of the gamma/beta forms is fixed by V
-        constexpr int kW = gb_waves(kCols);
-        if constexpr (kGb) {
-          if (do_gb && one_row) {
-            if constexpr (kCols <= kOneRowMaxCols<T>) {
-              const hipError_t attr = write_dx ? one_row_lds_limit<T, V, true>()
-                                               : one_row_lds_limit<T, V, false>();
-              HK_RETURN_IF_ERROR(attr);
-              k = write_dx ? ln_bwd_reg<T, V, true, true, kOneRowWaves, true>
-                           : ln_bwd_reg<T, V, false, true, kOneRowWaves, true>;
-            } else {
-              return hipErrorInvalidValue;  // the smallest VPL holding cols has kCols <= the cap
-            }
-          } else if (do_gb) {
-            if (waves != kW) return hipErrorInvalidValue;
-            k = write_dx ? ln_bwd_reg<T, V, true, true, kW> : ln_bwd_reg<T, V, false, true, kW>;
-          }
-        }
-        if (do_gb && !kGb) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k, dim3(grid), dim3(waves * HK_WAVE), lds, stream,
-                           reinterpret_cast<const uint4*>(dy), reinterpret_cast<const uint4*>(x),
-                           mean, rstd, reinterpret_cast<const uint4*>(gamma),
-                           reinterpret_cast<uint4*>(dx), part, rows, nvec, inv_cols);
+        hipLaunchKernelGGL((vec ? ln_bwd_few_rows<T, V, false> : ln_bwd_few_rows<T, V, true>),
+                           dim3(grid), dim3(kFinCols * kFinGroups), 0, stream, dy, x, mean, rstd,
+                           gamma, dx, dgamma, dbeta, rows, cols, inv_cols, row_groups);
         return hk::launch_status();
       }
-    }));
-    if (do_gb) {
-      hipLaunchKernelGGL(ln_gb_finalize,
-                         dim3(static_cast<unsigned>(hk::ceil_div(2 * cols, kFinCols))),
-                         dim3(kFinCols * kFinGroups), 0, stream, part, grid, cols, dgamma, dbeta);
-      HK_RETURN_IF_ERROR(hk::launch_status());
-    }
-    return hipSuccess;
+    });
   }
-  if (write_dx) {
-    hipLaunchKernelGGL(ln_bwd_input_rowblock<T>, dim3(rows), dim3(kThreads), 0, stream, dy, x,
-                       mean, rstd, gamma, dx, cols);
+  // Whole vectors of up to kMaxGbCols columns have always used the stream's workspace. The other
+  // shapes do without it while a graph is being captured: the graph would keep its address, and a
+  // later call may grow it.
+  const bool capturing = (!vec || cols > kMaxGbCols) && hk::stream_capturing(stream);
+  if (cols >= T::kPerVec && cols <= kMaxWideCols && !capturing) {
+    GbForm<T> f;
+    HK_RETURN_IF_ERROR(vec ? (gb_form<T, false>(rows, cols, write_dx, &f))
+                           : (gb_form<T, true>(rows, cols, write_dx, &f)));
+    void* ws = nullptr;
+    HK_RETURN_IF_ERROR(hk::device_workspace(static_cast<size_t>(f.grid) * 2 * cols * sizeof(float),
+                                            stream, &ws));
+    float* part = static_cast<float*>(ws);
+    hipLaunchKernelGGL(f.kernel, dim3(f.grid), dim3(f.waves * HK_WAVE), f.lds, stream, dy, x, mean,
+                       rstd, gamma, dx, part, rows, cols, inv_cols);
     HK_RETURN_IF_ERROR(hk::launch_status());
+    return launch_finalize<T>(part, f.grid, cols, dgamma, dbeta, stream);
   }
-  if (do_gb) {
-    hipLaunchKernelGGL(ln_gb_columns<T>, dim3(static_cast<unsigned>(hk::ceil_div(cols, kThreads))),
-                       dim3(kThreads), 0, stream, dy, x, mean, rstd, dgamma, dbeta, rows, cols);
-    HK_RETURN_IF_ERROR(hk::launch_status());
+  if (write_dx)
+    HK_RETURN_IF_ERROR(launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream));
+  // slabs of at least 16 rows, at most four workgroups per CU
+  const int64_t blocks = hk::ceil_div(cols, kThreads);
+  int64_t nslab = capturing ? 1 : hk::ceil_div(4 * static_cast<int64_t>(hk::device_cu_count()), blocks);
+  if (nslab > hk::ceil_div(rows, 16)) nslab = hk::ceil_div(rows, 16);
+  const int slab = static_cast<int>(hk::ceil_div(rows, nslab));
+  nslab = hk::ceil_div(rows, slab);
+  float* part = nullptr;
+  if (nslab > 1) {
+    void* ws = nullptr;
+    HK_RETURN_IF_ERROR(hk::device_workspace(static_cast<size_t>(nslab) * 2 * cols * sizeof(float),
+                                            stream, &ws));
+    part = static_cast<float*>(ws);
   }
+  hipLaunchKernelGGL(ln_gb_slab<T>,
+                     dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(nslab)),
+                     dim3(kThreads), 0, stream, dy, x, mean, rstd, part, dgamma, dbeta, rows, cols,
+                     slab);
+  HK_RETURN_IF_ERROR(hk::launch_status());
+  if (nslab > 1)
+    return launch_finalize<T>(part, static_cast<int>(nslab), cols, dgamma, dbeta, stream);
   return hipSuccess;
 }
 
