@@ -97,8 +97,14 @@ class HKError(RuntimeError):
         self.status = status
 
 
+_fns: dict[str, object] = {}  # bound entry points by name
+
+
 def call(fn: str, *args) -> None:
     """Calls one entry point and raises HKError on a non-success status."""
-    status = getattr(lib(), fn)(*args)
+    f = _fns.get(fn)
+    if f is None:
+        f = _fns[fn] = getattr(lib(), fn)
+    status = f(*args)
     if status != 0:
         raise HKError(fn, status)
