@@ -898,11 +898,7 @@ Rows packed_rows(bool ta, bool tb, int M, int N, int K) {
                   static_cast<int64_t>(M) * N, true, true, true);
 }
 
-// How a product runs: on the 256-wide tiles (flex == 0) or on tile shape `flex` of
-// bgemm_flex.hip, in `used` k splits of kps.
-struct Plan {
-  int flex, used, kps;
-};
+using Plan = hk::GemmPlan;
 
 // Modelled time (us) of the 256-wide tiles' plan for one k split (auto_split_k covers the others),
 // with the tile shape run_regions picks.
@@ -1026,21 +1022,31 @@ void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, in
   *used = static_cast<int>(hk::ceil_div(K, *kps));
 }
 
+GemmPlan bgemm_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_k) {
+  return make_plan(ta, tb, M, N, K, batch, split_k, Rows::kAligned);
+}
+
 hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* A, int64_t lda,
                           int64_t sA, const hk_bf16* B, int64_t ldb, int64_t sB, int batch,
-                          int used, int kps, float* part, const F32Out* out,
+                          const GemmPlan& plan, float* part, const F32Out* out,
                           hipStream_t stream) {
+  const int used = plan.used, kps = plan.kps;
   const int contig_a = ta ? M : K, contig_b = tb ? K : N;
-  HK_CHECK_ARG(M > 0 && N > 0 && K > 0 && batch > 0 && used >= 1 && kps % BK == 0);
+  HK_CHECK_ARG(M > 0 && N > 0 && K > 0 && batch > 0 && used >= 1 && (used == 1 || kps % BK == 0));
   HK_CHECK_ARG(contig_a % 8 == 0 && contig_b % 8 == 0 && N % 8 == 0 && lda % 8 == 0 &&
                ldb % 8 == 0 && sA % 8 == 0 && sB % 8 == 0 && hk::aligned16(A) &&
                hk::aligned16(B) && lda < (1 << 22) && ldb < (1 << 22));
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batch) * used <= 65535);
+  if (plan.flex)
+    return bgemm_flex_run(plan.flex,
+                          FlexCall{ta, tb, M, N, K, batch, A, lda, sA, B, ldb, sB, nullptr, 0, 0,
+                                   nullptr, used, kps, part, out},
+                          stream);
   const Epi ep{1.0f, 0.0f, nullptr, 0, 0, false};
   const F32Out fo = used == 1 && out ? *out : F32Out{};
   return run_regions<true>(ta, tb, batch * used, stream, M, N, K, ep, A, lda, sA, B, ldb, sB,
-                           nullptr, 0, 0, used, kps, part, fo);
+                           nullptr, 0, 0, used, used == 1 ? K : kps, part, fo);
 }
 
 }  // namespace hk

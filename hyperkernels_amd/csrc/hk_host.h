@@ -59,14 +59,20 @@ struct F32Out {
 // fp32 product of bf16 operands on the BF16 GEMM tiles (bgemm.hip), written as split-K partials
 // part[s][batch][M][N] (s < used) of op(A) op(B) over k-range [s kps, (s + 1) kps); their sum
 // in split order is the product. With used == 1 and out != NULL the tiles write out->C through
-// its epilogue instead (part is not touched). Needs the tiled path's alignment: 8-element
-// multiples and 16-byte aligned bases. bgemm_split_plan picks (used, kps) for a shape: split_k
-// ranges of kps k each (split_k == 0: the library's choice), `used` of them non-empty.
+// its epilogue instead (part is not touched). Needs whole, 16-byte aligned rows: 8-element
+// multiples and 16-byte aligned bases. bgemm_plan picks how a shape runs: the tile family (flex:
+// a tile shape of bgemm_flex.hip, 0 for the 256-wide tiles), and split_k ranges of kps k each
+// (split_k == 0: the library's choice), `used` of them non-empty. bgemm_split_plan does so for the
+// 256-wide tiles alone; cost: the modelled time (us) of split_k == 0.
+struct GemmPlan {
+  int flex, used, kps;
+};
+GemmPlan bgemm_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_k);
 void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, int* kps,
-                      double* cost = nullptr);  // cost: the modelled time (us) of split_k == 0
+                      double* cost = nullptr);
 hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* A, int64_t lda,
                           int64_t sA, const hk_bf16* B, int64_t ldb, int64_t sB, int batch,
-                          int used, int kps, float* part, const F32Out* out,
+                          const GemmPlan& plan, float* part, const F32Out* out,
                           hipStream_t stream);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

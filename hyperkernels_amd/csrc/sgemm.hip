@@ -12,7 +12,7 @@
 //   tile-specialised kernels (sgemm_nn_256x128_..., sgemm_nt_..., sgemm_tn_...): the same
 //       product without bias for one layout each; splitK where the reference has it.
 // The reference multiplies with single-pass TF32 MMA; gfx950 has no TF32 matrix instruction.
-// Two paths:
+// Three paths:
 //   bf16x3 (shapes whose dimensions are multiples of 8, the common case): A and B are split into
 //     bf16 hi / lo operands over a tripled k axis (split3) so that one bf16 GEMM on the BF16 GEMM
 //     tiles of this library (bgemm.hip) sums ah bh + ah bl + al bh in fp32. With one k split
@@ -22,6 +22,7 @@
 //     MFMA. Roofline: the bf16 peak / 3 (three products per fp32 product).
 //   fp32 MFMA tiles (other 4-element-aligned shapes): v_mfma_f32_32x32x2_f32, exact fp32
 //     products; roofline the fp32 matrix peak (157.3 TFLOP/s).
+// sgemm_flex.hip: the same on smaller tiles and rows of any length and alignment.
 //
 // Design of the fp32 tiles (gfx950): the same tiling as the BF16 GEMM of this library - 256 x 256 workgroup
 // tile, 8 waves of 128 x 64 (2 x 4, two per SIMD; 4 x 2 MFMA tiles, 128 fp32 accumulators per
@@ -40,6 +41,7 @@
 
 #include "hk_device.h"
 #include "hk_host.h"
+#include "sgemm_flex.h"
 
 namespace {
 
@@ -405,7 +407,8 @@ hipError_t launch_finalize(hipStream_t stream, const float* part, int used, int 
   return hk::launch_status();
 }
 
-// Fallback for shapes the tiled kernel does not take: one thread per output, k-order fp32 sum.
+// Fallback for K == 0 and leading dimensions that no tile takes (under 4, from 2^21 on): one thread
+// per output, k-order fp32 sum.
 __global__ __launch_bounds__(256) void sgemm_simple(int ta, int tb, int M, int N, int K,
                                                     const float* __restrict__ A, int64_t lda,
                                                     int64_t sA, const float* __restrict__ B,
@@ -536,29 +539,36 @@ hipError_t dispatch_layout(bool ta, bool tb, dim3 grid, hipStream_t stream, int 
                                       ep, split_k, kps, part);
 }
 
-// The three product paths of an fp32 GEMM and the k-split plan each runs.
-enum class SgemmPath { kSimple, kBf16x3, kFp32Tiles };
+// The product paths of an fp32 GEMM and the k-split plan each runs.
+enum class SgemmPath { kSimple, kFlex, kBf16x3, kFp32Tiles };
 
-// Which path takes a product. Tiles: 4-element multiples for every contiguous extent, leading
+// Which path takes a product. kFlex: the fp32 MFMA tiles of sgemm_flex.hip, any alignment; it also
+// takes the products of 4-element multiples that leave a quarter of the CUs without a 256 x 256
+// tile, unless the caller gives the split. Tiles: 4-element multiples for every contiguous extent, leading
 // dimension and batch stride, 16-byte aligned bases. bf16x3 additionally needs every dimension
 // the split copies touch to be a multiple of 8 and the tripled k axis to fit the BF16 tiles'
 // 32-bit per-lane offsets.
 SgemmPath sgemm_path(bool ta, bool tb, int M, int N, int K, int64_t lda, int64_t ldb,
                      int64_t ldc, int64_t sA, int64_t sB, int64_t sC, int batchCount,
-                     bool aligned) {
+                     bool aligned, int split_k) {
   const int contig_a = ta ? M : K, contig_b = tb ? K : N;
   const bool tiled_ok = (contig_a % 4 == 0) && (contig_b % 4 == 0) && (N % 4 == 0) &&
                         (lda % 4 == 0) && (ldb % 4 == 0) && (ldc % 4 == 0) && (sA % 4 == 0) &&
                         (sB % 4 == 0) && (sC % 4 == 0) && aligned && K > 0 &&
                         // per-lane source offsets inside a tile are 32-bit byte offsets
                         lda < (1 << 21) && ldb < (1 << 21);
-  if (!tiled_ok) return SgemmPath::kSimple;
+  const bool flex_ok = K > 0 && lda >= 4 && ldb >= 4 && lda < (1 << 21) && ldb < (1 << 21) &&
+                       batchCount <= 65535;
+  if (!tiled_ok) return flex_ok ? SgemmPath::kFlex : SgemmPath::kSimple;
   const bool x3_ok = K % 8 == 0 && N % 8 == 0 && (!ta || M % 8 == 0) &&
                      3LL * K < (1 << 22) && (ta ? M : 3LL * K) < (1 << 22) &&
                      (tb ? 3LL * K : N) < (1 << 22) && batchCount <= 65535 &&
                      static_cast<int64_t>(M) * K < (int64_t{1} << 33) &&
                      static_cast<int64_t>(K) * N < (int64_t{1} << 33);
-  return x3_ok ? SgemmPath::kBf16x3 : SgemmPath::kFp32Tiles;
+  if (x3_ok) return SgemmPath::kBf16x3;
+  const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN) * batchCount;
+  return split_k == 0 && flex_ok && 4 * tiles < 3 * hk::device_cu_count() ? SgemmPath::kFlex
+                                                                          : SgemmPath::kFp32Tiles;
 }
 
 // k-split plan of the fp32 MFMA tiles (BK = 32 fp32 per k-tile): split_k ranges of kps k, the
@@ -595,7 +605,8 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
   const Epilogue ep{alpha, beta, bias, bias ? static_cast<int64_t>(bias_stride) : 0, bias_scale};
   const SgemmPath path = sgemm_path(ta, tb, M, N, K, lda, ldb, ldc, strideA, strideB, strideC,
                                     batchCount,
-                                    hk::aligned16(A) && hk::aligned16(B) && hk::aligned16(C));
+                                    hk::aligned16(A) && hk::aligned16(B) && hk::aligned16(C),
+                                    splitK);
   if (path == SgemmPath::kSimple) {
     dim3 grid((N + 15) / 16, (M + 15) / 16, batchCount);
     hipLaunchKernelGGL(sgemm_simple, grid, dim3(256), 0, stream, ta ? 1 : 0, tb ? 1 : 0, M, N, K,
@@ -603,6 +614,16 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
                        static_cast<int64_t>(ldb), static_cast<int64_t>(strideB), C,
                        static_cast<int64_t>(ldc), static_cast<int64_t>(strideC), ep);
     return hk::launch_status();
+  }
+  if (path == SgemmPath::kFlex) {
+    double cost = 0.0;
+    const int shape = hk::sgemm_flex_plan(M, N, K, batchCount, &cost);
+    return hk::sgemm_flex_run(
+        shape,
+        hk::SgemmFlexCall{ta, tb, M, N, K, batchCount, A, lda, strideA, B, ldb, strideB,
+                          hk::F32Out{C, ldc, strideC, ep.alpha, ep.beta, ep.bias, ep.bias_stride,
+                                     ep.bias_scale}},
+        stream);
   }
   // bf16x3 on the BF16 GEMM tiles when every dimension the split copies touch is a multiple
   // of 8: A and B are split into bf16 hi / lo operands over a tripled k axis and multiplied on
@@ -614,8 +635,8 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
     // A' is [M][3K] (k-major) or [3K][M]; B' is [3K][N] or [N][3K]
     const int64_t la = ta ? M : K3, lb = tb ? K3 : N;
     const int64_t na = static_cast<int64_t>(M) * K3, nb = static_cast<int64_t>(K3) * N;
-    int used = 1, kps = 0;
-    hk::bgemm_split_plan(M, N, K3, batchCount, splitK, &used, &kps);
+    const hk::GemmPlan plan = hk::bgemm_plan(ta, tb, M, N, K3, batchCount, splitK);
+    const int used = plan.used, kps = plan.kps;
     // the plan never exceeds the k-tile count; refuse a grid the tiles cannot take before
     // anything is allocated or launched
     HK_CHECK_ARG(static_cast<int64_t>(batchCount) * used <= 65535);
@@ -627,7 +648,8 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
     // finalize pass. 4096^3 + bias at split-K 4: 489.7 -> 462.8 us, max-rel vs a float64
     // product 2.9e-6 both ways. Fewer tiles than CUs keep concurrent partials.
     const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const bool serial = used > 1 && tiles * batchCount >= hk::device_cu_count();
+    const bool serial =
+        used > 1 && plan.flex == 0 && tiles * batchCount >= hk::device_cu_count();
     // one split (or serial ranges): the GEMM tiles write C themselves, no partials
     const int64_t p_bytes =
         used == 1 || serial ? 0 : static_cast<int64_t>(used) * batchCount * M * N * 4;
@@ -668,15 +690,13 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
           o.beta = 1.0f;
           o.bias = nullptr;
         }
-        constexpr int kBf16KTile = 64;  // the BF16 tiles' k step: kps must be a multiple
-        HK_RETURN_IF_ERROR(hk::bgemm_partials(
-            ta, tb, M, N, kr, Ar, la, na, Br, lb, nb, batchCount, 1,
-            (kr + kBf16KTile - 1) / kBf16KTile * kBf16KTile, nullptr, &o, stream));
+        HK_RETURN_IF_ERROR(hk::bgemm_partials(ta, tb, M, N, kr, Ar, la, na, Br, lb, nb, batchCount,
+                                              hk::GemmPlan{0, 1, kr}, nullptr, &o, stream));
       }
       return hipSuccess;
     }
-    HK_RETURN_IF_ERROR(hk::bgemm_partials(ta, tb, M, N, K3, A3, la, na, B3, lb, nb, batchCount,
-                                          used, kps, part, &out, stream));
+    HK_RETURN_IF_ERROR(hk::bgemm_partials(ta, tb, M, N, K3, A3, la, na, B3, lb, nb, batchCount, plan,
+                                          part, &out, stream));
     if (used == 1) return hipSuccess;
     return launch_finalize(stream, part, used, batchCount, M, N, C, static_cast<int64_t>(ldc),
                            static_cast<int64_t>(strideC), ep);
@@ -718,10 +738,10 @@ extern "C" int hk_sgemm_split_count(int layout, int M, int N, int K, int batchCo
   const int64_t lda = ta ? M : K, ldb = tb ? K : N;
   const SgemmPath path = sgemm_path(ta, tb, M, N, K, lda, ldb, N, lda * (ta ? K : M),
                                     ldb * (tb ? N : K), static_cast<int64_t>(M) * N, batchCount,
-                                    true);
+                                    true, splitK);
   int used = 1, kps = 0;
   if (path == SgemmPath::kBf16x3)
-    hk::bgemm_split_plan(M, N, 3 * K, batchCount, splitK, &used, &kps);
+    used = hk::bgemm_plan(ta, tb, M, N, 3 * K, batchCount, splitK).used;
   else if (path == SgemmPath::kFp32Tiles)
     fp32_split_plan(M, N, K, batchCount, splitK, &used, &kps);
   return used;

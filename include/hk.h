@@ -423,11 +423,12 @@ HK_API hipError_t hk_bgemm_core_bias(int layout, int splitK, int M, int N, int K
  *   the library's choice.
  * hk_sgemm_split_count (no counterpart in the reference: a host-only planning query) returns
  *   the number of k splits hk_sgemm / hk_sgemm_layout run for this shape and splitK
- *   (contiguous operands, 16-byte aligned): 1 on the k-order fallback, 0 for an empty product,
- *   -1 for an invalid argument. hk_sgemm_addmm runs with splitK = 0.
- * Any M, N, K; the MFMA path needs the contiguous extents, leading dimensions and strides to
- * be multiples of 4 and 16-byte aligned pointers (sgemm_test.cu:240-243); other shapes run on a
- * slower k-order kernel.
+ *   (contiguous operands, 16-byte aligned): 1 on the k-order fallback and on the tiles for rows of
+ *   any alignment, 0 for an empty product, -1 for an invalid argument. hk_sgemm_addmm runs with
+ *   splitK = 0.
+ * Any M, N, K, leading dimension and stride (the reference needs multiples of 4 and 16-byte aligned
+ * pointers, sgemm_test.cu:240-243): shapes that the bf16x3 path does not take run on exact fp32 MFMA
+ * products; leading dimensions under 4 or from 2^21 on on a slower k-order kernel.
  * ---------------------------------------------------------------------------------------- */
 HK_API hipError_t hk_sgemm(int layout, int M, int N, int K, float alpha, const float* A, int lda,
                            long long strideA, const float* B, int ldb, long long strideB,
