@@ -72,10 +72,28 @@ __device__ __forceinline__ float dot8(const uint4& a, const uint4& b) {
   return s;
 }
 
+// How 16-byte vectors of a row are loaded: not at all (element loads: a strided x), from 16-byte
+// aligned addresses, or from any 2-byte address. gfx950 serves unaligned 16-byte loads at close to
+// the aligned rate: 50304 x 921 (rows of odd length), two of them, 81 -> 17 us on MI355X.
+enum Rows { kElements, kAligned, kAnywhere };
+typedef uint32_t u32x4a2_t __attribute__((ext_vector_type(4), aligned(2)));
+template <int ROWS>
+__device__ __forceinline__ uint4 load8_nt(const uint16_t* p) {
+  if (ROWS == kAligned) return hk::ld_nt(reinterpret_cast<const uint4*>(p));
+  const u32x4a2_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4a2_t*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <int ROWS>
+__device__ __forceinline__ uint4 load8(const uint16_t* p) {
+  if (ROWS == kAligned) return *reinterpret_cast<const uint4*>(p);
+  const u32x4a2_t v = *reinterpret_cast<const u32x4a2_t*>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // ---- dot form --------------------------------------------------------------------------------
-// grid: (ceil(R / 16), nsplit, batch). VEC: matrix rows and x start 16-byte aligned (ld, sM,
-// sx multiples of 8, incx == 1); otherwise element loads.
-template <bool VEC>
+// grid: (ceil(R / 16), nsplit, batch). kAligned: matrix rows and x start 16-byte aligned (ld, sM,
+// sx multiples of 8); kAnywhere and kAligned need incx == 1.
+template <int ROWS>
 __global__ __launch_bounds__(kThreads) void gemv_dot(int R, int K, int kchunk,
                                                      const uint16_t* __restrict__ mtx,
                                                      int64_t ld, int64_t sm,
@@ -90,7 +108,7 @@ __global__ __launch_bounds__(kThreads) void gemv_dot(int R, int K, int kchunk,
   if (r < R) {
     const uint16_t* row = mtx + b * sm + static_cast<int64_t>(r) * ld;
     const uint16_t* xb = x + b * sx;
-    if (VEC) {
+    if (ROWS != kElements) {
       const int kvec = kbeg + ((kend - kbeg) & ~7);  // end of the whole 8-element vectors
       // kUnroll vectors in flight per lane, the last round predicated
       for (int k = kbeg + 8 * j; k < kvec; k += kUnroll * kDotStep) {
@@ -98,8 +116,8 @@ __global__ __launch_bounds__(kThreads) void gemv_dot(int R, int K, int kchunk,
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
           if (k + u * kDotStep < kvec) {
-            m[u] = hk::ld_nt(reinterpret_cast<const uint4*>(row + k + u * kDotStep));
-            v[u] = *reinterpret_cast<const uint4*>(xb + k + u * kDotStep);
+            m[u] = load8_nt<ROWS>(row + k + u * kDotStep);
+            v[u] = load8<ROWS>(xb + k + u * kDotStep);
           }
         }
 #pragma unroll
@@ -118,9 +136,9 @@ __global__ __launch_bounds__(kThreads) void gemv_dot(int R, int K, int kchunk,
 }
 
 // ---- bcast form ------------------------------------------------------------------------------
-// grid: (ceil(R / 512), nsplit, batch). VEC: matrix rows start 16-byte aligned (ld, sM
-// multiples of 8); the workgroup whose 512 outputs cross R loads element by element.
-template <bool VEC>
+// grid: (ceil(R / 512), nsplit, batch). kAligned: matrix rows start 16-byte aligned (ld, sM
+// multiples of 8), else kAnywhere; the workgroup whose 512 outputs cross R loads element by element.
+template <int ROWS>
 __global__ __launch_bounds__(kBcastThreads) void gemv_bcast(int R, int K, int kchunk,
                                                        const uint16_t* __restrict__ mtx,
                                                        int64_t ld, int64_t sm,
@@ -137,7 +155,7 @@ __global__ __launch_bounds__(kBcastThreads) void gemv_bcast(int R, int K, int kc
   const uint16_t* xb = x + b * sx;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   int k = kbeg + wave;
-  if (VEC && static_cast<int>(blockIdx.x + 1) * kColsPerWave <= R) {
+  if (static_cast<int>(blockIdx.x + 1) * kColsPerWave <= R) {
     // Every lane of the workgroup owns 8 outputs (uniform branch). Whole rounds: kUnroll rows
     // of 16 bytes in flight per lane with no condition between them; the round's kUnroll x
     // values come from one load spread over the first lanes, broadcast with readlane, so no
@@ -147,7 +165,7 @@ __global__ __launch_bounds__(kBcastThreads) void gemv_bcast(int R, int K, int kc
       uint4 m[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u)
-        m[u] = hk::ld_nt(reinterpret_cast<const uint4*>(base + (k + u * kWaves) * ld));
+        m[u] = load8_nt<ROWS>(base + (k + u * kWaves) * ld);
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         const float xv =
@@ -160,13 +178,13 @@ __global__ __launch_bounds__(kBcastThreads) void gemv_bcast(int R, int K, int kc
     }
     for (; k < kend; k += kWaves) {  // fewer than kUnroll rows left
       float f[8];
-      hk::BF16::unpack(hk::ld_nt(reinterpret_cast<const uint4*>(base + k * ld)), f);
+      hk::BF16::unpack(load8_nt<ROWS>(base + k * ld), f);
       const float xv = hk::bf16_to_f32(xb[k * incx]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] += xv * f[i];
     }
   } else if (n0 < R) {
-    // the strip that straddles R, or rows that are not 16-byte aligned: element loads
+    // the strip that straddles R: element loads
     for (; k < kend; k += kWaves) {
       const float xv = hk::bf16_to_f32(xb[k * incx]);
       const uint16_t* rowp = base + k * ld;
@@ -271,13 +289,14 @@ hipError_t bgemv_run(bool dot_form, int R, int K, hk_bf16 alpha, hk_bf16 beta,
   const dim3 grid(static_cast<unsigned>(strips), static_cast<unsigned>(nsplit),
                   static_cast<unsigned>(batch));
   if (dot_form) {
-    const bool vec = ld % 8 == 0 && sm % 8 == 0 && incx == 1 && sx % 8 == 0 &&
-                     hk::aligned16(mtx) && hk::aligned16(x);
-    hipLaunchKernelGGL(vec ? gemv_dot<true> : gemv_dot<false>, grid, dim3(kThreads), 0, stream, R,
+    const bool vec = ld % 8 == 0 && sm % 8 == 0 && sx % 8 == 0 && hk::aligned16(mtx) &&
+                     hk::aligned16(x);
+    auto* k = incx != 1 ? gemv_dot<kElements> : vec ? gemv_dot<kAligned> : gemv_dot<kAnywhere>;
+    hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, stream, R,
                        K, kchunk, mtx, ld, sm, x, incx, sx, out);
   } else {
     const bool vec = ld % 8 == 0 && sm % 8 == 0 && hk::aligned16(mtx);
-    hipLaunchKernelGGL(vec ? gemv_bcast<true> : gemv_bcast<false>, grid, dim3(kBcastThreads), 0,
+    hipLaunchKernelGGL(vec ? gemv_bcast<kAligned> : gemv_bcast<kAnywhere>, grid, dim3(kBcastThreads), 0,
                        stream, R, K, kchunk, mtx, ld, sm, x, incx, sx, out);
   }
   HK_RETURN_IF_ERROR(hk::launch_status());
