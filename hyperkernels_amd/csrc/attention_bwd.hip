@@ -32,7 +32,8 @@
 // with no exchange between waves. The two query halves' dK / dV partials are summed through LDS
 // at the end. 128-key tiles mean 8 dQ passes per query row at T = 1024 (the reference's 16-key tiles
 // make 64). Workgroups are ordered key tile major, so under causal masking the longest ones are
-// dispatched first.
+// dispatched first. Few heads share each key tile's queries between workgroups (Deal, pick_chunk).
+#include <initializer_list>
 #include <mutex>
 
 #include "hk_device.h"
@@ -180,6 +181,24 @@ struct QPlanes {
   const float* d;
 };
 
+// How the (key tile, query tile) pairs of a head are dealt to workgroups. A workgroup owns a key tile
+// and at most `chunk` of its query tiles; a key tile of several workgroups has its dK / dV summed
+// from partials ([item][b, h][dK, dV][128 keys][64], fp32) in item order by attn_bwd_sum. A head's
+// items are numbered key tile by key tile.
+struct Deal {
+  int chunk;    // query tiles per workgroup
+  float* part;  // NULL when every key tile has one workgroup
+};
+// Query tiles of key tile kt: all of them, or under causal masking from the one that holds the
+// tile's first key.
+__host__ __device__ inline int query_tiles(int64_t T, bool causal, int kt) {
+  const int64_t first = causal ? static_cast<int64_t>(kt) * kBKV / kBQ * kBQ : 0;
+  return static_cast<int>((T - first + kBQ - 1) / kBQ);
+}
+__host__ __device__ inline int key_items(int64_t T, bool causal, int kt, int chunk) {
+  return (query_tiles(T, causal, kt) + chunk - 1) / chunk;
+}
+
 // Vector memory operations each lane issues after a tile's copies: the dQ atomics. A wave
 // waits with vmcnt(kAtomicsPerTile) for its copies of the next tile (vector memory operations
 // complete in issue order), so the atomics themselves are never waited for.
@@ -188,7 +207,8 @@ constexpr int kAtomicsPerTile = 8;
 // The pre-pass: grid (ceil(T * 8 / 256), B * nh); thread t of the row-chunk index covers 8
 // consecutive d of one row of Q and of dO.
 __global__ __launch_bounds__(256) void attn_bwd_prepare(hk_attn_bwd_params p, char* qh, char* ql,
-                                                        char* oh, char* ol, float* l2, float* dd) {
+                                                        char* oh, char* ol, float* l2, float* dd,
+                                                        bool zero_dq) {
   const int bh = blockIdx.y;
   const int b = bh / p.nh, h = bh - b * p.nh;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -211,6 +231,17 @@ __global__ __launch_bounds__(256) void attn_bwd_prepare(hk_attn_bwd_params p, ch
   split8(xo, hi, lo);
   *reinterpret_cast<u32x4_t*>(oh + dst) = hi;
   *reinterpret_cast<u32x4_t*>(ol + dst) = lo;
+  if (zero_dq) {
+    float* z = p.dQ + b * p.dq_strideB + h * p.dq_strideH + row * p.dq_strideM + 8 * chunk;
+    if (((p.dq_strideB | p.dq_strideH | p.dq_strideM) & 3) == 0 &&
+        (reinterpret_cast<uintptr_t>(p.dQ) & 15) == 0) {
+      *reinterpret_cast<f32x4_t*>(z) = f32x4_t{};
+      *reinterpret_cast<f32x4_t*>(z + 4) = f32x4_t{};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) z[e] = 0.f;
+    }
+  }
   if (chunk == 0) {
     const int64_t r = static_cast<int64_t>(bh) * p.T + row;
     l2[r] = p.LSE[b * p.lse_strideB + h * p.lse_strideH + row] * kLog2e;
@@ -218,8 +249,11 @@ __global__ __launch_bounds__(256) void attn_bwd_prepare(hk_attn_bwd_params p, ch
   }
 }
 
+// RAGGED: T is no multiple of the query tile, so tiles end past T. SPLIT: several workgroups may
+// share a key tile (deal.part). Both off, the loop tests nothing per tile.
+template <bool RAGGED, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_params p, int nbh,
-                                                                QPlanes qp) {
+                                                                QPlanes qp, Deal deal) {
   extern __shared__ __attribute__((aligned(16))) char lds_generic[];
   char HK_LDS* lds = (char HK_LDS*)lds_generic;
   char HK_LDS* sKh = lds + kOffKh;
@@ -235,8 +269,18 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   // Linear order: all (batch, head)s of key tile 0 first, then key tile 1, ... Under causal
   // masking the first key tiles meet the most query tiles, so the hardware's in-order dispatch
   // hands out the longest workgroups first (longest-processing-time-first scheduling).
-  const int kt = static_cast<int>(blockIdx.x) / nbh;
-  const int bh = static_cast<int>(blockIdx.x) - kt * nbh;
+  const int item = static_cast<int>(blockIdx.x) / nbh;
+  const int bh = static_cast<int>(blockIdx.x) - item * nbh;
+  int kt = item, piece = 0, pieces = 1;
+  if (SPLIT) {
+    kt = 0;
+    piece = item;
+    for (pieces = key_items(T, p.is_causal, 0, deal.chunk); piece >= pieces;) {
+      piece -= pieces;
+      ++kt;
+      pieces = key_items(T, p.is_causal, kt, deal.chunk);
+    }
+  }
   const int b = bh / p.nh, h = bh - b * p.nh;
   const int64_t k0 = static_cast<int64_t>(kt) * kBKV;
 
@@ -251,18 +295,15 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   const int kg = wave & 3, qh = wave >> 2;
   const float sl2 = p.scale * kLog2e;
 
-  // K and V tiles (128 x 64) once
-  {
-    Stager<kBKV> st;
-    st.load(Kb, p.k_strideM, k0, T);
-    st.store(sKh, sKl);
-    st.load(Vb, p.v_strideM, k0, T);
-    st.store(sVh, sVl);
-  }
-
   // query tiles: causal starts at the tile holding the first key of this workgroup
-  const int64_t q_first = p.is_causal ? (k0 / kBQ) * kBQ : 0;
-  const int nq = static_cast<int>((T - q_first + kBQ - 1) / kBQ);
+  // (SPLIT: this workgroup's share of them, pieces of nearly equal length)
+  int64_t q_first = p.is_causal ? (k0 / kBQ) * kBQ : 0;
+  int nq = static_cast<int>((T - q_first + kBQ - 1) / kBQ);
+  if (SPLIT) {
+    const int qt0 = static_cast<int>(static_cast<int64_t>(nq) * piece / pieces);
+    nq = static_cast<int>(static_cast<int64_t>(nq) * (piece + 1) / pieces) - qt0;
+    q_first += static_cast<int64_t>(qt0) * kBQ;
+  }
   // Without causal masking every key tile of a head visits all query tiles; key tile kt starts
   // at query tile 2 kt (mod nq), so the key tiles of one head add into different dQ rows at
   // any one time (measured ~2% faster than all starting at tile 0).
@@ -281,7 +322,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   const int cchunk = (lane & 7) ^ swz(crow);
   const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
   auto copy_tile = [&](int64_t q0) {
-    const int64_t r = q0 + crow < T ? q0 + crow : T - 1;
+    const int64_t r = !RAGGED || q0 + crow < T ? q0 + crow : T - 1;
     const int voff = static_cast<int>(r * kRowBytes) + (cchunk << 4);
     const int64_t head = plane_row0 * kRowBytes;
     const unsigned dst = lds_base + 1024 * wave;
@@ -290,12 +331,21 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
     copy16_to_lds(qp.oh + head, voff, dst + kOffOh);
     copy16_to_lds(qp.ol + head, voff, dst + kOffOl);
     if (wave < 2) {
-      const int64_t rr = q0 + lane < T ? q0 + lane : T - 1;
+      const int64_t rr = !RAGGED || q0 + lane < T ? q0 + lane : T - 1;
       copy4_to_lds((wave == 0 ? qp.l2 : qp.d) + plane_row0, static_cast<int>(rr * 4),
                    lds_base + (wave == 0 ? kOffL : kOffD));
     }
   };
-  if (nq > 0) copy_tile(tile_q(0));
+  // K and V tiles (128 x 64) once: both are loaded, and the first query tile's copies issued, before
+  // the first of them is split, so a workgroup starts with one memory latency instead of three
+  {
+    Stager<kBKV> sk, sv;
+    sk.load(Kb, p.k_strideM, k0, T);
+    sv.load(Vb, p.v_strideM, k0, T);
+    if (nq > 0) copy_tile(tile_q(0));
+    sk.store(sKh, sKl);
+    sv.store(sVh, sVl);
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // dV, dK: C layout of (A = P^T or dS^T: rows = keys, B = dO or Q: columns = d):
@@ -362,7 +412,12 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
     // This tile's copies were issued before the previous tile's atomics: with those still in
     // flight they are done once at most kAtomicsPerTile operations are outstanding. The barrier
     // then publishes every wave's copies (and orders the previous tile's dQ exchange reads).
-    if (it > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAtomicsPerTile) : "memory");
+    if (it > 0) {
+      if (!RAGGED || tile_q(it - 1) + kBQ <= T)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAtomicsPerTile) : "memory");
+      else  // fewer atomics than that
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
     __syncthreads();
 
     // This wave's block: keys k0 + 32 kg .. + 31, queries q0 + 32 qh .. + 31. Under causal
@@ -538,22 +593,26 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
       __builtin_amdgcn_sched_barrier(0);
     }
     {
-      // dq[jb][r]: query 16 qb16 + 4 g16 + r, d 32 dh + 16 jb + j15. Every lane issues exactly
-      // kAtomicsPerTile atomics (the count the next tile's vmcnt wait assumes): a row past T
-      // adds 0 to row T - 1 instead.
+      // dq[jb][r]: query 16 qb16 + 4 g16 + r, d 32 dh + 16 jb + j15. In a whole tile every lane
+      // issues exactly kAtomicsPerTile atomics (the count the next tile's vmcnt wait assumes); a
+      // tile that ends past T adds its rows below T only, and the next tile waits for everything.
+      // (Adding 0 to row T - 1 for the others, to keep the count, put up to 63 x 64 adds of every
+      // key tile on 64 addresses: 36 of the 42 us of 2 x 12 heads at T = 333 on MI355X.)
       const int64_t qblk = q0 + 16 * qb16 + 4 * g16;
-      const int rows_left = T - qblk < 4 ? static_cast<int>(T - qblk) : 4;  // may be <= 0
       float* dqu = dQb + qblk * p.dq_strideM + 32 * dh + j15;
+      if (!RAGGED || q0 + kBQ <= T) {
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb)
+        for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const bool in = r < rows_left;
-          const float v = in ? dq[jb][r] * p.scale : 0.f;
-          float* dst = in ? dqu + r * p.dq_strideM + 16 * jb
-                          : dQb + (T - 1) * p.dq_strideM + 32 * dh + 16 * jb + j15;
-          unsafeAtomicAdd(dst, v);
-        }
+          for (int r = 0; r < 4; ++r)
+            unsafeAtomicAdd(dqu + r * p.dq_strideM + 16 * jb, dq[jb][r] * p.scale);
+      } else {
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (qblk + r < T) unsafeAtomicAdd(dqu + r * p.dq_strideM + 16 * jb, dq[jb][r] * p.scale);
+      }
     }
   }
 
@@ -572,7 +631,20 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
       }
   }
   __syncthreads();
-  if (qh == 0) {
+  if (SPLIT && qh == 0 && pieces > 1) {
+    float* dkp = deal.part + (static_cast<int64_t>(item) * nbh + bh) * (2 * kBKV * kHD) +
+                 (32 * kg + 4 * hh) * kHD + c;
+    float* dvp = dkp + kBKV * kHD;
+#pragma unroll
+    for (int d2 = 0; d2 < 2; ++d2)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int rs = 8 * (i >> 2) + (i & 3);
+        const int r = rs + 4 * hh;
+        dkp[rs * kHD + 32 * d2] = dk[d2][i] + pk[r * 65 + 32 * d2 + c];
+        dvp[rs * kHD + 32 * d2] = dv[d2][i] + pk[32 * 65 + r * 65 + 32 * d2 + c];
+      }
+  } else if (qh == 0) {
     float* dKb = p.dK + b * p.dk_strideB + h * p.dk_strideH;
     float* dVb = p.dV + b * p.dv_strideB + h * p.dv_strideH;
     const int64_t krow0 = k0 + 32 * kg + 4 * hh;
@@ -592,14 +664,74 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   }
 }
 
+// dK / dV of the key tiles that several workgroups share: the sum of their partials in item order,
+// dK scaled. Grid (key tiles x kSumBlocks, B * nh): a lane per 4 consecutive d of a key, dK in the
+// first half of a key tile's blocks, dV in the second.
+constexpr int kSumThreads = 256;
+constexpr int kSumBlocks = 2 * kBKV * kHD / 4 / kSumThreads;
+__global__ __launch_bounds__(kSumThreads) void attn_bwd_sum(hk_attn_bwd_params p, int nbh,
+                                                            Deal deal) {
+  const int kt = blockIdx.x / kSumBlocks, bh = blockIdx.y;
+  const int pieces = key_items(p.T, p.is_causal, kt, deal.chunk);
+  if (pieces == 1) return;
+  int item = 0;
+  for (int k = 0; k < kt; ++k) item += key_items(p.T, p.is_causal, k, deal.chunk);
+  const int idx = (blockIdx.x % kSumBlocks) * kSumThreads + threadIdx.x;
+  const bool is_dv = idx >= kBKV * kHD / 4;
+  const int i = idx - (is_dv ? kBKV * kHD / 4 : 0);
+  const int64_t key = static_cast<int64_t>(kt) * kBKV + i / (kHD / 4);
+  if (key >= p.T) return;
+  const int b = bh / p.nh, h = bh - b * p.nh;
+  const int64_t step = static_cast<int64_t>(nbh) * (2 * kBKV * kHD);
+  const float* s =
+      deal.part + (static_cast<int64_t>(item) * nbh + bh) * (2 * kBKV * kHD) + 4 * idx;
+  f32x4_t v = *reinterpret_cast<const f32x4_t*>(s);
+  for (int j = 1; j < pieces; ++j) v += *reinterpret_cast<const f32x4_t*>(s + j * step);
+  const float scale = is_dv ? 1.0f : p.scale;
+  float* d = (is_dv ? p.dV + b * p.dv_strideB + h * p.dv_strideH + key * p.dv_strideM
+                    : p.dK + b * p.dk_strideB + h * p.dk_strideH + key * p.dk_strideM) +
+             4 * (i % (kHD / 4));
+#pragma unroll
+  for (int e = 0; e < 4; ++e) d[e] = v[e] * scale;
+}
+
+// Query tiles per workgroup: the number with the least modelled time. A workgroup takes about 11 us
+// plus 3 us per query tile; the launch lasts as long as its longest workgroup and, with more
+// workgroups than CUs (one runs per CU), as the work per CU; a split adds the sum's 5 us. Large
+// grids stay unsplit. Whole backward on MI355X, us unsplit and as picked: 12 causal heads at
+// T = 1024 66.5 and 35.2 (4 tiles), 24 heads at T = 333 34.1 and 26.9 (2 tiles).
+int pick_chunk(int64_t T, bool causal, int nkt, int64_t nbh) {
+  const double cus = static_cast<double>(hk::device_cu_count());
+  const int most = query_tiles(T, causal, 0);
+  double best = 0.0;
+  int best_chunk = most;
+  if (nkt * nbh >= 4 * static_cast<int64_t>(cus)) return most;
+  for (int chunk = most; chunk >= 1; --chunk) {
+    int64_t wgs = 0, tiles = 0;
+    for (int kt = 0; kt < nkt; ++kt) {
+      wgs += key_items(T, causal, kt, chunk);
+      tiles += query_tiles(T, causal, kt);
+    }
+    if (wgs * nbh > 8 * static_cast<int64_t>(cus)) break;
+    const double longest = 11.0 + 3.0 * chunk;
+    const double share = (11.0 * static_cast<double>(wgs) + 3.0 * static_cast<double>(tiles)) *
+                         static_cast<double>(nbh) / cus;
+    double cost = wgs * nbh <= cus ? longest : (share > longest ? share : longest) + 0.3 * longest;
+    if (wgs > nkt) cost += 5.0;
+    if (chunk == most || cost < 0.95 * best) {
+      best = cost;
+      best_chunk = chunk;
+    }
+  }
+  return best_chunk;
+}
+
 bool rows_aligned(const void* base, int64_t strideB, int64_t strideH, int64_t strideM) {
   return hk::aligned16(base) && strideB % 4 == 0 && strideH % 4 == 0 && strideM % 4 == 0;
 }
 
-}  // namespace
-
-extern "C" hipError_t hk_attn_backward(const hk_attn_bwd_params* params, int head_dim,
-                                       hipStream_t stream) {
+hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool zero_dq,
+                         hipStream_t stream) {
   HK_CHECK_ARG(params != nullptr);
   const hk_attn_bwd_params& p = *params;
   HK_CHECK_ARG(head_dim == kHD);
@@ -617,29 +749,66 @@ extern "C" hipError_t hk_attn_backward(const hk_attn_bwd_params* params, int hea
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [] {
-    attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               static_cast<int>(kLdsBytes));
+    for (const void* k : {reinterpret_cast<const void*>(&attn_bwd_kernel<false, false>),
+                          reinterpret_cast<const void*>(&attn_bwd_kernel<false, true>),
+                          reinterpret_cast<const void*>(&attn_bwd_kernel<true, false>),
+                          reinterpret_cast<const void*>(&attn_bwd_kernel<true, true>)}) {
+      const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               static_cast<int>(kLdsBytes));
+      if (e != hipSuccess) attr = e;
+    }
   });
   HK_RETURN_IF_ERROR(attr);
   const int64_t nkt = (static_cast<int64_t>(p.T) + kBKV - 1) / kBKV;
   HK_CHECK_ARG(nkt * bh <= INT32_MAX);
-  // the query-side planes in the stream's workspace: 4 x [b, h][T][64] bf16, 2 x [b, h][T] fp32
+  // the query-side planes in the stream's workspace: 4 x [b, h][T][64] bf16, 2 x [b, h][T] fp32;
+  // then the partials of split key tiles, from a 256-byte boundary
   const int64_t rows = bh * p.T;
   const size_t plane = static_cast<size_t>(rows) * kRowBytes;
+  const size_t planes = (4 * plane + 2 * static_cast<size_t>(rows) * 4 + 255) & ~size_t{255};
+  Deal deal{pick_chunk(p.T, p.is_causal, static_cast<int>(nkt), bh), nullptr};
+  int64_t items = nkt;
+  if (deal.chunk < query_tiles(p.T, p.is_causal, 0)) {
+    items = 0;
+    for (int64_t kt = 0; kt < nkt; ++kt)
+      items += key_items(p.T, p.is_causal, static_cast<int>(kt), deal.chunk);
+  }
+  const bool split = items > nkt;
+  const size_t part_bytes =
+      split ? static_cast<size_t>(items * bh) * 2 * kBKV * kHD * sizeof(float) : 0;
   void* ws = nullptr;
-  HK_RETURN_IF_ERROR(hk::device_workspace(4 * plane + 2 * static_cast<size_t>(rows) * 4, stream,
-                                          &ws));
+  HK_RETURN_IF_ERROR(hk::device_workspace(planes + part_bytes, stream, &ws));
   char* wsb = static_cast<char*>(ws);
   float* l2 = reinterpret_cast<float*>(wsb + 4 * plane);
   hipLaunchKernelGGL(attn_bwd_prepare,
                      dim3(static_cast<unsigned>(hk::ceil_div(static_cast<int64_t>(p.T) * 8, 256)),
                           static_cast<unsigned>(bh)),
                      dim3(256), 0, stream, p, wsb, wsb + plane, wsb + 2 * plane, wsb + 3 * plane, l2,
-                     l2 + rows);
+                     l2 + rows, zero_dq);
   HK_RETURN_IF_ERROR(hk::launch_status());
   const QPlanes qp{wsb, wsb + plane, wsb + 2 * plane, wsb + 3 * plane, l2, l2 + rows};
-  hipLaunchKernelGGL(attn_bwd_kernel, dim3(static_cast<unsigned>(nkt * bh)), dim3(kThreads),
-                     kLdsBytes, stream, p, static_cast<int>(bh), qp);
+  if (split) deal.part = reinterpret_cast<float*>(wsb + planes);
+  const bool ragged = p.T % kBQ != 0;
+  auto* kernel = split ? (ragged ? attn_bwd_kernel<true, true> : attn_bwd_kernel<false, true>)
+                       : (ragged ? attn_bwd_kernel<true, false> : attn_bwd_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(items * bh)), dim3(kThreads), kLdsBytes,
+                     stream, p, static_cast<int>(bh), qp, deal);
+  HK_RETURN_IF_ERROR(hk::launch_status());
+  if (!split) return hipSuccess;
+  hipLaunchKernelGGL(attn_bwd_sum,
+                     dim3(static_cast<unsigned>(nkt * kSumBlocks), static_cast<unsigned>(bh)),
+                     dim3(kSumThreads), 0, stream, p, static_cast<int>(bh), deal);
   return hk::launch_status();
+}
+
+}  // namespace
+
+extern "C" hipError_t hk_attn_backward(const hk_attn_bwd_params* params, int head_dim,
+                                       hipStream_t stream) {
+  return attn_backward(params, head_dim, false, stream);
+}
+
+extern "C" hipError_t hk_attn_backward_set(const hk_attn_bwd_params* params, int head_dim,
+                                           hipStream_t stream) {
+  return attn_backward(params, head_dim, true, stream);
 }

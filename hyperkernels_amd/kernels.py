@@ -364,15 +364,17 @@ def attn_backward(q, k, v, do, lse, D, causal: bool, scale: float | None = None,
                   dv=None, o=None):
     """OwnTensor::mem_efficient_bwd_unified_kernel_exp12<64, Causal>: returns (dQ, dK, dV).
 
-    dK and dV are written; dQ is ADDED into (zeroed here when not passed in), as in the
-    reference where the caller zeroes dQ before the launch."""
+    dK and dV are written; dQ is ADDED into, as in the reference where the caller zeroes dQ before
+    the launch, or written when it is not passed in."""
     B, H, T, Dh = q.shape
     scale = Dh ** -0.5 if scale is None else scale
-    dq = torch.zeros_like(q) if dq is None else dq
+    fn = "hk_attn_backward"
+    if dq is None:
+        dq, fn = torch.empty_like(q), "hk_attn_backward_set"
     dk = torch.empty_like(k) if dk is None else dk
     dv = torch.empty_like(v) if dv is None else dv
     p = _bwd_params(q, k, v, o, do, lse, D, dq, dk, dv, causal, scale)
-    call("hk_attn_backward", ctypes.byref(p), Dh, _stream())
+    call(fn, ctypes.byref(p), Dh, _stream())
     return dq, dk, dv
 
 

@@ -525,6 +525,10 @@ HK_API hipError_t hk_attn_bwd_precompute_D(const hk_attn_bwd_params* params, int
                                            hipStream_t stream);
 HK_API hipError_t hk_attn_backward(const hk_attn_bwd_params* params, int head_dim,
                                    hipStream_t stream);
+/* hk_attn_backward_set (no counterpart in the reference) is hk_attn_backward for callers that do
+ * not accumulate: dQ is written, whatever it held before, without a clearing launch of its own. */
+HK_API hipError_t hk_attn_backward_set(const hk_attn_bwd_params* params, int head_dim,
+                                       hipStream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * Measurement
