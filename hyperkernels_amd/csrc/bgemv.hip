@@ -135,6 +135,69 @@ __global__ __launch_bounds__(kThreads) void gemv_dot(int R, int K, int kchunk,
   if (r < R && j == 0) emit(out, b, s, R, r, acc);
 }
 
+// Batches that share one matrix: a workgroup multiplies its rows with NB of their vectors, so the
+// matrix is read once for them. grid: (ceil(R / 16), nsplit, ceil(batch / NB)); sums in the order of
+// gemv_dot. (One kernel for every NB made a single vector 0.2 us slower, 50257 x 768: a longer
+// prologue before its first load.)
+template <int ROWS, int NB>
+__global__ __launch_bounds__(kThreads) void gemv_dot_shared(int R, int K, int kchunk, int batch,
+                                                            const uint16_t* __restrict__ mtx,
+                                                            int64_t ld,
+                                                            const uint16_t* __restrict__ x,
+                                                            int64_t incx, int64_t sx, Out out) {
+  constexpr int kLoads = kUnroll / 2;  // matrix vectors in flight per lane
+  const int b0 = blockIdx.z * NB, s = blockIdx.y;
+  const int j = threadIdx.x & (kDotLanes - 1);
+  const int r = blockIdx.x * kDotRows + (threadIdx.x >> 4);
+  const int kbeg = s * kchunk;
+  const int kend = min(K, kbeg + kchunk);
+  float acc[NB] = {};
+  if (r < R) {
+    const uint16_t* row = mtx + static_cast<int64_t>(r) * ld;
+    const uint16_t* xb[NB];  // past the last batch: the last one again, not stored
+#pragma unroll
+    for (int n = 0; n < NB; ++n) xb[n] = x + min(b0 + n, batch - 1) * sx;
+    if (ROWS != kElements) {
+      const int kvec = kbeg + ((kend - kbeg) & ~7);  // end of the whole 8-element vectors
+      // kLoads vectors in flight per lane, the last round predicated
+      for (int k = kbeg + 8 * j; k < kvec; k += kLoads * kDotStep) {
+        uint4 m[kLoads], v[kLoads][NB];
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+          if (k + u * kDotStep < kvec) {
+            m[u] = load8_nt<ROWS>(row + k + u * kDotStep);
+#pragma unroll
+            for (int n = 0; n < NB; ++n) v[u][n] = load8<ROWS>(xb[n] + k + u * kDotStep);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+          if (k + u * kDotStep < kvec) {
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[n] += dot8(m[u], v[u][n]);
+          }
+      }
+      if (kvec + j < kend) {
+        const float m = hk::bf16_to_f32(row[kvec + j]);
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[n] += m * hk::bf16_to_f32(xb[n][kvec + j]);
+      }
+    } else {
+      for (int k = kbeg + j; k < kend; k += kDotLanes) {
+        const float m = hk::bf16_to_f32(row[k]);
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[n] += m * hk::bf16_to_f32(xb[n][k * incx]);
+      }
+    }
+  }
+  static_assert(kDotLanes == 16, "the dot form sums each row over one 16-lane DPP row");
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const float sum = hk::row16_sum(acc[n]);
+    if (r < R && j == 0 && b0 + n < batch) emit(out, b0 + n, s, R, r, sum);
+  }
+}
+
 // ---- bcast form ------------------------------------------------------------------------------
 // grid: (ceil(R / 512), nsplit, batch). kAligned: matrix rows start 16-byte aligned (ld, sM
 // multiples of 8), else kAnywhere; the workgroup whose 512 outputs cross R loads element by element.
@@ -286,14 +349,30 @@ hipError_t bgemv_run(bool dot_form, int R, int K, hk_bf16 alpha, hk_bf16 beta,
     out.part = static_cast<float*>(ws);
     out.nsplit = nsplit;
   }
-  const dim3 grid(static_cast<unsigned>(strips), static_cast<unsigned>(nsplit),
-                  static_cast<unsigned>(batch));
+  dim3 grid(static_cast<unsigned>(strips), static_cast<unsigned>(nsplit),
+            static_cast<unsigned>(batch));
   if (dot_form) {
     const bool vec = ld % 8 == 0 && sm % 8 == 0 && sx % 8 == 0 && hk::aligned16(mtx) &&
                      hk::aligned16(x);
-    auto* k = incx != 1 ? gemv_dot<kElements> : vec ? gemv_dot<kAligned> : gemv_dot<kAnywhere>;
-    hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, stream, R,
-                       K, kchunk, mtx, ld, sm, x, incx, sx, out);
+    const int rows = incx != 1 ? kElements : vec ? kAligned : kAnywhere;
+    if (sm == 0 && batch > 1) {
+      // batches of one matrix (the logits of several sequences): 2 or 4 vectors per pass over it.
+      // Measured on MI355X, 50257 x 768: two vectors 23.6 -> 15.8 us, three 33.5 -> 21.3 (as four,
+      // one of them not stored), four 44.2 -> 21.5, eight 85.4 -> 38.1 (two passes).
+      const bool two = batch == 2;
+      grid.z = static_cast<unsigned>(hk::ceil_div(batch, two ? 2 : 4));
+      auto* k = rows == kElements  ? (two ? gemv_dot_shared<kElements, 2> : gemv_dot_shared<kElements, 4>)
+                : rows == kAligned ? (two ? gemv_dot_shared<kAligned, 2> : gemv_dot_shared<kAligned, 4>)
+                                   : (two ? gemv_dot_shared<kAnywhere, 2> : gemv_dot_shared<kAnywhere, 4>);
+      hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, stream, R, K, kchunk, batch, mtx, ld, x, incx,
+                         sx, out);
+    } else {
+      auto* k = rows == kElements  ? gemv_dot<kElements>
+                : rows == kAligned ? gemv_dot<kAligned>
+                                   : gemv_dot<kAnywhere>;
+      hipLaunchKernelGGL(k, grid, dim3(kThreads), 0, stream, R, K, kchunk, mtx, ld, sm, x, incx, sx,
+                         out);
+    }
   } else {
     const bool vec = ld % 8 == 0 && sm % 8 == 0 && hk::aligned16(mtx);
     hipLaunchKernelGGL(vec ? gemv_bcast<kAligned> : gemv_bcast<kAnywhere>, grid, dim3(kBcastThreads), 0,
