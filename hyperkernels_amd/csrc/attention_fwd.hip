@@ -23,9 +23,9 @@
 // scale * log2 e, so the softmax uses the hardware exp2, split once); each K / V tile of 32 keys
 // is split while it is staged into LDS (K as [key][d], V transposed as [d][key]), with the next
 // tile's global loads in flight. 36 KB of LDS and <= 168 VGPRs per workgroup let 3 workgroups
-// share a CU, so the BASELINE grid (768 workgroups) runs in one round on 256 CUs. Causal
+// share a CU, so a grid of 768 workgroups (8 x 12 heads of 1024 queries) runs in one round on 256
+// CUs; where the grid leaves a CU one workgroup at most, eight waves share its keys (KG). Causal
 // workgroups stop at the diagonal; their order is described at snake_item.
-#include <initializer_list>
 #include <mutex>
 
 #include "hk_device.h"
@@ -63,7 +63,10 @@ constexpr size_t kLdsBytes = 2 * kStageBytes;             // 36864, two stages
 // row segments and read back as the lane's 16 factors.
 constexpr int kMaskPitch = 144;
 constexpr int kMaskWaveBytes = 32 * kMaskPitch;           // 4608
-constexpr size_t kLdsBytesDrop = kLdsBytes + 4 * kMaskWaveBytes;  // 55296
+// KG key groups per workgroup (256 threads each) have their own stages and mask areas.
+constexpr size_t lds_bytes(bool drop, int kg) {
+  return kg * (kLdsBytes + (drop ? 4 * kMaskWaveBytes : 0));
+}
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
@@ -130,9 +133,11 @@ struct KVLoader {
   int64_t ks, vs;    // row strides (elements)
   int64_t T;
 
+  __device__ static int thread() { return threadIdx.x & 255; }  // within the key group
+
   __device__ KVLoader(const float* k, const float* v, int64_t ks_, int64_t vs_, int64_t T_)
       : ks(ks_), vs(vs_), T(T_) {
-    const int pr = threadIdx.x >> 4, col = (threadIdx.x & 15) * 4;
+    const int pr = thread() >> 4, col = (thread() & 15) * 4;
     k0p = k + 2 * pr * ks + col;
     v0p = v + 2 * pr * vs + col;
   }
@@ -149,7 +154,7 @@ struct KVLoader {
       }
       return;
     }
-    const int pr = threadIdx.x >> 4;
+    const int pr = thread() >> 4;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t row = k0 + 2 * pr + j;
@@ -160,7 +165,7 @@ struct KVLoader {
     }
   }
   __device__ static void store(char* st, const f32x4_t (&rk)[2], const f32x4_t (&rv)[2]) {
-    const int pr = threadIdx.x >> 4, d0 = (threadIdx.x & 15) * 4;
+    const int pr = thread() >> 4, d0 = (thread() & 15) * 4;
     char* kh = st;
     char* kl = st + kKBytes;
 #pragma unroll
@@ -212,8 +217,11 @@ __device__ __forceinline__ int snake_item(int L, int n, int P) {
 // dropout_mask[(bh*T + q)*T + key] before it enters the row sum, so O is normalised by the
 // post-dropout sum and a row with nothing kept gets O = 0 and LSE = -inf. mvec: mask rows are
 // 16-byte aligned (T % 4 == 0, aligned base), so four keys load at once.
-template <bool DROP>
-__global__ __launch_bounds__(256, DROP ? 2 : 3) void attn_fwd_kernel(hk_attn_fwd_params p,
+// KG == 2: two groups of four waves take alternate key tiles of the same 128 queries, and the second
+// group's max, sum and O^T are folded into the first's through LDS at the end. A grid that gives a
+// CU at most one workgroup is bound by one workgroup's chain of key tiles, which this halves.
+template <bool DROP, int KG>
+__global__ __launch_bounds__(256 * KG, KG > 1 ? 1 : DROP ? 2 : 3) void attn_fwd_kernel(hk_attn_fwd_params p,
                                                                      int nbh, int ncu, int mvec) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
@@ -226,10 +234,12 @@ __global__ __launch_bounds__(256, DROP ? 2 : 3) void attn_fwd_kernel(hk_attn_fwd
   const float* Qb = p.Q + b * p.q_strideB + h * p.q_strideH;
   float* Ob = p.O + b * p.o_strideB + h * p.o_strideH;
 
-  const int wave = threadIdx.x >> 6;
+  const int kg = KG > 1 ? threadIdx.x >> 8 : 0;
+  const int wave = (threadIdx.x >> 6) & 3;
   const int lane = threadIdx.x & 63;
   const int c = lane & 31;
   const int hh = lane >> 5;
+  char* const stages = lds + kg * kLdsBytes;
   const int64_t q0w = static_cast<int64_t>(qt) * kBQ + wave * 32;
   const int64_t q = q0w + c;
 
@@ -329,7 +339,7 @@ __global__ __launch_bounds__(256, DROP ? 2 : 3) void attn_fwd_kernel(hk_attn_fwd
   // reads of one tile precede the writes of the next.
   auto mask_to_lanes = [&](float4 (&mk)[4]) {
     if (!mvec) return;
-    char* reg = lds + kLdsBytes + wave * kMaskWaveBytes;
+    char* reg = lds + KG * kLdsBytes + (4 * kg + wave) * kMaskWaveBytes;
 #pragma unroll
     for (int g = 0; g < 4; ++g)
       *reinterpret_cast<float4*>(reg + (8 * g + (lane >> 3)) * kMaskPitch + 16 * (lane & 7)) =
@@ -429,35 +439,57 @@ __global__ __launch_bounds__(256, DROP ? 2 : 3) void attn_fwd_kernel(hk_attn_fwd
   };
 
   // Two LDS stages: step kt forms and finishes tile kt from one stage while the global loads
-  // of tile kt + 1 are in flight; they land in the other stage at the end of the step.
-  if (nkv > 0) {
-    ld.load(0, rk, rv);
-    KVLoader::store(lds, rk, rv);
+  // of the group's next tile are in flight; they land in the other stage at the end of the step.
+  // A group without a tile in the last step only joins its barrier.
+  if (kg < nkv) {
+    ld.load(kg * kBKV, rk, rv);
+    KVLoader::store(stages, rk, rv);
   }
   __syncthreads();
-  // dropout: the mask factors of tile kt + 1 are loaded while tile
+  // dropout: the mask factors of the next tile are loaded while tile
   // kt is computed
   float4 mk_next[4];
-  if (DROP && nkv > 0 && active(0)) load_mask(0, mk_next);
-  for (int kt = 0; kt < nkv; ++kt) {
-    const int cur = kt & 1;
-    const bool more = kt + 1 < nkv;
-    if (more) ld.load(static_cast<int64_t>(kt + 1) * kBKV, rk, rv);
+  if (DROP && kg < nkv && active(kg)) load_mask(kg, mk_next);
+  for (int base = 0, cur = 0; base < nkv; base += KG, cur ^= 1) {
+    const int kt = base + kg;
+    const bool more = kt + KG < nkv;
+    if (more) ld.load(static_cast<int64_t>(kt + KG) * kBKV, rk, rv);
+    const bool work = (KG == 1 || kt < nkv) && active(kt);
     float4 mk[4];
     if (DROP) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) mk[g] = mk_next[g];
-      if (more && active(kt + 1)) load_mask(kt + 1, mk_next);
-      if (active(kt)) mask_to_lanes(mk);
+      if (more && active(kt + KG)) load_mask(kt + KG, mk_next);
+      if (work) mask_to_lanes(mk);
     }
-    const char* st = lds + cur * kStageBytes;
-    if (active(kt)) {
+    const char* st = stages + cur * kStageBytes;
+    if (work) {
       const float c0 = base_of(m);
       f32x16_t sc = qk(st, c0);
       softmax_pv(kt, sc, c0, st, mk);
     }
-    if (more) KVLoader::store(lds + (cur ^ 1) * kStageBytes, rk, rv);
+    if (more) KVLoader::store(stages + (cur ^ 1) * kStageBytes, rk, rv);
     __syncthreads();
+  }
+  if (KG > 1) {
+    // the stages are free now: element i of thread t at [i][t]
+    float* ex = reinterpret_cast<float*>(lds) + KVLoader::thread();
+    if (kg == 1) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) ex[256 * i] = o[i >> 4][i & 15];
+      ex[256 * 32] = m;
+      ex[256 * 33] = l;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = ex[256 * 32], l1 = ex[256 * 33];
+    const float mm = fmaxf(m, m1);
+    const float a0 = m == -INFINITY ? 0.f : fast_exp2(m - mm);
+    const float a1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mm);
+    l = l * a0 + l1 * a1;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) o[i >> 4][i & 15] = o[i >> 4][i & 15] * a0 + ex[256 * i] * a1;
+    m = mm;
   }
 
   const float lt = hk::half32_reduce(l, hk::AddOp{});
@@ -516,6 +548,22 @@ __global__ __launch_bounds__(256) void attn_precompute_d_scalar(hk_attn_bwd_para
   if (row < p.T && sub == 0) p.D[b * p.d_strideB + h * p.d_strideH + row] = s;
 }
 
+template <bool DROP, int KG>
+hipError_t launch_fwd(const hk_attn_fwd_params& p, int grid, int nbh, int mvec,
+                      hipStream_t stream) {
+  constexpr size_t kLds = lds_bytes(DROP, KG);
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [] {
+    attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_kernel<DROP, KG>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLds));
+  });
+  HK_RETURN_IF_ERROR(attr);
+  hipLaunchKernelGGL((attn_fwd_kernel<DROP, KG>), dim3(static_cast<unsigned>(grid)),
+                     dim3(256 * KG), kLds, stream, p, nbh, hk::device_cu_count(), mvec);
+  return hk::launch_status();
+}
+
 bool rows_aligned(const void* base, int64_t strideB, int64_t strideH, int64_t strideM) {
   return hk::aligned16(base) && strideB % 4 == 0 && strideH % 4 == 0 && strideM % 4 == 0;
 }
@@ -540,23 +588,14 @@ extern "C" hipError_t hk_fused_attn_forward(const hk_attn_fwd_params* params, in
   const int64_t bh = static_cast<int64_t>(p.B) * p.nh;
   const int64_t nqt = (p.T + kBQ - 1) / kBQ;
   HK_CHECK_ARG(bh * nqt <= INT32_MAX);
-  static std::once_flag once;
-  static hipError_t attr = hipSuccess;
-  std::call_once(once, [] {
-    for (int d = 0; d < 2; ++d) {
-      const void* k = d ? reinterpret_cast<const void*>(&attn_fwd_kernel<true>)
-                        : reinterpret_cast<const void*>(&attn_fwd_kernel<false>);
-      const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               static_cast<int>(d ? kLdsBytesDrop : kLdsBytes));
-      if (e != hipSuccess) attr = e;
-    }
-  });
-  HK_RETURN_IF_ERROR(attr);
-  hipLaunchKernelGGL(drop ? attn_fwd_kernel<true> : attn_fwd_kernel<false>,
-                     dim3(static_cast<unsigned>(nqt * bh)), dim3(256),
-                     drop ? kLdsBytesDrop : kLdsBytes, stream, p,
-                     static_cast<int>(bh), hk::device_cu_count(), mvec);
-  return hk::launch_status();
+  // Two key groups while no CU gets a second workgroup: measured on MI355X, causal T 1024: 96
+  // workgroups 40.8 -> 31.5 us, 192 workgroups 40.6 -> 32.4; T 2048, 256 workgroups 74.9 -> 56.0;
+  // not causal T 333, 72 workgroups 18.0 -> 16.2. Beyond that the second workgroup fills the CU
+  // already: T 1300, 264 workgroups 64.8 with one group, 74.8 with two.
+  const bool groups = nqt * bh <= hk::device_cu_count();
+  auto* run = drop ? (groups ? launch_fwd<true, 2> : launch_fwd<true, 1>)
+                   : (groups ? launch_fwd<false, 2> : launch_fwd<false, 1>);
+  return run(p, static_cast<int>(nqt * bh), static_cast<int>(bh), mvec, stream);
 }
 
 extern "C" hipError_t hk_attn_bwd_precompute_D(const hk_attn_bwd_params* params, int head_dim,
