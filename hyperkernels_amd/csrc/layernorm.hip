@@ -18,7 +18,7 @@
 // gamma/beta gradient is accumulated per lane in registers across the rows a wave visits,
 // reduced across the workgroup's waves in LDS, written as one partial per workgroup, and summed over
 // the workgroups in a fixed order by a second small kernel: the result is deterministic, unlike
-// the reference's atomics. Rows of 2049 to 4096 columns are shared by two waves there; few rows
+// the reference's atomics. Rows of 2049 to 4096 columns are shared by four waves there; few rows
 // take one launch for both gradients (ln_bwd_few_rows). Longer rows use a workgroup-per-row
 // fallback and a column-slab reduction.
 #include <initializer_list>
