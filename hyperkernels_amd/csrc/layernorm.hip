@@ -690,6 +690,14 @@ hipError_t lds_limit(size_t bytes) {
   return status;
 }
 
+// Whether two arrays of n elements share memory.
+template <typename S>
+bool overlap(const S* a, const S* b, int64_t n) {
+  const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+  const uintptr_t bytes = static_cast<uintptr_t>(n) * sizeof(S);
+  return pa < pb + bytes && pb < pa + bytes;
+}
+
 // Workgroups of a gamma/beta backward: one per `waves` rows, at most 8 / waves per CU.
 int bwd_gb_grid(int rows, int waves) {
   const int64_t want = hk::ceil_div(rows, waves);
@@ -838,10 +846,16 @@ hipError_t launch_bwd(const St<T>* dy, const St<T>* x, const float* mean, const 
   HK_CHECK_ARG(dy && x && mean && rstd);
   HK_CHECK_ARG(!write_dx || dx);
   const bool vec = vec_rows<T>(cols, {dy, x, gamma, dx});
+  // grad_x may be dy or x itself. The register forms load a row before they store it, and the
+  // workgroup-per-row form reads and writes an element in the same lane; ln_bwd_few_rows reads whole
+  // columns while other workgroups store rows, and the slabs read after a grad_x launch of their own
+  // would, so the first is left out for such calls and the second run before it.
+  const int64_t n = static_cast<int64_t>(rows) * cols;
+  const bool in_place = write_dx && (overlap(dx, dy, n) || overlap(dx, x, n));
   if (!do_gb) return launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream);
   const int vpl = row_vpl<T>(cols);
   const float inv_cols = 1.0f / static_cast<float>(cols);
-  if (rows <= kFewRows && vpl > 0 && vpl <= kMaxFewVpl<T>) {
+  if (rows <= kFewRows && vpl > 0 && vpl <= kMaxFewVpl<T> && !in_place) {
     const int row_groups =
         write_dx ? static_cast<int>(hk::ceil_div(rows, kFinCols * kFinGroups / HK_WAVE)) : 0;
     const unsigned grid = static_cast<unsigned>(row_groups + hk::ceil_div(cols, kFinCols));
@@ -874,8 +888,6 @@ hipError_t launch_bwd(const St<T>* dy, const St<T>* x, const float* mean, const 
     HK_RETURN_IF_ERROR(hk::launch_status());
     return launch_finalize<T>(part, f.grid, cols, dgamma, dbeta, stream);
   }
-  if (write_dx)
-    HK_RETURN_IF_ERROR(launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream));
   // slabs of at least 16 rows, at most four workgroups per CU
   const int64_t blocks = hk::ceil_div(cols, kThreads);
   int64_t nslab = capturing ? 1 : hk::ceil_div(4 * static_cast<int64_t>(hk::device_cu_count()), blocks);
@@ -895,7 +907,9 @@ hipError_t launch_bwd(const St<T>* dy, const St<T>* x, const float* mean, const 
                      slab);
   HK_RETURN_IF_ERROR(hk::launch_status());
   if (nslab > 1)
-    return launch_finalize<T>(part, static_cast<int>(nslab), cols, dgamma, dbeta, stream);
+    HK_RETURN_IF_ERROR(
+        launch_finalize<T>(part, static_cast<int>(nslab), cols, dgamma, dbeta, stream));
+  if (write_dx) return launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream);
   return hipSuccess;
 }
 

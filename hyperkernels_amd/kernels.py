@@ -141,7 +141,7 @@ def ln_backward_gamma_beta(grad_y, x, mean, rstd, grad_gamma, grad_beta):
 
 
 def layer_norm_backward(grad_y, x, mean, rstd, gamma, grad_gamma, grad_beta, grad_x=None):
-    """Fused backward: grad_x written, grad_gamma / grad_beta added into, one pass over dy, x."""
+    """Fused backward: grad_x written (grad_y or x itself, too), grad_gamma / grad_beta added into."""
     _dev(grad_y, x, mean, rstd, gamma, grad_gamma, grad_beta, grad_x)
     rows, cols = _rows_cols(x)
     grad_x = torch.empty_like(x) if grad_x is None else grad_x

@@ -82,8 +82,9 @@ HK_API hipError_t hk_gelu_backward_f16(const hk_f16* grad, const hk_f16* in, hk_
  *   (kernels/layernorm/ln_backward_gamma_beta_sm89_kernel.cu:15-21). As in the reference the
  *   result is ADDED to grad_gamma / grad_beta (the reference adds with atomics into
  *   caller-zeroed buffers); here the sum is formed in a fixed order, so it is deterministic.
- * The fused backward computes grad_x and adds into grad_gamma / grad_beta in one pass over
- *   dy and x (no counterpart in the reference, which reads dy and x twice).
+ * The fused backward computes grad_x and adds into grad_gamma / grad_beta in one call (no
+ *   counterpart in the reference, which takes two). Up to 4096 columns that is one pass over dy and
+ *   x; few rows and longer ones read them a second time. grad_x may be grad_y or x itself.
  * ---------------------------------------------------------------------------------------- */
 HK_API hipError_t hk_layer_norm_forward_f32(const float* x, const float* gamma, const float* beta,
                                      float* y, float* mean_out, float* rstd_out, int rows,

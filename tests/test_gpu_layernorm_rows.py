@@ -114,3 +114,49 @@ def test_layernorm_backward_under_capture(hk, orc, rows, cols):
         _, bm, br = hk.layer_norm_forward(big)
         hk.layer_norm_backward(big, big, bm, br, None, torch.zeros(4096, device=DEV),
                                torch.zeros(4096, device=DEV))
+
+
+# Both sides of the one-launch limit (512 rows) in every form of a row: whole vectors of one wave,
+# overlapping vectors, four waves, a workgroup per row, less than a vector
+@pytest.mark.parametrize("rows,cols", [(64, 768), (512, 768), (513, 768), (512, 333), (600, 333),
+                                       (512, 2560), (600, 2560), (512, 8200), (600, 8200), (512, 3)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("into", ["dy", "x"])
+@pytest.mark.parametrize("captured", [False, True])
+def test_layernorm_backward_in_place(hk, rows, cols, dtype, into, captured):
+    # grad_x written over dy or x: the same grad_x and the same sums (in another order, 1e-5) as in a
+    # buffer of its own
+    say("layernorm in place", rows, cols, dtype, into, captured)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(rows + cols)
+    x, dy = (torch.randn(rows, cols, generator=g, device=DEV).to(dtype) for _ in range(2))
+    gamma = torch.rand(cols, generator=g, device=DEV).to(dtype)
+    _, m, r = hk.layer_norm_forward(x)
+    want = torch.zeros(2, cols, device=DEV)
+    want_dx = hk.layer_norm_backward(dy, x, m, r, gamma, want[0], want[1])
+    bufs = {"x": x.clone(), "dy": dy.clone()}
+    sums = torch.zeros(2, cols, device=DEV)
+
+    def call():
+        hk.layer_norm_backward(bufs["dy"], bufs["x"], m, r, gamma, sums[0], sums[1],
+                               grad_x=bufs[into])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()  # also gives the stream's workspace its size before a capture
+    torch.cuda.synchronize()
+    run = call
+    if captured:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            call()
+        run = graph.replay
+    for _ in range(3):
+        bufs["x"].copy_(x)
+        bufs["dy"].copy_(dy)
+        sums.zero_()
+        run()
+        torch.cuda.synchronize()
+        assert max_rel(host(bufs[into].float()), host(want_dx.float())) <= (
+            1e-6 if dtype == torch.float32 else 2.0 ** -8)
+        assert max_rel(host(sums), host(want)) <= 1e-5
