@@ -122,8 +122,8 @@ __global__ __launch_bounds__(kThreads) void reduce_inner_wave(const float* __res
 // alignment), eight rows in flight, and are summed through LDS in wave order. Measured on MI355X,
 // 4096 x 4096 fp32 from cache with its finalize: 31.2 us with a 4-byte load per lane and row (and the
 // finalize below as it was), 16.0 us so; 100000 x 300: 145 -> 48 us.
-// The last group of a row that is no multiple of four long reads its last four columns again: two
-// lanes then store the same sums.
+// The last group of a single run that is no multiple of four long reads its last four columns again:
+// two lanes then store the same sums.
 constexpr int kOuterCols = 4;
 typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -317,12 +317,13 @@ hipError_t reduce_outer_launch(const float* src, float* dst, int64_t nout, int64
   float* out = dst;
   if (split > 1)
     HK_RETURN_IF_ERROR(ps.get(static_cast<size_t>(split * nout) * sizeof(float), stream, &out));
-  // four adjacent outputs read four adjacent columns: every group of four lies in one run of
-  // `inner` columns. Rows of more than an eighth of the CUs' worth of workgroups (8192 columns)
-  // keep the 4-byte loads: they stream from HBM better (8192 x 28000: 159.8 us against 168.8,
-  // 512 x 100001: 43.0 against 45.7; 8192 x 6001: 52.4 against 48.5).
-  const bool wide = nout >= kOuterCols && (inner >= nout || inner % kOuterCols == 0) &&
-                    8 * gx <= hk::device_cu_count();
+  // Four adjacent outputs read four adjacent columns where every group of four lies in one run of
+  // `inner` columns: one run, or runs of a multiple of four and no part of a group in the last one
+  // (num_outputs may end inside a run). Rows of more than an eighth of the CUs' worth of workgroups
+  // (8192 columns) keep the 4-byte loads: they stream from HBM better (8192 x 28000: 159.8 us
+  // against 168.8, 512 x 100001: 43.0 against 45.7; 8192 x 6001: 52.4 against 48.5).
+  const bool groups = inner >= nout || (inner % kOuterCols == 0 && nout % kOuterCols == 0);
+  const bool wide = nout >= kOuterCols && groups && 8 * gx <= hk::device_cu_count();
   hipLaunchKernelGGL(wide ? reduce_outer_wide : reduce_outer,
                      dim3(static_cast<unsigned>(gx), static_cast<unsigned>(split)), dim3(kThreads), 0,
                      stream, src, out, nout, inner, outer_stride, row_stride, len, slice_len);

@@ -29,3 +29,15 @@ def test_outer_sums_are_exact(hk, runs, inner, pad, off, length):
     want = x.astype(np.float64).sum(1).reshape(-1)
     got = hk.unified_reduce_sum(src[off:], layout).cpu().numpy()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("nout,inner", [(10, 8), (21, 8), (262, 256), (7, 4), (12, 8), (9, 16)])
+def test_outputs_end_inside_a_run(hk, nout, inner):
+    # num_outputs is no whole number of runs: the last outputs are the first columns of the last run
+    length, runs = 37, -(-nout // inner)
+    print("[case] reduce outer part run", nout, inner, flush=True)
+    x = np.random.default_rng(nout).integers(-9, 10, (runs, length, inner)).astype(np.float32)
+    layout = hk.ReductionLayout(hk.REDUCE_OUTER, nout, length, length * inner, inner, inner)
+    want = x.astype(np.float64).sum(1).reshape(-1)[:nout]
+    got = hk.unified_reduce_sum(torch.from_numpy(x).cuda(), layout).cpu().numpy()
+    assert np.array_equal(got, want)
