@@ -27,7 +27,9 @@ int device_cu_count();
 // process ends. Work on one stream runs in order, so consecutive calls on that stream reuse
 // the buffer safely; calls on different streams get different buffers. The pointer is valid
 // until the next call on the same (device, stream) asks for more bytes, so a launcher fetches
-// it once per call; growing it first waits for the work queued on that stream.
+// it once per call; growing it first waits for the work queued on that stream. A buffer handed out
+// while the stream was being captured stays allocated when the workspace grows, so a graph's replays
+// keep the memory that they were captured with.
 hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out);
 
 // Whether the stream is being captured into a graph.

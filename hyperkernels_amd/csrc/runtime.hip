@@ -19,12 +19,14 @@ struct DeviceState {
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
+  bool captured = false;  // handed out during a stream capture: a graph may hold the address
 };
 std::mutex g_mu;
 std::vector<DeviceState> g_devices;
 // One grow-only workspace per (device, stream): work on one stream is ordered, so a call may
 // reuse the buffer the previous call on that stream used; calls on different streams never
-// share one.
+// share one. A buffer that a graph may hold is never freed: the buffer that takes its place is at
+// least twice as large, so those kept add up to less than the one in use.
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 
 DeviceState* state_for_current(hipError_t* err) {
@@ -68,17 +70,24 @@ hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out) {
   HK_RETURN_IF_ERROR(hipGetDevice(&dev));
   Workspace& w = g_ws[std::make_pair(dev, stream)];
   if (bytes > w.bytes) {
-    if (w.ptr) {
-      // Work already queued on this stream may still read the old buffer.
-      HK_RETURN_IF_ERROR(hipStreamSynchronize(stream));
-      HK_RETURN_IF_ERROR(hipFree(w.ptr));
-      w.ptr = nullptr;
-      w.bytes = 0;
-    }
     size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
-    HK_RETURN_IF_ERROR(hipMalloc(&w.ptr, want));
-    w.bytes = want;
+    if (w.captured) {
+      void* ptr = nullptr;
+      if (want < 2 * w.bytes) want = 2 * w.bytes;
+      HK_RETURN_IF_ERROR(hipMalloc(&ptr, want));
+      w = Workspace{ptr, want, false};
+    } else {
+      if (w.ptr) {
+        // Work already queued on this stream may still read the old buffer.
+        HK_RETURN_IF_ERROR(hipStreamSynchronize(stream));
+        HK_RETURN_IF_ERROR(hipFree(w.ptr));
+        w = Workspace{};
+      }
+      HK_RETURN_IF_ERROR(hipMalloc(&w.ptr, want));
+      w.bytes = want;
+    }
   }
+  if (!w.captured && stream_capturing(stream)) w.captured = true;
   *out = w.ptr;
   return hipSuccess;
 }
