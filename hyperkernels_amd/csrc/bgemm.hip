@@ -834,7 +834,7 @@ hipError_t run_regions(bool ta, bool tb, int grid_z, hipStream_t stream, int M, 
                                static_cast<int>(nfull));
 }
 
-// Split-K chosen by the library when the caller gives none: the split with the least modelled
+// Split-K chosen by the library when the caller gives none, at most `most`: the split with the least modelled
 // time (us), summed over the rounds of 256 x 256 work items on the CUs:
 //   - a round costs (k-tiles per split) x t(busy) plus a fixed prologue / epilogue (8 us with
 //     bf16 C, 12 us with a 256 KiB fp32 partial per tile);
@@ -845,7 +845,7 @@ hipError_t run_regions(bool ta, bool tb, int grid_z, hipStream_t stream, int M, 
 // Calibrated on the 8192 x 1280 x 5120 and 1280 x 5120 x 8192 products (160 and 100 tiles):
 // measured 123 / 149 / 131 us at 1 / 2 / 3 splits for the first, 120 / 115 / 151 / 137 / 135
 // us at 1 to 5 for the second; the model picks 1 and 2.
-int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs, double* best_cost) {
+int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs, int most, double* best_cost) {
   const int64_t cus = hk::device_cu_count();
   auto t_kt = [&](int64_t busy) {
     const double f = static_cast<double>(busy) / static_cast<double>(cus);
@@ -854,7 +854,7 @@ int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs, double* be
   };
   double best = 0.0;
   int best_s = 1;
-  for (int s = 1; s <= 8; ++s) {
+  for (int s = 1; s <= most; ++s) {
     if (s > 1 && ktiles / s < 4) break;
     const int64_t items = work_tiles * s, kps = hk::ceil_div(ktiles, static_cast<int64_t>(s));
     const double fixed = s > 1 ? 12.0 : 8.0;
@@ -873,6 +873,9 @@ int auto_split_k(int64_t work_tiles, int64_t ktiles, int64_t outputs, double* be
   return best_s;
 }
 
+constexpr int kMostSplits = 8;      // of the library's own choice on the 256-wide tiles
+constexpr int kMaxGridZ = 65535;  // batches x k splits of one launch
+
 // What the rows of a product's matrices are, as the kernels see them.
 enum class Rows {
   kAligned,  // whole 16-byte vectors: 8-element multiples for every contiguous extent, leading
@@ -880,22 +883,25 @@ enum class Rows {
   kRaggedC,  // A and B like that, C at any 2-byte address and any N
   kRagged,   // any 2-byte address, any extent
   kNone      // no MFMA path: no k, a leading dimension whose per-lane 32-bit byte offsets do not
-             // fit, or one under 8 (a vector could leave the matrix)
+             // fit, or one under 8 (a vector could leave the matrix); more batches of unaligned
+             // rows than the tiles' grid takes
 };
 Rows row_kind(bool ta, bool tb, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
-              int64_t sA, int64_t sB, int64_t sC, bool a16, bool b16, bool c16) {
+              int64_t sA, int64_t sB, int64_t sC, int batch, bool a16, bool b16, bool c16) {
   if (K <= 0 || lda >= (1 << 22) || ldb >= (1 << 22)) return Rows::kNone;
   const int contig_a = ta ? M : K, contig_b = tb ? K : N;
   const bool ab = contig_a % 8 == 0 && contig_b % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
                   sA % 8 == 0 && sB % 8 == 0 && a16 && b16;
-  if (!ab) return lda >= 8 && ldb >= 8 ? Rows::kRagged : Rows::kNone;
-  return N % 8 == 0 && ldc % 8 == 0 && sC % 8 == 0 && c16 ? Rows::kAligned : Rows::kRaggedC;
+  if (ab && N % 8 == 0 && ldc % 8 == 0 && sC % 8 == 0 && c16) return Rows::kAligned;
+  if (batch > kMaxGridZ) return Rows::kNone;
+  if (ab) return Rows::kRaggedC;
+  return lda >= 8 && ldb >= 8 ? Rows::kRagged : Rows::kNone;
 }
 // The same for contiguous, 16-byte aligned operands (the planning queries).
-Rows packed_rows(bool ta, bool tb, int M, int N, int K) {
+Rows packed_rows(bool ta, bool tb, int M, int N, int K, int batch) {
   const int64_t lda = ta ? M : K, ldb = tb ? K : N;
   return row_kind(ta, tb, M, N, K, lda, ldb, N, lda * (ta ? K : M), ldb * (tb ? N : K),
-                  static_cast<int64_t>(M) * N, true, true, true);
+                  static_cast<int64_t>(M) * N, batch, true, true, true);
 }
 
 using Plan = hk::GemmPlan;
@@ -925,6 +931,19 @@ Plan make_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_k, Ro
   const hk::FlexPlan f = hk::bgemm_flex_plan(M, N, K, batch, split_k, ragged);
   if (!ragged && f.cost > 0.95 * cost) return wide;
   return Plan{f.tile, f.used, f.kps};
+}
+
+// The better of the two families with one k split, which needs no workspace.
+Plan whole_plan(bool ta, bool tb, int M, int N, int K, int batch, Rows rows) {
+  const bool ragged = rows == Rows::kRagged;
+  const hk::FlexPlan f = hk::bgemm_flex_plan(M, N, K, batch, 1, ragged);
+  if (!ragged) {
+    const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    double cost = 0.0;
+    auto_split_k(tiles * batch, hk::ceil_div(K, BK), static_cast<int64_t>(M) * N * batch, 1, &cost);
+    if (f.cost > 0.95 * wide_cost(ta, tb, M, N, K, batch, 1, cost)) return Plan{0, 1, K};
+  }
+  return Plan{f.tile, 1, K};
 }
 
 // bias == NULL: C = alpha * op(A) op(B) + beta * C. Otherwise C = alpha * op(A) op(B) +
@@ -962,7 +981,7 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
   }
 
   const Rows rows = row_kind(ta, tb, M, N, K, lda, ldb, ldc, strideA, strideB, strideC,
-                             hk::aligned16(A), hk::aligned16(B), hk::aligned16(C));
+                             batchCount, hk::aligned16(A), hk::aligned16(B), hk::aligned16(C));
   if (rows == Rows::kNone) {
     dim3 grid((N + 15) / 16, (M + 15) / 16, batchCount);
     hipLaunchKernelGGL(bgemm_simple, grid, dim3(256), 0, stream, ta ? 1 : 0, tb ? 1 : 0, M, N,
@@ -980,16 +999,26 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
         hk::bgemm_flex_plan(M, N, K, batchCount, 1, rows == Rows::kRagged);
     plan = Plan{f.tile, 1, K};
   }
+  // Unaligned rows and the small tiles can do without splits: a split that the grid or the memory
+  // does not take is left out.
+  const bool optional = plan.flex || ep.ragged;
+  if (optional && static_cast<int64_t>(batchCount) * plan.used > kMaxGridZ)
+    plan = whole_plan(ta, tb, M, N, K, batchCount, rows);
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batchCount) * plan.used <= 65535);
-  float* part = nullptr;
+  HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batchCount) * plan.used <= kMaxGridZ);
+  void* ws = nullptr;
   if (plan.used > 1) {
-    void* ws = nullptr;
     const size_t part_bytes =
         static_cast<size_t>(plan.used) * batchCount * M * part_pitch(N) * sizeof(float);
-    HK_RETURN_IF_ERROR(hk::device_workspace(part_bytes, stream, &ws));
-    part = static_cast<float*>(ws);
+    const hipError_t e = hk::device_workspace(part_bytes, stream, &ws);
+    if (e == hipErrorOutOfMemory && optional) {
+      (void)hipGetLastError();
+      plan = whole_plan(ta, tb, M, N, K, batchCount, rows);
+    } else {
+      HK_RETURN_IF_ERROR(e);
+    }
   }
+  float* part = static_cast<float*>(ws);
   if (plan.flex) {
     HK_RETURN_IF_ERROR(hk::bgemm_flex_run(
         plan.flex, hk::FlexCall{ta, tb, M, N, K, batchCount, A, lda, strideA, B, ldb, strideB, C,
@@ -1017,7 +1046,7 @@ void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, in
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   const int s = split_k > 0 ? split_k
                             : auto_split_k(tiles * batch, hk::ceil_div(K, BK),
-                                           static_cast<int64_t>(M) * N * batch, cost);
+                                           static_cast<int64_t>(M) * N * batch, kMostSplits, cost);
   *kps = static_cast<int>(hk::ceil_div(hk::ceil_div(K, s), BK) * BK);
   *used = static_cast<int>(hk::ceil_div(K, *kps));
 }
@@ -1058,7 +1087,7 @@ static int query_kind(int transA, int transB, int M, int N, int K, int batchCoun
     return -1;
   if (M == 0 || N == 0 || batchCount == 0) return 0;
   if (splitK == 0 && (M == 1 || N == 1)) return 1;
-  return packed_rows(transA != 0, transB != 0, M, N, K) == Rows::kNone ? 1 : 2;
+  return packed_rows(transA != 0, transB != 0, M, N, K, batchCount) == Rows::kNone ? 1 : 2;
 }
 
 extern "C" int hk_bgemm_split_count(int transA, int transB, int M, int N, int K, int batchCount,
@@ -1066,7 +1095,7 @@ extern "C" int hk_bgemm_split_count(int transA, int transB, int M, int N, int K,
   const int kind = query_kind(transA, transB, M, N, K, batchCount, splitK);
   if (kind < 2) return kind;
   const bool ta = transA != 0, tb = transB != 0;
-  return make_plan(ta, tb, M, N, K, batchCount, splitK, packed_rows(ta, tb, M, N, K)).used;
+  return make_plan(ta, tb, M, N, K, batchCount, splitK, packed_rows(ta, tb, M, N, K, batchCount)).used;
 }
 
 extern "C" int hk_bgemm_small_tile(int transA, int transB, int M, int N, int K, int batchCount,
@@ -1075,7 +1104,7 @@ extern "C" int hk_bgemm_small_tile(int transA, int transB, int M, int N, int K, 
   if (kind < 2) return kind < 0 ? -1 : 0;
   const bool ta = transA != 0, tb = transB != 0;
   return hk::bgemm_flex_tile_rows(
-      make_plan(ta, tb, M, N, K, batchCount, splitK, packed_rows(ta, tb, M, N, K)).flex);
+      make_plan(ta, tb, M, N, K, batchCount, splitK, packed_rows(ta, tb, M, N, K, batchCount)).flex);
 }
 
 // The 256-wide tiles' own plan for a product whose operands they take; splits: its k splits.
@@ -1084,7 +1113,7 @@ static int wide_tile(int transA, int transB, int M, int N, int K, int batchCount
   const int kind = query_kind(transA, transB, M, N, K, batchCount, splitK);
   if (kind <= 0) return kind;
   const bool ta = transA != 0, tb = transB != 0;
-  if (kind == 1 || packed_rows(ta, tb, M, N, K) == Rows::kRagged) return 0;
+  if (kind == 1 || packed_rows(ta, tb, M, N, K, batchCount) == Rows::kRagged) return 0;
   int used = 1, kps = 0;
   hk::bgemm_split_plan(M, N, K, batchCount, splitK, &used, &kps);
   if (w160_plan(ta, tb, M, N, K, batchCount * used, used)) return cols ? w160::kBN : w160::kBM;

@@ -123,6 +123,26 @@ def test_bgemm_flex_batches_and_split(hk, orc, ta, tb):
                C0, ta, tb, 1.0, 0.5)
 
 
+@pytest.mark.parametrize("batch,K,split,odd_c", [(40000, 130, 2, False), (40000, 136, 2, True),
+                                                 (65535, 65, 2, False), (65536, 72, 1, True),
+                                                 (65537, 9, 1, False)])
+def test_bgemm_flex_more_batches_than_a_grid_takes(hk, batch, K, split, odd_c):
+    # batch x splits past 65535, and batches past it, of rows that are no whole vectors (of A and B, or
+    # of C alone): a given split is left out
+    M, N = 3, 9
+    say("bgemm flex batches x splits", batch, K, split)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(K)
+    a, b = (torch.randn(batch, r, K, generator=g, device=DEV).to(torch.bfloat16) for r in (M, N))
+    c = torch.full((batch, M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    assert a.shape[2] % 8 == 0 if odd_c else a.shape[2] % 8
+    assert hk.lib().hk_bgemm_core(0, split, M, N, K, bits(1.0), a.data_ptr(), K, M * K, b.data_ptr(), K,
+                                  N * K, 0, c.data_ptr(), N, M * N, batch,
+                                  torch.cuda.current_stream().cuda_stream) == 0
+    ref = (a.float()[:, :, None] * b.float()[:, None]).sum(3)
+    assert (c.float() - ref).abs().max() <= 1e-2 * ref.abs().max()
+
+
 def test_bgemm_flex_split_plan_under_capture(hk, orc):
     # A split plan takes the stream's workspace in eager calls and runs unsplit in a captured graph,
     # whose replays stay right after a larger call has grown the workspace.
