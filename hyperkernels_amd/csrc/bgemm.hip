@@ -933,15 +933,26 @@ Plan make_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_k, Ro
   return Plan{f.tile, f.used, f.kps};
 }
 
-// The better of the two families with one k split, which needs no workspace.
-Plan whole_plan(bool ta, bool tb, int M, int N, int K, int batch, Rows rows) {
+size_t partial_bytes(int used, int M, int N, int batch) {
+  return static_cast<size_t>(used) * batch * M * part_pitch(N) * sizeof(float);
+}
+
+// The better of the two families where partials may take `held` bytes at most: the small and
+// any-alignment tiles with one k split, the 256-wide ones with their own splits or with one.
+Plan lean_plan(bool ta, bool tb, int M, int N, int K, int batch, Rows rows, size_t held) {
   const bool ragged = rows == Rows::kRagged;
   const hk::FlexPlan f = hk::bgemm_flex_plan(M, N, K, batch, 1, ragged);
   if (!ragged) {
-    const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    Plan wide{0, 1, K};
     double cost = 0.0;
-    auto_split_k(tiles * batch, hk::ceil_div(K, BK), static_cast<int64_t>(M) * N * batch, 1, &cost);
-    if (f.cost > 0.95 * wide_cost(ta, tb, M, N, K, batch, 1, cost)) return Plan{0, 1, K};
+    hk::bgemm_split_plan(M, N, K, batch, 0, &wide.used, &wide.kps, &cost);
+    if (wide.used > 1 && partial_bytes(wide.used, M, N, batch) > held) {
+      const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+      wide = Plan{0, 1, K};
+      auto_split_k(tiles * batch, hk::ceil_div(K, BK), static_cast<int64_t>(M) * N * batch, 1,
+                   &cost);
+    }
+    if (f.cost > 0.95 * wide_cost(ta, tb, M, N, K, batch, wide.used, cost)) return wide;
   }
   return Plan{f.tile, 1, K};
 }
@@ -992,28 +1003,26 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
   }
   ep.ragged = rows != Rows::kAligned;
   Plan plan = make_plan(ta, tb, M, N, K, batchCount, splitK, rows);
-  // A captured graph would keep the address of the stream's workspace, which a later call may
-  // grow: under capture the small and any-alignment tiles run unsplit and need none.
-  if (plan.flex && plan.used > 1 && hk::stream_capturing(stream)) {
-    const hk::FlexPlan f =
-        hk::bgemm_flex_plan(M, N, K, batchCount, 1, rows == Rows::kRagged);
-    plan = Plan{f.tile, 1, K};
-  }
-  // Unaligned rows and the small tiles can do without splits: a split that the grid or the memory
-  // does not take is left out.
+  // The small tiles' splits and those of unaligned rows are left out where the grid or the memory
+  // does not take them, and under capture: such calls need no workspace then, whose size the capture
+  // could not change and which replays would share with the stream's eager calls. Aligned rows may
+  // still take the 256-wide tiles' splits there, in the workspace that the stream has.
   const bool optional = plan.flex || ep.ragged;
-  if (optional && static_cast<int64_t>(batchCount) * plan.used > kMaxGridZ)
-    plan = whole_plan(ta, tb, M, N, K, batchCount, rows);
+  if (plan.used > 1 && optional) {
+    const bool capturing = hk::stream_capturing(stream);
+    if (capturing || static_cast<int64_t>(batchCount) * plan.used > kMaxGridZ)
+      plan = lean_plan(ta, tb, M, N, K, batchCount, rows,
+                       capturing && !ep.ragged ? hk::device_workspace_bytes(stream) : 0);
+  }
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batchCount) * plan.used <= kMaxGridZ);
   void* ws = nullptr;
   if (plan.used > 1) {
-    const size_t part_bytes =
-        static_cast<size_t>(plan.used) * batchCount * M * part_pitch(N) * sizeof(float);
-    const hipError_t e = hk::device_workspace(part_bytes, stream, &ws);
+    const hipError_t e =
+        hk::device_workspace(partial_bytes(plan.used, M, N, batchCount), stream, &ws);
     if (e == hipErrorOutOfMemory && optional) {
       (void)hipGetLastError();
-      plan = whole_plan(ta, tb, M, N, K, batchCount, rows);
+      plan = lean_plan(ta, tb, M, N, K, batchCount, rows, 0);
     } else {
       HK_RETURN_IF_ERROR(e);
     }

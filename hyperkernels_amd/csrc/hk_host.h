@@ -32,6 +32,9 @@ int device_cu_count();
 // keep the memory that they were captured with.
 hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out);
 
+// Bytes the stream's workspace has now: what a call can use under capture, where it cannot grow.
+size_t device_workspace_bytes(hipStream_t stream);
+
 // Whether the stream is being captured into a graph.
 bool stream_capturing(hipStream_t stream);
 

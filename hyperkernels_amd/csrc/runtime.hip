@@ -92,4 +92,12 @@ hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out) {
   return hipSuccess;
 }
 
+size_t device_workspace_bytes(hipStream_t stream) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  const auto it = g_ws.find(std::make_pair(dev, stream));
+  return it == g_ws.end() ? 0 : it->second.bytes;
+}
+
 }  // namespace hk

@@ -143,6 +143,58 @@ def test_bgemm_flex_more_batches_than_a_grid_takes(hk, batch, K, split, odd_c):
     assert (c.float() - ref).abs().max() <= 1e-2 * ref.abs().max()
 
 
+@pytest.mark.parametrize("split_k", [0, 3])
+@pytest.mark.parametrize("M,N,K", [(64, 33, 8192), (300, 299, 4001)])
+def test_bgemm_unaligned_rows_need_no_workspace_under_capture(hk, orc, M, N, K, split_k):
+    # products that split k (N odd: only the rows of C are unaligned) on a stream without a workspace
+    say("bgemm capture cold", M, N, K, split_k)
+    assert hk.lib().hk_bgemm_split_count(0, 1, M, N, K, 1, split_k) > 1
+    A, B, C0 = _operands(orc, M, N, K, 0, 1, 2550)
+    dA, dB, dC = to_dev_bf16(A), to_dev_bf16(B), to_dev_bf16(C0)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        args = (M, N, K, bits(1.0), dA.data_ptr(), K, 0, dB.data_ptr(), K, 0, 0, dC.data_ptr(), N, 0, 1,
+                torch.cuda.current_stream().cuda_stream)
+        rc = (hk.lib().hk_bgemm_core(0, split_k, *args) if split_k
+              else hk.lib().hk_bgemm(0, 1, *args))
+    assert rc == 0
+    for _ in range(3):
+        dC.zero_()
+        graph.replay()
+        _check(orc, to_host_bits(dC), A, B, C0, 0, 1, 1.0, 0.0)
+
+
+def test_bgemm_deep_k_keeps_the_wide_splits_under_capture(hk, orc):
+    # one aligned 256 x 256 tile over a deep k: eager calls split it over small tiles; a captured one
+    # takes the 256-wide tiles' splits (bit for bit those of an explicit split), not one chain
+    M, N, K = 256, 256, 65536
+    lib = hk.lib()
+    assert lib.hk_bgemm_small_tile(0, 0, M, N, K, 1, 0) > 0
+    assert lib.hk_bgemm_split_count(0, 0, M, N, K, 1, 0) > 1
+    say("bgemm capture deep k")
+    A, B, C0 = _operands(orc, M, N, K, 0, 0, 2560)
+    dA, dB, dC = to_dev_bf16(A), to_dev_bf16(B), to_dev_bf16(C0)
+    side = torch.cuda.Stream()
+
+    def call(stream, split_k=0):
+        args = (M, N, K, bits(1.0), dA.data_ptr(), K, 0, dB.data_ptr(), N, 0, 0, dC.data_ptr(), N, 0, 1,
+                stream)
+        assert (lib.hk_bgemm_core(2, split_k, *args) if split_k else lib.hk_bgemm(0, 0, *args)) == 0
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(side.cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(torch.cuda.current_stream().cuda_stream)
+    call(torch.cuda.current_stream().cuda_stream, 8)
+    wide = to_host_bits(dC)
+    for _ in range(3):
+        dC.zero_()
+        graph.replay()
+        assert np.array_equal(to_host_bits(dC), wide)
+
+
 def test_bgemm_flex_split_plan_under_capture(hk, orc):
     # A split plan takes the stream's workspace in eager calls and runs unsplit in a captured graph,
     # whose replays stay right after a larger call has grown the workspace.
