@@ -196,33 +196,46 @@ def test_bgemm_deep_k_keeps_the_wide_splits_under_capture(hk, orc):
 
 
 def test_bgemm_flex_split_plan_under_capture(hk, orc):
-    # A split plan takes the stream's workspace in eager calls and runs unsplit in a captured graph,
-    # whose replays stay right after a larger call has grown the workspace.
+    # A split plan takes the stream's workspace in eager calls and runs unsplit in a captured graph: the
+    # replays give the bits of an explicit split of one, which are not the eager call's, also after a
+    # larger call has grown the workspace.
     M, N, K = 300, 299, 4001
-    assert hk.lib().hk_bgemm_split_count(0, 0, M, N, K, 1, 0) > 1
+    lib = hk.lib()
+    assert lib.hk_bgemm_split_count(0, 0, M, N, K, 1, 0) > 1
     say("bgemm flex capture")
     A, B, C0 = _operands(orc, M, N, K, 0, 0, 2500)
     dA, dB, dC = to_dev_bf16(A), to_dev_bf16(B), to_dev_bf16(C0)
+    big = torch.randn(1500, K, device=DEV).to(torch.bfloat16)
+    out = torch.empty(1500, N, device=DEV, dtype=torch.bfloat16)
 
-    def call(stream):
-        assert hk.lib().hk_bgemm(0, 0, M, N, K, bits(1.0), dA.data_ptr(), K, 0, dB.data_ptr(), N, 0, 0,
-                                 dC.data_ptr(), N, 0, 1, stream) == 0
+    def call(stream, split_k=0, a=dA, c=dC, rows=M):
+        args = (rows, N, K, bits(1.0), a.data_ptr(), K, 0, dB.data_ptr(), N, 0, 0, c.data_ptr(), N, 0, 1,
+                stream)
+        assert (lib.hk_bgemm_core(2, split_k, *args) if split_k else lib.hk_bgemm(0, 0, *args)) == 0
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(side):
-        call(side.cuda_stream)
-    torch.cuda.synchronize()
-    eager = to_host_bits(dC)
+    got = {}
+    for name, split_k in (("whole", 1), ("eager", 0)):
+        with torch.cuda.stream(side):
+            call(side.cuda_stream, split_k)
+        torch.cuda.synchronize()
+        got[name] = to_host_bits(dC)
+        _check(orc, got[name], A, B, C0, 0, 0, 1.0, 0.0)
+    assert not np.array_equal(got["whole"], got["eager"])
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
         call(torch.cuda.current_stream().cuda_stream)
-    for _ in range(3):
+    for i in range(3):
         dC.zero_()
         graph.replay()
-        _check(orc, to_host_bits(dC), A, B, C0, 0, 0, 1.0, 0.0)
+        assert np.array_equal(to_host_bits(dC), got["whole"])
         with torch.cuda.stream(side):
             call(side.cuda_stream)
-        assert np.array_equal(to_host_bits(dC), eager)
+        assert np.array_equal(to_host_bits(dC), got["eager"])
+        # 8 x 1500 x 304 fp32 partials: more than the products above take (at most 32 x 300 x 304)
+        with torch.cuda.stream(side):
+            call(side.cuda_stream, 8, big, out, 1500)
+        torch.cuda.synchronize()
 
 
 # The 256-wide tiles at sizes that the library itself now gives to the small ones.
