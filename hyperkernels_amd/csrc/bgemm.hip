@@ -1064,6 +1064,10 @@ GemmPlan bgemm_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_
   return make_plan(ta, tb, M, N, K, batch, split_k, Rows::kAligned);
 }
 
+GemmPlan bgemm_lean_plan(bool ta, bool tb, int M, int N, int K, int batch, size_t held) {
+  return lean_plan(ta, tb, M, N, K, batch, Rows::kAligned, held);
+}
+
 hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* A, int64_t lda,
                           int64_t sA, const hk_bf16* B, int64_t ldb, int64_t sB, int batch,
                           const GemmPlan& plan, float* part, const F32Out* out,

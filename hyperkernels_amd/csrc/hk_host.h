@@ -68,11 +68,13 @@ struct F32Out {
 // multiples and 16-byte aligned bases. bgemm_plan picks how a shape runs: the tile family (flex:
 // a tile shape of bgemm_flex.hip, 0 for the 256-wide tiles), and split_k ranges of kps k each
 // (split_k == 0: the library's choice), `used` of them non-empty. bgemm_split_plan does so for the
-// 256-wide tiles alone; cost: the modelled time (us) of split_k == 0.
+// 256-wide tiles alone; cost: the modelled time (us) of split_k == 0. bgemm_lean_plan: the plan of
+// split_k == 0 where partials may take `held` bytes at most.
 struct GemmPlan {
   int flex, used, kps;
 };
 GemmPlan bgemm_plan(bool ta, bool tb, int M, int N, int K, int batch, int split_k);
+GemmPlan bgemm_lean_plan(bool ta, bool tb, int M, int N, int K, int batch, size_t held);
 void bgemm_split_plan(int M, int N, int K, int batch, int split_k, int* used, int* kps,
                       double* cost = nullptr);
 hipError_t bgemm_partials(bool ta, bool tb, int M, int N, int K, const hk_bf16* A, int64_t lda,

@@ -635,27 +635,47 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
     // A' is [M][3K] (k-major) or [3K][M]; B' is [3K][N] or [N][3K]
     const int64_t la = ta ? M : K3, lb = tb ? K3 : N;
     const int64_t na = static_cast<int64_t>(M) * K3, nb = static_cast<int64_t>(K3) * N;
-    const hk::GemmPlan plan = hk::bgemm_plan(ta, tb, M, N, K3, batchCount, splitK);
-    const int used = plan.used, kps = plan.kps;
+    hk::GemmPlan plan = hk::bgemm_plan(ta, tb, M, N, K3, batchCount, splitK);
     // the plan never exceeds the k-tile count; refuse a grid the tiles cannot take before
     // anything is allocated or launched
-    HK_CHECK_ARG(static_cast<int64_t>(batchCount) * used <= 65535);
+    HK_CHECK_ARG(static_cast<int64_t>(batchCount) * plan.used <= 65535);
     auto up = [](int64_t bytes) { return (bytes + 255) & ~int64_t{255}; };
     const int64_t a_bytes = up(na * batchCount * 2), b_bytes = up(nb * batchCount * 2);
+    const size_t ab_bytes = static_cast<size_t>(a_bytes + b_bytes);
     // Serial split-K: when the output tiles alone fill the device, concurrent k ranges add no
     // parallelism, so the ranges are added into C one after the other, in split order (the
     // first applies beta and the bias, the others beta = 1), with no fp32 partials and no
     // finalize pass. 4096^3 + bias at split-K 4: 489.7 -> 462.8 us, max-rel vs a float64
     // product 2.9e-6 both ways. Fewer tiles than CUs keep concurrent partials.
     const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    const bool serial =
-        used > 1 && plan.flex == 0 && tiles * batchCount >= hk::device_cu_count();
+    auto is_serial = [&] {
+      return plan.used > 1 && plan.flex == 0 && tiles * batchCount >= hk::device_cu_count();
+    };
     // one split (or serial ranges): the GEMM tiles write C themselves, no partials
-    const int64_t p_bytes =
-        used == 1 || serial ? 0 : static_cast<int64_t>(used) * batchCount * M * N * 4;
+    auto bytes = [&] {
+      return ab_bytes + (plan.used == 1 || is_serial()
+                             ? 0
+                             : static_cast<size_t>(plan.used) * batchCount * M * N * 4);
+    };
+    // The small tiles split k further than the 256-wide ones: where the memory for that is not
+    // there, or the workspace would have to grow under capture, a plan that does with less runs.
+    const bool optional = plan.flex && plan.used > 1;
+    if (optional && hk::stream_capturing(stream)) {
+      const size_t held = hk::device_workspace_bytes(stream);
+      if (bytes() > held)
+        plan = hk::bgemm_lean_plan(ta, tb, M, N, K3, batchCount,
+                                   held > ab_bytes ? held - ab_bytes : 0);
+    }
     void* ws = nullptr;
-    HK_RETURN_IF_ERROR(hk::device_workspace(static_cast<size_t>(a_bytes + b_bytes + p_bytes),
-                                            stream, &ws));
+    hipError_t got = hk::device_workspace(bytes(), stream, &ws);
+    if (got == hipErrorOutOfMemory && optional) {
+      (void)hipGetLastError();
+      plan = hk::bgemm_lean_plan(ta, tb, M, N, K3, batchCount, 0);
+      got = hk::device_workspace(bytes(), stream, &ws);
+    }
+    HK_RETURN_IF_ERROR(got);
+    const int used = plan.used, kps = plan.kps;
+    const bool serial = is_serial();
     uint16_t* A3 = static_cast<uint16_t*>(ws);
     uint16_t* B3 = reinterpret_cast<uint16_t*>(static_cast<char*>(ws) + a_bytes);
     float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + a_bytes + b_bytes);

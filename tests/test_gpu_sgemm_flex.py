@@ -108,3 +108,32 @@ def test_sgemm_bf16x3_small_tiles(hk, orc, M, N, K, lay):
     out = _sg_call(hk, "hk_sgemm", enum, t(A), t(B), t(C0), M, N, K, 1.5, 0.5, bias=t(bias),
                    bias_stride=N, split_k=0)
     assert max_rel(out, _ref(A, B, ta, tb, 1.5, 0.5, C0, bias)) <= 5e-5
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 256, 4096), (64, 128, 8192)])
+def test_sgemm_bf16x3_under_capture_in_the_workspace_it_has(hk, orc, M, N, K):
+    # a workspace that holds the split operands and no partials: the captured product does without
+    say("sgemm capture", M, N, K)
+    lib = hk.lib()
+    assert lib.hk_sgemm_split_count(2, M, N, K, 1, 0) > 1
+    A, B, C0, _ = _sg_operands(orc, M, N, K, 0, 0, 81)
+    a, b, c = (torch.from_numpy(x.copy()).to(DEV) for x in (A, B, C0))
+    side = torch.cuda.Stream()
+
+    def call(split_k):
+        assert lib.hk_sgemm(2, M, N, K, 1.0, a.data_ptr(), K, 0, b.data_ptr(), N, 0, 0.0, c.data_ptr(), N,
+                            0, None, 0, 1, split_k, torch.cuda.current_stream().cuda_stream) == 0
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(1)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(0)
+    for _ in range(3):
+        c.zero_()
+        graph.replay()
+        assert max_rel(c.cpu().numpy(), _ref(A, B, 0, 0)) <= 5e-5
+        with torch.cuda.stream(side):
+            call(0)  # eager: grows the workspace
+        torch.cuda.synchronize()
