@@ -773,11 +773,26 @@ hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool ze
     for (int64_t kt = 0; kt < nkt; ++kt)
       items += key_items(p.T, p.is_causal, static_cast<int>(kt), deal.chunk);
   }
-  const bool split = items > nkt;
+  bool split = items > nkt;
   const size_t part_bytes =
       split ? static_cast<size_t>(items * bh) * 2 * kBKV * kHD * sizeof(float) : 0;
+  // Where the workspace would have to grow under capture, or the memory for the partials is not
+  // there, the key tiles stay whole.
+  bool whole = split && hk::stream_capturing(stream) &&
+               planes + part_bytes > hk::device_workspace_bytes(stream);
   void* ws = nullptr;
-  HK_RETURN_IF_ERROR(hk::device_workspace(planes + part_bytes, stream, &ws));
+  if (!whole) {
+    const hipError_t e = hk::device_workspace(planes + part_bytes, stream, &ws);
+    whole = split && e == hipErrorOutOfMemory;
+    if (whole) (void)hipGetLastError();
+    else HK_RETURN_IF_ERROR(e);
+  }
+  if (whole) {
+    HK_RETURN_IF_ERROR(hk::device_workspace(planes, stream, &ws));
+    split = false;
+    items = nkt;
+    deal.chunk = query_tiles(p.T, p.is_causal, 0);
+  }
   char* wsb = static_cast<char*>(ws);
   float* l2 = reinterpret_cast<float*>(wsb + 4 * plane);
   hipLaunchKernelGGL(attn_bwd_prepare,

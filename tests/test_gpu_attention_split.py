@@ -90,3 +90,37 @@ def test_attn_backward_set_replayed_graph(hk, orc):
         torch.cuda.synchronize()
         for got, ref in zip(out, want):
             assert max_rel(got.cpu().numpy(), ref) <= 2e-3
+
+
+def test_attn_backward_under_capture_in_the_workspace_it_has(hk, orc):
+    # a workspace that holds the planes of 12 x 1024 queries and not the partials of shared key tiles,
+    # as other shapes leave it: the captured call keeps its key tiles whole
+    B, H, T = 1, 12, 1024
+    say("attn bwd capture without partials")
+    (q, k, v, do, lse), D, want = _case(hk, orc, B, H, T, True)
+    out = [torch.empty_like(q) for _ in range(3)]
+    small = [torch.randn(25, 12, 64, 64, device=DEV) for _ in range(4)]  # 19,200 rows, none shared
+    so, sl = hk.fused_attn_forward(*small[:3], True)
+    sd = hk.attn_bwd_precompute_D(small[3], so)
+    p = hk._bwd_params(q, k, v, None, do, lse, D, *out, True, 0.125)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        hk.attn_backward(*small, sl, sd, True)
+    torch.cuda.synchronize()
+
+    def call():
+        assert hk.lib().hk_attn_backward_set(ctypes.byref(p), 64,
+                                             torch.cuda.current_stream().cuda_stream) == 0
+    with torch.cuda.graph(graph, stream=side):
+        call()
+    for _ in range(3):
+        for t in out:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, ref in zip(out, want):
+            assert max_rel(got.cpu().numpy(), ref) <= 2e-3
+        with torch.cuda.stream(side):
+            call()  # eager: shares the key tiles, in a larger workspace
+        torch.cuda.synchronize()
