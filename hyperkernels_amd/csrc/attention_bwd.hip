@@ -36,14 +36,14 @@
 #include <initializer_list>
 #include <mutex>
 
+#include "attention_deal.h"
 #include "hk_device.h"
 #include "hk_host.h"
 
 namespace {
 
 constexpr int kHD = 64;
-constexpr int kBKV = 128;        // keys per workgroup
-constexpr int kBQ = 64;          // queries per inner tile
+using namespace hk::attn;        // kBKV keys per workgroup, kBQ queries per inner tile
 constexpr int kThreads = 512;    // 8 waves: 4 key groups x 2 query halves
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -189,16 +189,6 @@ struct Deal {
   int chunk;    // query tiles per workgroup
   float* part;  // NULL when every key tile has one workgroup
 };
-// Query tiles of key tile kt: all of them, or under causal masking from the one that holds the
-// tile's first key.
-__host__ __device__ inline int query_tiles(int64_t T, bool causal, int kt) {
-  const int64_t first = causal ? static_cast<int64_t>(kt) * kBKV / kBQ * kBQ : 0;
-  return static_cast<int>((T - first + kBQ - 1) / kBQ);
-}
-__host__ __device__ inline int key_items(int64_t T, bool causal, int kt, int chunk) {
-  return (query_tiles(T, causal, kt) + chunk - 1) / chunk;
-}
-
 // Vector memory operations each lane issues after a tile's copies: the dQ atomics. A wave
 // waits with vmcnt(kAtomicsPerTile) for its copies of the next tile (vector memory operations
 // complete in issue order), so the atomics themselves are never waited for.
@@ -273,13 +263,10 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   const int bh = static_cast<int>(blockIdx.x) - item * nbh;
   int kt = item, piece = 0, pieces = 1;
   if (SPLIT) {
-    kt = 0;
-    piece = item;
-    for (pieces = key_items(T, p.is_causal, 0, deal.chunk); piece >= pieces;) {
-      piece -= pieces;
-      ++kt;
-      pieces = key_items(T, p.is_causal, kt, deal.chunk);
-    }
+    const int nkt = static_cast<int>((T + kBKV - 1) / kBKV);
+    kt = item_key_tile(T, p.is_causal, nkt, item, deal.chunk);
+    piece = item - first_item(T, p.is_causal, nkt, kt, deal.chunk);
+    pieces = key_items(T, p.is_causal, kt, deal.chunk);
   }
   const int b = bh / p.nh, h = bh - b * p.nh;
   const int64_t k0 = static_cast<int64_t>(kt) * kBKV;
@@ -674,8 +661,7 @@ __global__ __launch_bounds__(kSumThreads) void attn_bwd_sum(hk_attn_bwd_params p
   const int kt = blockIdx.x / kSumBlocks, bh = blockIdx.y;
   const int pieces = key_items(p.T, p.is_causal, kt, deal.chunk);
   if (pieces == 1) return;
-  int item = 0;
-  for (int k = 0; k < kt; ++k) item += key_items(p.T, p.is_causal, k, deal.chunk);
+  const int item = first_item(p.T, p.is_causal, static_cast<int>((p.T + kBKV - 1) / kBKV), kt, deal.chunk);
   const int idx = (blockIdx.x % kSumBlocks) * kSumThreads + threadIdx.x;
   const bool is_dv = idx >= kBKV * kHD / 4;
   const int i = idx - (is_dv ? kBKV * kHD / 4 : 0);
@@ -693,37 +679,6 @@ __global__ __launch_bounds__(kSumThreads) void attn_bwd_sum(hk_attn_bwd_params p
              4 * (i % (kHD / 4));
 #pragma unroll
   for (int e = 0; e < 4; ++e) d[e] = v[e] * scale;
-}
-
-// Query tiles per workgroup: the number with the least modelled time. A workgroup takes about 11 us
-// plus 3 us per query tile; the launch lasts as long as its longest workgroup and, with more
-// workgroups than CUs (one runs per CU), as the work per CU; a split adds the sum's 5 us. Large
-// grids stay unsplit. Whole backward on MI355X, us unsplit and as picked: 12 causal heads at
-// T = 1024 66.5 and 35.2 (4 tiles), 24 heads at T = 333 34.1 and 26.9 (2 tiles).
-int pick_chunk(int64_t T, bool causal, int nkt, int64_t nbh) {
-  const double cus = static_cast<double>(hk::device_cu_count());
-  const int most = query_tiles(T, causal, 0);
-  double best = 0.0;
-  int best_chunk = most;
-  if (nkt * nbh >= 4 * static_cast<int64_t>(cus)) return most;
-  for (int chunk = most; chunk >= 1; --chunk) {
-    int64_t wgs = 0, tiles = 0;
-    for (int kt = 0; kt < nkt; ++kt) {
-      wgs += key_items(T, causal, kt, chunk);
-      tiles += query_tiles(T, causal, kt);
-    }
-    if (wgs * nbh > 8 * static_cast<int64_t>(cus)) break;
-    const double longest = 11.0 + 3.0 * chunk;
-    const double share = (11.0 * static_cast<double>(wgs) + 3.0 * static_cast<double>(tiles)) *
-                         static_cast<double>(nbh) / cus;
-    double cost = wgs * nbh <= cus ? longest : (share > longest ? share : longest) + 0.3 * longest;
-    if (wgs > nkt) cost += 5.0;
-    if (chunk == most || cost < 0.95 * best) {
-      best = cost;
-      best_chunk = chunk;
-    }
-  }
-  return best_chunk;
 }
 
 bool rows_aligned(const void* base, int64_t strideB, int64_t strideH, int64_t strideM) {
@@ -766,13 +721,10 @@ hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool ze
   const int64_t rows = bh * p.T;
   const size_t plane = static_cast<size_t>(rows) * kRowBytes;
   const size_t planes = (4 * plane + 2 * static_cast<size_t>(rows) * 4 + 255) & ~size_t{255};
-  Deal deal{pick_chunk(p.T, p.is_causal, static_cast<int>(nkt), bh), nullptr};
+  Deal deal{pick_chunk(p.T, p.is_causal, static_cast<int>(nkt), bh, hk::device_cu_count()), nullptr};
   int64_t items = nkt;
-  if (deal.chunk < query_tiles(p.T, p.is_causal, 0)) {
-    items = 0;
-    for (int64_t kt = 0; kt < nkt; ++kt)
-      items += key_items(p.T, p.is_causal, static_cast<int>(kt), deal.chunk);
-  }
+  if (deal.chunk < query_tiles(p.T, p.is_causal, 0))
+    items = first_item(p.T, p.is_causal, static_cast<int>(nkt), static_cast<int>(nkt), deal.chunk);
   bool split = items > nkt;
   const size_t part_bytes =
       split ? static_cast<size_t>(items * bh) * 2 * kBKV * kHD * sizeof(float) : 0;

@@ -27,7 +27,7 @@ def _case(hk, orc, B, H, T, causal, seeds=(301, 302, 303, 304)):
 # few heads: split into pieces of 1 to 5 query tiles, with and without a partial last tile; the last
 # shapes fill the device and stay whole
 @pytest.mark.parametrize("B,H,T", [(1, 1, 128), (1, 1, 129), (1, 1, 1000), (1, 2, 1024), (2, 12, 333),
-                                   (1, 3, 2031), (3, 5, 450), (4, 40, 190)])
+                                   (1, 3, 2031), (3, 5, 450), (4, 40, 190), (1, 1, 4000)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_attn_backward_split_queries(hk, orc, B, H, T, causal):
     say("attn bwd split", B, H, T, causal)
