@@ -424,10 +424,20 @@ FlexPlan bgemm_flex_plan(int M, int N, int K, int batch, int split_k, bool ragge
     const Shape& s = kShapes[i];
     if (s.ragged != ragged) continue;
     const int64_t tiles = ceil_div(M, s.bm) * ceil_div(N, s.bn) * batch;
+    // what each further split costs at least: the partials' finalize, a launch and an HBM pass
+    auto finalize = [&](int64_t used) {
+      return 4.5 + 0.35 * static_cast<double>(used) +
+             static_cast<double>(4 * used + 2) * M * static_cast<double>(N) * batch / 6.0e6;
+    };
     for (int want = split_k > 0 ? split_k : 1; want <= (split_k > 0 ? split_k : 32); ++want) {
       // the k range of a split is a whole number of k-tiles; `used` splits are not empty
       const int64_t kt = ceil_div(ktiles, want), used = ceil_div(ktiles, kt);
-      if (split_k == 0 && want > 1 && (used != want || kt < 4 || batch * used > 65535)) continue;
+      if (split_k == 0 && want > 1) {
+        // no later `want` can be better: its ranges are no longer, its finalize no cheaper
+        if (kt < 4 || batch * used > 65535) break;
+        if (best.tile && s.fixed + finalize(want) >= best.cost) break;
+        if (used != want) continue;
+      }
       const int64_t wgs = tiles * used, held = cus * s.per_cu;
       const int64_t full = wgs / held, last = wgs % held;
       // `share` workgroups on each CU: the slower of one's serial chain and the CU's throughput;
@@ -440,10 +450,7 @@ FlexPlan bgemm_flex_plan(int M, int N, int K, int batch, int split_k, bool ragge
       double cost = s.fixed + 1.5 * static_cast<double>(full + (last > 0) - 1);
       if (full > 0) cost += static_cast<double>(kt * full) * per_ktile(held);
       if (last > 0) cost += static_cast<double>(kt) * per_ktile(last);
-      // the partials' finalize: a launch and an HBM pass
-      if (used > 1)
-        cost += 4.5 + 0.35 * static_cast<double>(used) +
-                static_cast<double>(4 * used + 2) * M * static_cast<double>(N) * batch / 6.0e6;
+      if (used > 1) cost += finalize(used);
       if (best.tile == 0 || cost < best.cost)
         best = FlexPlan{i + 1, static_cast<int>(used), static_cast<int>(kt * BK), cost};
     }

@@ -1,8 +1,8 @@
 // runtime.hip - library-level state: ABI version, per-device facts and the workspaces.
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <utility>
-#include <vector>
 
 #include "hk_host.h"
 
@@ -13,46 +13,32 @@ extern "C" const char* hk_error_string(hipError_t status) { return hipGetErrorSt
 namespace hk {
 
 namespace {
-struct DeviceState {
-  int cu_count = 0;
-};
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
   bool captured = false;  // handed out during a stream capture: a graph may hold the address
 };
 std::mutex g_mu;
-std::vector<DeviceState> g_devices;
 // One grow-only workspace per (device, stream): work on one stream is ordered, so a call may
 // reuse the buffer the previous call on that stream used; calls on different streams never
 // share one. A buffer that a graph may hold is never freed: the buffer that takes its place is at
 // least twice as large, so those kept add up to less than the one in use.
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
-
-DeviceState* state_for_current(hipError_t* err) {
-  int dev = 0;
-  *err = hipGetDevice(&dev);
-  if (*err != hipSuccess) return nullptr;
-  if (static_cast<int>(g_devices.size()) <= dev) g_devices.resize(dev + 1);
-  return &g_devices[dev];
-}
 }  // namespace
 
+// Read several times by each call that plans a launch, so without a lock: every thread that finds no
+// count yet asks for the same number.
 int device_cu_count() {
-  std::lock_guard<std::mutex> lk(g_mu);
-  hipError_t e;
-  DeviceState* s = state_for_current(&e);
-  if (!s) return 256;
-  if (s->cu_count == 0) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        cus > 0)
-      s->cu_count = cus;
-    else
-      s->cu_count = 256;
-  }
-  return s->cu_count;
+  constexpr int kDevices = 64;
+  static std::atomic<int> count[kDevices];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev < kDevices && (cus = count[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus <= 0)
+    cus = 256;
+  if (dev < kDevices) count[dev].store(cus, std::memory_order_relaxed);
+  return cus;
 }
 
 bool stream_capturing(hipStream_t stream) {
