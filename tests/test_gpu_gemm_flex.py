@@ -238,6 +238,16 @@ def test_bgemm_flex_split_plan_under_capture(hk, orc):
         torch.cuda.synchronize()
 
 
+# Large outputs of few k are bound by their stores: several rounds of small tiles lose to the 256-wide
+# ones there (43.4 us against 28.3 for the first), one round wins.
+@pytest.mark.parametrize("M,N,K,small", [(5208, 6880, 80, False), (1704, 6208, 64, False),
+                                         (536, 9576, 312, False), (512, 50304, 64, False),
+                                         (1024, 4096, 64, True), (2048, 2048, 16, True),
+                                         (1432, 2160, 368, True)])
+def test_bgemm_small_tiles_by_rounds(hk, M, N, K, small):
+    assert (hk.lib().hk_bgemm_small_tile(0, 1, M, N, K, 1, 0) > 0) == small
+
+
 # The 256-wide tiles at sizes that the library itself now gives to the small ones.
 @pytest.mark.parametrize("M,N,K,ta,tb,rows,cols", [
     (192, 256, 64, 0, 0, 192, 256), (200, 264, 136, 0, 1, 192, 256), (400, 512, 72, 0, 0, 192, 256),
