@@ -542,21 +542,25 @@ hipError_t dispatch_layout(bool ta, bool tb, dim3 grid, hipStream_t stream, int 
 // The product paths of an fp32 GEMM and the k-split plan each runs.
 enum class SgemmPath { kSimple, kFlex, kBf16x3, kFp32Tiles };
 
+// Rows that the fp32 MFMA tiles take: 4-element multiples for every contiguous extent, leading
+// dimension and batch stride, 16-byte aligned bases.
+bool tiled_rows(bool ta, bool tb, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
+                int64_t sA, int64_t sB, int64_t sC, bool aligned) {
+  const int contig_a = ta ? M : K, contig_b = tb ? K : N;
+  return (contig_a % 4 == 0) && (contig_b % 4 == 0) && (N % 4 == 0) && (lda % 4 == 0) &&
+         (ldb % 4 == 0) && (ldc % 4 == 0) && (sA % 4 == 0) && (sB % 4 == 0) && (sC % 4 == 0) &&
+         aligned && K > 0 &&
+         // per-lane source offsets inside a tile are 32-bit byte offsets
+         lda < (1 << 21) && ldb < (1 << 21);
+}
 // Which path takes a product. kFlex: the fp32 MFMA tiles of sgemm_flex.hip, any alignment; it also
-// takes the products of 4-element multiples that leave a quarter of the CUs without a 256 x 256
-// tile, unless the caller gives the split. Tiles: 4-element multiples for every contiguous extent, leading
-// dimension and batch stride, 16-byte aligned bases. bf16x3 additionally needs every dimension
-// the split copies touch to be a multiple of 8 and the tripled k axis to fit the BF16 tiles'
-// 32-bit per-lane offsets.
+// takes the products of tiled_rows that leave a quarter of the CUs without a 256 x 256 tile, unless the
+// caller gives the split. bf16x3 additionally needs every dimension the split copies touch to be a
+// multiple of 8 and the tripled k axis to fit the BF16 tiles' 32-bit per-lane offsets.
 SgemmPath sgemm_path(bool ta, bool tb, int M, int N, int K, int64_t lda, int64_t ldb,
                      int64_t ldc, int64_t sA, int64_t sB, int64_t sC, int batchCount,
                      bool aligned, int split_k) {
-  const int contig_a = ta ? M : K, contig_b = tb ? K : N;
-  const bool tiled_ok = (contig_a % 4 == 0) && (contig_b % 4 == 0) && (N % 4 == 0) &&
-                        (lda % 4 == 0) && (ldb % 4 == 0) && (ldc % 4 == 0) && (sA % 4 == 0) &&
-                        (sB % 4 == 0) && (sC % 4 == 0) && aligned && K > 0 &&
-                        // per-lane source offsets inside a tile are 32-bit byte offsets
-                        lda < (1 << 21) && ldb < (1 << 21);
+  const bool tiled_ok = tiled_rows(ta, tb, M, N, K, lda, ldb, ldc, sA, sB, sC, aligned);
   const bool flex_ok = K > 0 && lda >= 4 && ldb >= 4 && lda < (1 << 21) && ldb < (1 << 21) &&
                        batchCount <= 65535;
   if (!tiled_ok) return flex_ok ? SgemmPath::kFlex : SgemmPath::kSimple;
@@ -603,10 +607,9 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
                  bias_stride == 1);
   }
   const Epilogue ep{alpha, beta, bias, bias ? static_cast<int64_t>(bias_stride) : 0, bias_scale};
+  const bool aligned = hk::aligned16(A) && hk::aligned16(B) && hk::aligned16(C);
   const SgemmPath path = sgemm_path(ta, tb, M, N, K, lda, ldb, ldc, strideA, strideB, strideC,
-                                    batchCount,
-                                    hk::aligned16(A) && hk::aligned16(B) && hk::aligned16(C),
-                                    splitK);
+                                    batchCount, aligned, splitK);
   if (path == SgemmPath::kSimple) {
     dim3 grid((N + 15) / 16, (M + 15) / 16, batchCount);
     hipLaunchKernelGGL(sgemm_simple, grid, dim3(256), 0, stream, ta ? 1 : 0, tb ? 1 : 0, M, N, K,
@@ -616,10 +619,12 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
     return hk::launch_status();
   }
   if (path == SgemmPath::kFlex) {
-    double cost = 0.0;
-    const int shape = hk::sgemm_flex_plan(M, N, K, batchCount, &cost);
+    // rows that the 256 x 256 tiles take, too: serial sums no longer than in their k splits
+    int used = 1, kps = K;
+    if (tiled_rows(ta, tb, M, N, K, lda, ldb, ldc, strideA, strideB, strideC, aligned))
+      fp32_split_plan(M, N, K, batchCount, 0, &used, &kps);
     return hk::sgemm_flex_run(
-        shape,
+        hk::sgemm_flex_plan(M, N, K, batchCount, used),
         hk::SgemmFlexCall{ta, tb, M, N, K, batchCount, A, lda, strideA, B, ldb, strideB,
                           hk::F32Out{C, ldc, strideC, ep.alpha, ep.beta, ep.bias, ep.bias_stride,
                                      ep.bias_scale}},

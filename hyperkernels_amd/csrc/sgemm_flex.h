@@ -15,8 +15,9 @@ struct SgemmFlexCall {
   int64_t ldb, sB;
   F32Out out;
 };
-// Index of the tile shape for a product and its modelled time (us).
-int sgemm_flex_plan(int M, int N, int K, int batch, double* cost);
+// Index of the tile shape for a product: the least modelled time among those that form an output's sum
+// from min_chains serial ones at least, or from as many as any shape does.
+int sgemm_flex_plan(int M, int N, int K, int batch, int min_chains);
 hipError_t sgemm_flex_run(int shape, const SgemmFlexCall& call, hipStream_t stream);
 
 }  // namespace hk

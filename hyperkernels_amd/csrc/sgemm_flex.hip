@@ -9,8 +9,12 @@
 // 128 x 128 (2 x 2 waves). K-tiles of 32 fp32 are loaded 16 bytes per lane at any 4-byte address
 // into registers, one k-tile ahead, and written to a ring of two LDS slots; a vector that would
 // cross the end of K, or of the matrix in its last k-row, is read element by element, with zeros
-// past K. LDS holds K-major operands as [row][32 k] and M/N-major ones as [32 k][row], as in
-// sgemm.hip: lane (r, h) of a wave feeds k = 16 h + s of each k-tile at MFMA step s.
+// past K. An output's fp32 sum is formed from KG x NA serial ones (NA accumulator sets per wave, MFMA
+// steps in turn): 8, 4 and 1 for the three tiles, at no cost in time (1500 x 1500 x 772 NN 47 us with
+// one set and with four, error against 64 bits 5.0e-7 and 2.5e-7; 260 x 260 x 16388 NT 110 us, 1.15e-6
+// with 4 sums, 8.1e-7 with 8, as 8 k splits of the 256 x 256 tiles have). LDS holds K-major operands
+// as [row][32 k] and M/N-major ones as [32 k][row], as in sgemm.hip: lane (r, h) of a wave feeds
+// k = 16 h + s of each k-tile at MFMA step s.
 #include <mutex>
 
 #include "bgemm_tile.h"
@@ -62,9 +66,10 @@ __device__ __forceinline__ f32x4_t load_some(const float* p, int n) {
   return v;
 }
 
-template <int BMT_, int BNT_, int WM_, int WN_, int KG_>
+template <int BMT_, int BNT_, int WM_, int WN_, int KG_, int NA_>
 struct Tile {
-  static constexpr int BMT = BMT_, BNT = BNT_, WM = WM_, WN = WN_, KG = KG_;
+  static constexpr int BMT = BMT_, BNT = BNT_, WM = WM_, WN = WN_, KG = KG_, NA = NA_;
+  static constexpr int kChains = KG * NA;  // serial sums that an output is formed from
   static constexpr int kGroupWaves = WM * WN, kThreads = kGroupWaves * KG * 64;
   static constexpr int kWaveM = BMT / WM, kWaveN = BNT / WN;
   static constexpr int kBlkM = kWaveM / 32, kBlkN = kWaveN / 32;
@@ -164,11 +169,13 @@ __global__ __launch_bounds__(T::kThreads, 2) void sgemm_flex(hk::SgemmFlexCall g
           16 * lane) = reg[q];
   };
 
-  f32x16_t acc[kBlkM][kBlkN];
+  f32x16_t sum[T::NA][kBlkM][kBlkN];  // MFMA step s adds into set s % NA
 #pragma unroll
-  for (int i = 0; i < kBlkM; ++i)
+  for (int a = 0; a < T::NA; ++a)
 #pragma unroll
-    for (int j = 0; j < kBlkN; ++j) acc[i][j] = f32x16_t{};
+    for (int i = 0; i < kBlkM; ++i)
+#pragma unroll
+      for (int j = 0; j < kBlkN; ++j) sum[a][i][j] = f32x16_t{};
 
   if (ktiles > 0) {
     load(0);
@@ -193,8 +200,8 @@ __global__ __launch_bounds__(T::kThreads, 2) void sgemm_flex(hk::SgemmFlexCall g
       for (int i = 0; i < kBlkM; ++i)
 #pragma unroll
         for (int j = 0; j < kBlkN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[buf][j][e], fa[buf][i][e], acc[i][j],
-                                                           0, 0, 0);
+          sum[e % T::NA][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+              fb[buf][j][e], fa[buf][i][e], sum[e % T::NA][i][j], 0, 0, 0);
   };
   if (ktiles > 0) read(0, 0, 0);
   // Quads 0 .. 2 read the next quad's operands while they multiply, and the next k-tile is written
@@ -228,6 +235,13 @@ __global__ __launch_bounds__(T::kThreads, 2) void sgemm_flex(hk::SgemmFlexCall g
   for (; kt < loops; ++kt) ktile(kt, std::false_type{});
 
   __syncthreads();
+  f32x16_t (&acc)[kBlkM][kBlkN] = sum[0];
+#pragma unroll
+  for (int a = 1; a < T::NA; ++a)
+#pragma unroll
+    for (int i = 0; i < kBlkM; ++i)
+#pragma unroll
+      for (int j = 0; j < kBlkN; ++j) acc[i][j] += sum[a][i][j];
   if constexpr (T::KG > 1) {  // the k groups' sums, added in group order
     unsigned char HK_LDS* sums = lds + T::kGroupWaves * T::kStaging;
     constexpr int kPerWave = kBlkM * kBlkN * 4;
@@ -308,33 +322,40 @@ hipError_t layouts(const hk::SgemmFlexCall& c, hipStream_t stream) {
 // The tile shapes: us per k of one workgroup that has its CU alone, of each of several that share
 // one, and the fixed time of a launch. On MI355X, us (TFLOP/s; the fallback ran at about 2):
 //   4095^3 NT / NN / TN       1083 / 1055 / 999 (127 / 130 / 138) on 128 x 128, 1127 on 64 x 64
-//   2049 x 2047 x 1025 NN      103 (84) on 64 x 64, 144 on 128 x 128
+//   2049 x 2047 x 1025 NN       98 (88) on 64 x 64, 144 on 128 x 128
 //   511 x 511 x 2049 TT       20.3 (53) on 32 x 32, 47.7 on 64 x 64
 struct Shape {
-  int bm, bn;
+  int bm, bn, chains;
   double alone, shared, fixed;
   hipError_t (*run)(const hk::SgemmFlexCall&, hipStream_t);
 };
+template <class T>
+constexpr Shape shape(double alone, double shared, double fixed) {
+  return Shape{T::BMT, T::BNT, T::kChains, alone, shared, fixed, &layouts<T>};
+}
 const Shape kShapes[] = {
-    {32, 32, 0.0063, 0.0060, 3.8, &layouts<Tile<32, 32, 1, 1, 4>>},
-    {64, 64, 0.0205, 0.0178, 3.4, &layouts<Tile<64, 64, 2, 2, 1>>},
-    {128, 128, 0.070, 0.0643, 5.0, &layouts<Tile<128, 128, 2, 2, 1>>},
+    shape<Tile<32, 32, 1, 1, 4, 2>>(0.0063, 0.0060, 3.8),
+    shape<Tile<64, 64, 2, 2, 1, 4>>(0.0205, 0.0178, 3.4),
+    shape<Tile<128, 128, 2, 2, 1, 1>>(0.070, 0.0643, 5.0),
 };
+constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 
 }  // namespace
 
 namespace hk {
 
-int sgemm_flex_plan(int M, int N, int K, int batch, double* cost) {
+int sgemm_flex_plan(int M, int N, int K, int batch, int min_chains) {
   const int64_t cus = device_cu_count();
-  int best = 0;
-  for (int i = 0; i < 3; ++i) {
+  int best = 0;  // the first shape has the most chains
+  double cost = 0.0;
+  for (int i = 0; i < kNumShapes; ++i) {
     const Shape& s = kShapes[i];
+    if (i > 0 && s.chains < min_chains) continue;
     const int64_t wgs = ceil_div(M, s.bm) * ceil_div(N, s.bn) * batch;
     const double share = static_cast<double>(ceil_div(wgs, cus)) * s.shared;
     const double t = s.fixed + K * (share > s.alone ? share : s.alone);
-    if (i == 0 || t < *cost) {
-      *cost = t;
+    if (i == 0 || t < cost) {
+      cost = t;
       best = i;
     }
   }

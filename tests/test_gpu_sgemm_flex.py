@@ -56,6 +56,25 @@ def test_sgemm_any_rows_error_not_above_fp32_sums(hk, orc):
         assert err(out) <= err(serial)
 
 
+@pytest.mark.parametrize("M,N,K", [(132, 204, 2052), (68, 380, 2404), (260, 260, 4100),
+                                   (516, 516, 8196)])
+@pytest.mark.parametrize("lay", ["NN", "NT", "TN"])
+def test_sgemm_multiples_of_four_error_not_above_the_split_tiles(hk, orc, M, N, K, lay):
+    # few 256 x 256 tiles over a deep k ran split 8 ways; the small tiles that take them now may be no
+    # further from 64 bits. Both are root mean squares over more than 20,000 outputs: 5% for chance.
+    enum, ta, tb = SG_LAYOUT[lay]
+    A, B, _, _ = _sg_operands(orc, M, N, K, ta, tb, 43, normal=True)
+    assert hk.lib().hk_sgemm_split_count(enum, M, N, K, 1, 0) == 1
+    assert hk.lib().hk_sgemm_split_count(enum, M, N, K, 1, 8) >= 7
+    ref, err = _ref(A, B, ta, tb), []
+    for split_k in (8, 0):
+        out = _sg_call(hk, "hk_sgemm", enum, torch.from_numpy(A).to(DEV), torch.from_numpy(B).to(DEV),
+                       torch.zeros(M, N, device=DEV), M, N, K, 1.0, 0.0, split_k=split_k)
+        err.append(np.linalg.norm(out - ref) / np.linalg.norm(ref))
+    say("sgemm flex error", lay, M, N, K, "split 8", err[0], "small tiles", err[1])
+    assert err[1] <= 1.05 * err[0]
+
+
 @pytest.mark.parametrize("pad,offset", [(1, 1), (2, 0), (4, 3), (0, 2)])
 @pytest.mark.parametrize("lay", ["NN", "NT", "TN"])
 def test_sgemm_strided_rows_between_nans(hk, orc, pad, offset, lay):
