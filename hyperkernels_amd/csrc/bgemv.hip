@@ -74,7 +74,7 @@ __device__ __forceinline__ float dot8(const uint4& a, const uint4& b) {
 
 // How 16-byte vectors of a row are loaded: not at all (element loads: a strided x), from 16-byte
 // aligned addresses, or from any 2-byte address. gfx950 serves unaligned 16-byte loads at close to
-// the aligned rate: 50304 x 921 (rows of odd length), two of them, 81 -> 17 us on MI355X.
+// the aligned rate: 50304 x 921 (rows of odd length), two products, 81 -> 44 us on MI355X.
 enum Rows { kElements, kAligned, kAnywhere };
 typedef uint32_t u32x4a2_t __attribute__((ext_vector_type(4), aligned(2)));
 template <int ROWS>
@@ -335,6 +335,9 @@ hipError_t bgemv_run(bool dot_form, int R, int K, hk_bf16 alpha, hk_bf16 beta,
   Out out{bf16_bits_to_float(alpha), bf16_bits_to_float(beta), y, incy, sy, nullptr, 1};
   const int64_t strips = dot_form ? hk::ceil_div(R, kDotRows) : hk::ceil_div(R, kColsPerWave);
   HK_CHECK_ARG(strips <= INT32_MAX);
+  // Batches of one matrix launch fewer workgroups than are counted here (gemv_dot_shared). Counting
+  // those launched splits k further, which the finalize outweighs (MI355X, us: 20000 x 1024, two
+  // vectors 9.3 -> 11.2; 12000 x 1024, four 9.3 -> 11.1; the other way 5000 x 4096, four 17.8 -> 15.5).
   int nsplit = 1, kchunk = K;
   if (dot_form)
     pick_split(strips * batch, kDotTargetGroups, K, 4 * kDotStep, kDotStep, &nsplit, &kchunk);
