@@ -672,6 +672,10 @@ constexpr int kMaxWideCols = 4096;    // four waves per row
 // one launch against two, us per call back to back (a call costs its caller 3.4): 64 x 768 fp32 3.4
 // against 6.9, 512 x 768 4.1 against 7.0, 300 x 4096 bf16 7.6 against 11.3.
 constexpr int kFewRows = 512;
+// The same for rows of more than kMaxWideCols columns, whose slabs are the other way (gradients alone,
+// us, one launch against slabs: 20 x 8200 fp32 7.7 against 10.5, 100 x 8200 7.7 and 10.4, 512 x 8200 12.7
+// and 10.0).
+constexpr int kFewLongRows = 128;
 template <typename T>
 constexpr int kMaxFewVpl = T::kPerVec == 4 ? 12 : 8;  // fp32 rows of 16 vectors per lane spill
 template <typename T>
@@ -837,6 +841,19 @@ hipError_t launch_dx(const St<T>* dy, const St<T>* x, const float* mean, const f
   });
 }
 
+// Few rows: `row_groups` workgroups of grad_x rows (0: the gradients alone) and those of the columns.
+template <typename T>
+hipError_t launch_few_rows(void (*kernel)(const St<T>*, const St<T>*, const float*, const float*,
+                                          const St<T>*, St<T>*, float*, float*, int, int, float, int),
+                           const St<T>* dy, const St<T>* x, const float* mean, const float* rstd,
+                           const St<T>* gamma, St<T>* dx, float* dgamma, float* dbeta, int rows,
+                           int cols, int row_groups, hipStream_t stream) {
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(row_groups + hk::ceil_div(cols, kFinCols))),
+                     dim3(kFinCols * kFinGroups), 0, stream, dy, x, mean, rstd, gamma, dx, dgamma,
+                     dbeta, rows, cols, 1.0f / static_cast<float>(cols), row_groups);
+  return hk::launch_status();
+}
+
 template <typename T>
 hipError_t launch_bwd(const St<T>* dy, const St<T>* x, const float* mean, const float* rstd,
                       const St<T>* gamma, St<T>* dx, float* dgamma, float* dbeta, int rows,
@@ -855,21 +872,27 @@ hipError_t launch_bwd(const St<T>* dy, const St<T>* x, const float* mean, const 
   if (!do_gb) return launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream);
   const int vpl = row_vpl<T>(cols);
   const float inv_cols = 1.0f / static_cast<float>(cols);
-  if (rows <= kFewRows && vpl > 0 && vpl <= kMaxFewVpl<T> && !in_place) {
-    const int row_groups =
-        write_dx ? static_cast<int>(hk::ceil_div(rows, kFinCols * kFinGroups / HK_WAVE)) : 0;
-    const unsigned grid = static_cast<unsigned>(row_groups + hk::ceil_div(cols, kFinCols));
+  if (rows <= kFewRows && write_dx && vpl > 0 && vpl <= kMaxFewVpl<T> && !in_place) {
+    const int row_groups = static_cast<int>(hk::ceil_div(rows, kFinCols * kFinGroups / HK_WAVE));
     return with_vpl(vpl, [&](auto vpl_c) -> hipError_t {
       constexpr int V = decltype(vpl_c)::value;
       if constexpr (V > kMaxFewVpl<T>) {
         return hipErrorInvalidValue;
       } else {
-        hipLaunchKernelGGL((vec ? ln_bwd_few_rows<T, V, false> : ln_bwd_few_rows<T, V, true>),
-                           dim3(grid), dim3(kFinCols * kFinGroups), 0, stream, dy, x, mean, rstd,
-                           gamma, dx, dgamma, dbeta, rows, cols, inv_cols, row_groups);
-        return hk::launch_status();
+        return launch_few_rows<T>(vec ? ln_bwd_few_rows<T, V, false> : ln_bwd_few_rows<T, V, true>,
+                                  dy, x, mean, rstd, gamma, dx, dgamma, dbeta, rows, cols,
+                                  row_groups, stream);
       }
     });
+  }
+  // The gradients of few rows alone, of any length, since no row is held; rows of less than a vector get
+  // their grad_x from a second launch (it may be written over dy or x).
+  const int few = cols > kMaxWideCols ? kFewLongRows : kFewRows;
+  if (rows <= few && (!write_dx || cols < T::kPerVec)) {
+    HK_RETURN_IF_ERROR(launch_few_rows<T>(ln_bwd_few_rows<T, 1, false>, dy, x, mean, rstd, gamma, dx,
+                                          dgamma, dbeta, rows, cols, 0, stream));
+    if (write_dx) return launch_dx<T>(dy, x, mean, rstd, gamma, dx, rows, cols, vec, stream);
+    return hipSuccess;
   }
   // Whole vectors of up to kMaxGbCols columns have always used the stream's workspace. The other
   // shapes do without it while a graph is being captured: the graph would keep its address, and a

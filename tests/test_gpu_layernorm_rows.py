@@ -116,10 +116,28 @@ def test_layernorm_backward_under_capture(hk, orc, rows, cols):
                                torch.zeros(4096, device=DEV))
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (16, 4096), (20, 8200), (128, 5000), (129, 5000), (33, 3),
+                                       (512, 17)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layernorm_gradients_alone(hk, rows, cols, dtype):
+    # the gamma/beta entry point on few rows of any length, against 64 bits: fp32 sums of `rows` terms,
+    # pairwise over 32 groups
+    say("layernorm gradients alone", rows, cols, dtype)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(rows + cols)
+    x, dy = (torch.randn(rows, cols, generator=g, device=DEV).to(dtype) for _ in range(2))
+    _, m, r = hk.layer_norm_forward(x)
+    sums = torch.ones(2, cols, device=DEV)  # added into
+    hk.ln_backward_gamma_beta(dy, x, m, r, sums[0], sums[1])
+    xh = (x.double() - m.double()[:, None]) * r.double()[:, None]
+    want = torch.stack([(dy.double() * xh).sum(0), dy.double().sum(0)]) + 1
+    assert max_rel(host(sums), want.cpu().numpy()) <= 2e-6
+
+
 # Both sides of the one-launch limit (512 rows) in every form of a row: whole vectors of one wave,
 # overlapping vectors, four waves, a workgroup per row, less than a vector
 @pytest.mark.parametrize("rows,cols", [(64, 768), (512, 768), (513, 768), (512, 333), (600, 333),
-                                       (512, 2560), (600, 2560), (512, 8200), (600, 8200), (512, 3)])
+                                       (512, 2560), (600, 2560), (128, 8200), (600, 8200), (512, 3)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("into", ["dy", "x"])
 @pytest.mark.parametrize("captured", [False, True])
