@@ -591,8 +591,10 @@ extern "C" hipError_t hk_fused_attn_forward(const hk_attn_fwd_params* params, in
   // Two key groups while no CU gets a second workgroup: measured on MI355X, causal T 1024: 96
   // workgroups 40.8 -> 31.5 us, 192 workgroups 40.6 -> 32.4; T 2048, 256 workgroups 74.9 -> 56.0;
   // not causal T 333, 72 workgroups 18.0 -> 16.2. Beyond that the second workgroup fills the CU
-  // already: T 1300, 264 workgroups 64.8 with one group, 74.8 with two.
-  const bool groups = nqt * bh <= hk::device_cu_count();
+  // already: T 1300, 264 workgroups 64.8 with one group, 74.8 with two. Up to four key tiles the merge
+  // costs what the shorter chain saves or more: 192 heads of 64 6.4 us with one group, 7.2 with two, 12
+  // of 128 8.8 and 9.1; 12 of 200 12.4 and 11.8.
+  const bool groups = nqt * bh <= hk::device_cu_count() && p.T > 4 * kBKV;
   auto* run = drop ? (groups ? launch_fwd<true, 2> : launch_fwd<true, 1>)
                    : (groups ? launch_fwd<false, 2> : launch_fwd<false, 1>);
   return run(p, static_cast<int>(nqt * bh), static_cast<int>(bh), mvec, stream);

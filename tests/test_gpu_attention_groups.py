@@ -1,6 +1,6 @@
-"""hk_fused_attn_forward on grids small enough for two key groups per workgroup, against a float64
-reference: key counts that leave the second group without a tile, with a partial one, or one tile
-behind; dropout, and rows whose keys one group holds alone or that keep nothing. Tolerance: the
+"""hk_fused_attn_forward on grids small enough for two key groups per workgroup (more than 128 keys) and
+on fewer keys, against a float64 reference: key counts and masks that leave the second group without a
+tile, with a partial one, or one tile behind; dropout, and rows whose keys one group holds alone or that keep nothing. Tolerance: the
 bf16x3 products (relative 2^-16 each) summed over 64 products and T keys of weight 1 in all,
 1e-4 of max|ref|. The same heads in a grid too large for it take one group and agree as closely."""
 from __future__ import annotations
@@ -27,7 +27,7 @@ def _reference(q, k, v, causal, mask):
 
 @pytest.mark.parametrize("drop", [False, True])
 @pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("T", [1, 31, 32, 33, 63, 65, 128, 129, 333, 516])
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 63, 65, 128, 129, 160, 161, 193, 333, 516])
 def test_key_groups(hk, T, causal, drop):
     print("[case] attention groups", T, causal, drop, flush=True)
     torch.manual_seed(T)
