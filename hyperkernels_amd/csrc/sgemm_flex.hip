@@ -315,15 +315,16 @@ hipError_t launch(const hk::SgemmFlexCall& c, hipStream_t stream) {
 }
 template <class T>
 hipError_t layouts(const hk::SgemmFlexCall& c, hipStream_t stream) {
-  if (!c.ta) return c.tb ? launch<T, true, true>(c, stream) : launch<T, true, false>(c, stream);
-  return c.tb ? launch<T, false, true>(c, stream) : launch<T, false, false>(c, stream);
+  HK_CHECK_ARG(!(c.ta && c.tb));  // the fp32 entry points have NT, TN and NN
+  if (c.ta) return launch<T, false, false>(c, stream);
+  return c.tb ? launch<T, true, true>(c, stream) : launch<T, true, false>(c, stream);
 }
 
 // The tile shapes: us per k of one workgroup that has its CU alone, of each of several that share
 // one, and the fixed time of a launch. On MI355X, us (TFLOP/s; the fallback ran at about 2):
-//   4095^3 NT / NN / TN       1083 / 1055 / 999 (127 / 130 / 138) on 128 x 128, 1127 on 64 x 64
-//   2049 x 2047 x 1025 NN       98 (88) on 64 x 64, 144 on 128 x 128
-//   511 x 511 x 2049 TT       20.3 (53) on 32 x 32, 47.7 on 64 x 64
+//   4095^3 NT / NN / TN       1170 / 1058 / 1000 (117 / 130 / 137) on 128 x 128
+//   2049 x 2047 x 1025 NN       98 (88) on 64 x 64
+//   511 x 511 x 2049 NN       20.0 (53) on 32 x 32
 struct Shape {
   int bm, bn, chains;
   double alone, shared, fixed;
