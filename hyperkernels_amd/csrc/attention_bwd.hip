@@ -730,8 +730,8 @@ hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool ze
       split ? static_cast<size_t>(items * bh) * 2 * kBKV * kHD * sizeof(float) : 0;
   // Where the workspace would have to grow under capture, or the memory for the partials is not
   // there, the key tiles stay whole.
-  bool whole = split && hk::stream_capturing(stream) &&
-               planes + part_bytes > hk::device_workspace_bytes(stream);
+  bool whole = split && planes + part_bytes > hk::device_workspace_bytes(stream) &&
+               hk::stream_capturing(stream);
   void* ws = nullptr;
   if (!whole) {
     const hipError_t e = hk::device_workspace(planes + part_bytes, stream, &ws);

@@ -665,12 +665,10 @@ hipError_t sgemm_run(bool ta, bool tb, int M, int N, int K, float alpha, const f
     // The small tiles split k further than the 256-wide ones: where the memory for that is not
     // there, or the workspace would have to grow under capture, a plan that does with less runs.
     const bool optional = plan.flex && plan.used > 1;
-    if (optional && hk::stream_capturing(stream)) {
-      const size_t held = hk::device_workspace_bytes(stream);
-      if (bytes() > held)
-        plan = hk::bgemm_lean_plan(ta, tb, M, N, K3, batchCount,
-                                   held > ab_bytes ? held - ab_bytes : 0);
-    }
+    const size_t held = optional ? hk::device_workspace_bytes(stream) : 0;
+    if (optional && bytes() > held && hk::stream_capturing(stream))
+      plan = hk::bgemm_lean_plan(ta, tb, M, N, K3, batchCount,
+                                 held > ab_bytes ? held - ab_bytes : 0);
     void* ws = nullptr;
     hipError_t got = hk::device_workspace(bytes(), stream, &ws);
     if (got == hipErrorOutOfMemory && optional) {
