@@ -299,8 +299,8 @@ HK_API hipError_t hk_reduce_generic_f32(const float* src, float* dst, int out_nd
  *   backward entry points (the library's choice), the hk_bgemm_core argument otherwise. 1 for
  *   the GEMV and fallback kernels, 0 for an empty product, -1 for an invalid argument.
  * Any M, N, K, leading dimension, stride and 2-byte aligned pointer (the reference needs multiples
- *   of 8, bgemm_test.cu:252-256); leading dimensions under 8 or from 2^22 on run on a slower
- *   fp32-accumulating kernel unless the rows are aligned.
+ *   of 8, bgemm_test.cu:252-256). Leading dimensions from 2^22 on, those under 8 of unaligned rows and
+ *   more than 65,535 batches of unaligned rows run on a slower fp32-accumulating kernel.
  * ---------------------------------------------------------------------------------------- */
 #define HK_LAYOUT_NT 0
 #define HK_LAYOUT_TN 1
@@ -326,7 +326,10 @@ HK_API int hk_bgemm_split_count(int transA, int transB, int M, int N, int K, int
 /* hk_bgemm_small_tile (no counterpart in the reference: a host-only planning query, like
  * hk_bgemm_split_count) returns the rows per output tile, 64 to 256, when a product of this shape
  * runs on the small or any-alignment tiles, 0 when it runs on the 256-wide ones, the GEMV or the
- * fallback kernels, -1 for an invalid argument. An explicit splitK keeps the 256-wide tiles for
+ * fallback kernels, -1 for an invalid argument. Like hk_bgemm_split_count it describes eager calls: a
+ * call that is captured into a graph leaves out the splits of the small tiles and of unaligned rows
+ * (aligned ones take the 256-wide tiles' splits where the stream's workspace holds their partials and
+ * that is faster), and so does one whose splits the grid or the memory does not take. An explicit splitK keeps the 256-wide tiles for
  * rows they take. hk_bgemm_tile_rows and hk_bgemm_tile_cols describe the 256-wide tiles' plan of a
  * shape, whether or not its product runs on them.
  * hk_bgemm_tile_rows returns the rows per output tile of that plan: 256, or 192 when 256-row tiles
