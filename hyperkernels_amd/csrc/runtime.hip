@@ -22,7 +22,8 @@ std::mutex g_mu;
 // One grow-only workspace per (device, stream): work on one stream is ordered, so a call may
 // reuse the buffer the previous call on that stream used; calls on different streams never
 // share one. A buffer that a graph may hold is never freed: the buffer that takes its place is at
-// least twice as large, so those kept add up to less than the one in use.
+// least twice as large (while there is memory for that), so those kept add up to less than the one
+// in use.
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 }  // namespace
 
@@ -59,8 +60,15 @@ hipError_t device_workspace(size_t bytes, hipStream_t stream, void** out) {
     size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
     if (w.captured) {
       void* ptr = nullptr;
-      if (want < 2 * w.bytes) want = 2 * w.bytes;
-      HK_RETURN_IF_ERROR(hipMalloc(&ptr, want));
+      const size_t twice = 2 * w.bytes;
+      hipError_t e = hipMalloc(&ptr, want < twice ? twice : want);
+      if (e == hipErrorOutOfMemory && want < twice) {
+        (void)hipGetLastError();
+        e = hipMalloc(&ptr, want);
+      } else if (want < twice) {
+        want = twice;
+      }
+      HK_RETURN_IF_ERROR(e);
       w = Workspace{ptr, want, false};
     } else {
       if (w.ptr) {
