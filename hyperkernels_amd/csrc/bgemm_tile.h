@@ -331,6 +331,43 @@ __device__ __forceinline__ void store_f32(const f32x16_t (&acc)[kBlkM][kWaveN / 
   });
 }
 
+// Adds the accumulators of the T::KG k groups of a workgroup, in group order, into those of group 0,
+// through LDS behind the groups' staging areas (T::kSums bytes for each further group). True for the
+// waves of the other groups, which are done then.
+template <class T>
+__device__ __forceinline__ bool merge_groups(f32x16_t (&acc)[T::kBlkM][T::kBlkN],
+                                             unsigned char HK_LDS* lds, int group, int wave,
+                                             int lane) {
+  unsigned char HK_LDS* sums = lds + T::kGroupWaves * T::kStaging;
+  constexpr int kPerWave = T::kBlkM * T::kBlkN * 4;
+  auto at = [&](int grp, int b, int q) {
+    return reinterpret_cast<f32x4_t HK_LDS*>(
+        sums + (grp - 1) * T::kSums + ((wave * kPerWave + b * 4 + q) * 64 + lane) * 16);
+  };
+  if (group > 0) {
+#pragma unroll
+    for (int b = 0; b < T::kBlkM * T::kBlkN; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x16_t& v = acc[b / T::kBlkN][b % T::kBlkN];
+        *at(group, b, q) = f32x4_t{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+      }
+  }
+  __syncthreads();
+  if (group > 0) return true;
+#pragma unroll
+  for (int grp = 1; grp < T::KG; ++grp)
+#pragma unroll
+    for (int b = 0; b < T::kBlkM * T::kBlkN; ++b)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4_t v = *at(grp, b, q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[b / T::kBlkN][b % T::kBlkN][4 * q + e] += v[e];
+      }
+  return false;
+}
+
 // Row pitch (elements) of the fp32 split-K partials: whole 32-byte groups for any N.
 __host__ __device__ __forceinline__ int part_pitch(int N) { return (N + 7) & ~7; }
 

@@ -242,34 +242,8 @@ __global__ __launch_bounds__(T::kThreads, 2) void sgemm_flex(hk::SgemmFlexCall g
     for (int i = 0; i < kBlkM; ++i)
 #pragma unroll
       for (int j = 0; j < kBlkN; ++j) acc[i][j] += sum[a][i][j];
-  if constexpr (T::KG > 1) {  // the k groups' sums, added in group order
-    unsigned char HK_LDS* sums = lds + T::kGroupWaves * T::kStaging;
-    constexpr int kPerWave = kBlkM * kBlkN * 4;
-    auto at = [&](int grp, int b, int q) {
-      return reinterpret_cast<f32x4_t HK_LDS*>(
-          sums + (grp - 1) * T::kSums + ((wave * kPerWave + b * 4 + q) * 64 + lane) * 16);
-    };
-    if (group > 0) {
-#pragma unroll
-      for (int b = 0; b < kBlkM * kBlkN; ++b)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x16_t& v = acc[b / kBlkN][b % kBlkN];
-          *at(group, b, q) = f32x4_t{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-        }
-    }
-    __syncthreads();
-    if (group > 0) return;
-#pragma unroll
-    for (int grp = 1; grp < T::KG; ++grp)
-#pragma unroll
-      for (int b = 0; b < kBlkM * kBlkN; ++b)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4_t v = *at(grp, b, q);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[b / kBlkN][b % kBlkN][4 * q + e] += v[e];
-        }
+  if constexpr (T::KG > 1) {
+    if (merge_groups<T>(acc, lds, group, wave, lane)) return;
   }
   float* Cb = g.out.C + batch * g.out.sC;
   const int wrow0 = m0 + wm * T::kWaveM, wcol0 = n0 + wn * T::kWaveN;
