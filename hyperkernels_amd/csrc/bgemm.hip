@@ -911,6 +911,18 @@ using Plan = hk::GemmPlan;
 double wide_cost(bool ta, bool tb, int M, int N, int K, int batch, int splits, double split_cost) {
   if (splits > 1) return split_cost;
   const double kt = static_cast<double>(hk::ceil_div(K, BK));
+  if (N <= 128) {
+    // one column of 128-wide tiles: less per k-tile on a busy device and per further round (MI355X, us:
+    // 200 x 104 x 2176 in 200 batches 41, by auto_split_k's figures 54; 1216 x 112 x 24 in 400, 41 and 77)
+    const int64_t cus = hk::device_cu_count(), items = hk::ceil_div(M, BM) * batch;
+    auto t_kt = [&](int64_t busy) {
+      const double x = (static_cast<double>(busy) / static_cast<double>(cus) - 0.39) / 0.61;
+      return 0.79 + 0.25 * (x < 0.0 ? 0.0 : x);
+    };
+    const int64_t full = items / cus, last = items % cus;
+    return 8.0 + 4.0 * static_cast<double>(full + (last > 0) - 1) +
+           kt * (static_cast<double>(full) * t_kt(cus) + (last > 0 ? t_kt(last) : 0.0));
+  }
   if (w160_plan(ta, tb, M, N, K, batch, 1)) return 8.0 + 0.99 * kt;
   if (row_tile(ta, M, N, batch, 1) == 192) return 8.0 + (split_cost - 8.0) * 0.85;
   return split_cost;

@@ -40,6 +40,7 @@ struct Args {
   uint16_t* C;
   int64_t ldc, sC;
   int split_k, k_per_split;
+  bool by_matrix;  // matrix_order
   float* part;     // not NULL: fp32 partials [split][batch][M][part_pitch(N)] instead of C
   hk::F32Out fo;   // fo.C not NULL: fp32 C through its own epilogue instead
 };
@@ -88,11 +89,12 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads >= 512 ? 1 : 2) void bgemm
   unsigned char HK_LDS* lds = (unsigned char HK_LDS*)lds_raw;
 
   const int M = g.M, N = g.N;
-  const int batch = blockIdx.z / g.split_k;
-  const int split = blockIdx.z - batch * g.split_k;
   const int tiles_m = (M + T::BMT - 1) / T::BMT, tiles_n = (N + T::BNT - 1) / T::BNT;
-  int tm, tn;
-  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  int tile = blockIdx.x, z = blockIdx.z, tm, tn;
+  if (g.by_matrix) matrix_order(gridDim.x, gridDim.z, tile, z);
+  const int batch = z / g.split_k;
+  const int split = z - batch * g.split_k;
+  tile_coords(tile, tiles_m, tiles_n, tm, tn, g.by_matrix);
   const int m0 = tm * T::BMT, n0 = tn * T::BNT;
   const int kbeg = split * g.k_per_split;
   const int kend = min(g.K, kbeg + g.k_per_split);
@@ -337,9 +339,11 @@ hipError_t launch(const Args& g, int batch, hipStream_t stream) {
   HK_RETURN_IF_ERROR(attr_status);
   const int64_t tiles = hk::ceil_div(g.M, T::BMT) * hk::ceil_div(g.N, T::BNT);
   HK_CHECK_ARG(tiles <= INT32_MAX && static_cast<int64_t>(batch) * g.split_k <= 65535);
+  Args a = g;
+  a.by_matrix = batch > 1 && tiles * batch * g.split_k <= INT32_MAX;
   hipLaunchKernelGGL((bgemm_flex<T, AK, BKM, RAGGED>),
                      dim3(static_cast<unsigned>(tiles), 1, batch * g.split_k), dim3(T::kThreads),
-                     kLds, stream, g);
+                     kLds, stream, a);
   return hk::launch_status();
 }
 

@@ -123,6 +123,30 @@ def test_bgemm_flex_batches_and_split(hk, orc, ta, tb):
                C0, ta, tb, 1.0, 0.5)
 
 
+# several matrices in a launch: tiles x batches (x splits) that are and are no multiple of the 8 XCDs
+@pytest.mark.parametrize("batch,M,N,K,split", [(13, 136, 72, 96, 0), (5, 304, 200, 72, 0), (16, 64, 64, 128, 0),
+                                               (7, 67, 131, 45, 0), (9, 130, 67, 403, 3),
+                                               (2, 1000, 24, 40, 0), (257, 8, 16, 24, 0)])
+@pytest.mark.parametrize("ta,tb", LAYOUTS[:3])
+def test_bgemm_flex_matrices_in_a_launch(hk, batch, M, N, K, split, ta, tb):
+    say("bgemm flex matrices", batch, M, N, K, split, ta, tb)
+    assert hk.lib().hk_bgemm_small_tile(ta, tb, M, N, K, batch, split) > 0
+    g = torch.Generator(device=DEV)
+    g.manual_seed(M + N + K)
+    rand = lambda r, c: torch.randn(batch, r, c, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
+    a, b = rand(*((K, M) if ta else (M, K))), rand(*((N, K) if tb else (K, N)))
+    c = torch.full((batch, M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    tail = (M, N, K, bits(1.0), a.data_ptr(), a.shape[2], M * K, b.data_ptr(), b.shape[2], N * K, 0,
+            c.data_ptr(), N, M * N, batch, torch.cuda.current_stream().cuda_stream)
+    lay = {(0, 1): 0, (1, 0): 1, (0, 0): 2}[(ta, tb)]
+    rc = hk.lib().hk_bgemm_core(lay, split, *tail) if split else hk.lib().hk_bgemm(ta, tb, *tail)
+    assert rc == 0
+    A = (a.transpose(1, 2) if ta else a).float().contiguous()
+    B = (b.transpose(1, 2) if tb else b).float().contiguous()
+    ref = torch.stack([torch.mm(A[i], B[i]) for i in range(batch)])
+    assert (c.float() - ref).abs().max() <= 1e-2 * ref.abs().max()
+
+
 @pytest.mark.parametrize("batch,K,split,odd_c", [(40000, 130, 2, False), (40000, 136, 2, True),
                                                  (65535, 65, 2, False), (65536, 72, 1, True),
                                                  (65537, 9, 1, False)])
