@@ -950,21 +950,26 @@ size_t partial_bytes(int used, int M, int N, int batch) {
 }
 
 // The better of the two families where partials may take `held` bytes at most: the small and
-// any-alignment tiles with one k split, the 256-wide ones with their own splits or with one.
+// any-alignment tiles with one k split, the 256-wide ones with as many of their splits as fit.
 Plan lean_plan(bool ta, bool tb, int M, int N, int K, int batch, Rows rows, size_t held) {
   const bool ragged = rows == Rows::kRagged;
   const hk::FlexPlan f = hk::bgemm_flex_plan(M, N, K, batch, 1, ragged);
   if (!ragged) {
-    Plan wide{0, 1, K};
+    const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    const size_t fit = held / partial_bytes(1, M, N, batch);
+    const int most = fit < 2 ? 1 : fit < kMostSplits ? static_cast<int>(fit) : kMostSplits;
     double cost = 0.0;
-    hk::bgemm_split_plan(M, N, K, batch, 0, &wide.used, &wide.kps, &cost);
-    if (wide.used > 1 && partial_bytes(wide.used, M, N, batch) > held) {
-      const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-      wide = Plan{0, 1, K};
-      auto_split_k(tiles * batch, hk::ceil_div(K, BK), static_cast<int64_t>(M) * N * batch, 1,
-                   &cost);
+    const int s = auto_split_k(tiles * batch, hk::ceil_div(K, BK),
+                               static_cast<int64_t>(M) * N * batch, most, &cost);
+    Plan wide{0, 1, K};
+    if (s > 1) {
+      wide.kps = static_cast<int>(hk::ceil_div(hk::ceil_div(K, s), BK) * BK);
+      wide.used = static_cast<int>(hk::ceil_div(K, wide.kps));
     }
-    if (f.cost > 0.95 * wide_cost(ta, tb, M, N, K, batch, wide.used, cost)) return wide;
+    // one chain over a deep k runs up to 1.6 times the modelled time (176 x 312 x 6152 TN, unaligned to
+    // cache lines: 37 us for 23), so splits are given up for it only where it looks far better
+    const double margin = wide.used > 1 ? 0.65 : 0.95;
+    if (f.cost > margin * wide_cost(ta, tb, M, N, K, batch, wide.used, cost)) return wide;
   }
   return Plan{f.tile, 1, K};
 }
@@ -1030,8 +1035,13 @@ hipError_t bgemm_run(int transA, int transB, int M, int N, int K, hk_bf16 alpha_
   HK_CHECK_ARG(2 * tiles <= INT32_MAX && static_cast<int64_t>(batchCount) * plan.used <= kMaxGridZ);
   void* ws = nullptr;
   if (plan.used > 1) {
-    const hipError_t e =
-        hk::device_workspace(partial_bytes(plan.used, M, N, batchCount), stream, &ws);
+    // room for the 256-wide tiles' splits, too, which a captured call of the shape falls back on
+    int room = plan.used, wide = 1, kps = K;
+    if (plan.flex && !ep.ragged) {
+      hk::bgemm_split_plan(M, N, K, batchCount, 0, &wide, &kps);
+      if (wide > room) room = wide;
+    }
+    const hipError_t e = hk::device_workspace(partial_bytes(room, M, N, batchCount), stream, &ws);
     if (e == hipErrorOutOfMemory && optional) {
       (void)hipGetLastError();
       plan = lean_plan(ta, tb, M, N, K, batchCount, rows, 0);

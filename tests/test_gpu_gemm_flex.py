@@ -188,10 +188,11 @@ def test_bgemm_unaligned_rows_need_no_workspace_under_capture(hk, orc, M, N, K, 
         _check(orc, to_host_bits(dC), A, B, C0, 0, 1, 1.0, 0.0)
 
 
-def test_bgemm_deep_k_keeps_the_wide_splits_under_capture(hk, orc):
-    # one aligned 256 x 256 tile over a deep k: eager calls split it over small tiles; a captured one
-    # takes the 256-wide tiles' splits (bit for bit those of an explicit split), not one chain
-    M, N, K = 256, 256, 65536
+@pytest.mark.parametrize("M,N,K,splits", [(256, 256, 65536, 8), (176, 312, 6152, 8)])
+def test_bgemm_deep_k_keeps_the_wide_splits_under_capture(hk, orc, M, N, K, splits):
+    # few aligned tiles over a deep k: eager calls split it over small tiles and leave a workspace in which
+    # a captured one takes the 256-wide tiles' splits (bit for bit those of an explicit split), not one
+    # chain
     lib = hk.lib()
     assert lib.hk_bgemm_small_tile(0, 0, M, N, K, 1, 0) > 0
     assert lib.hk_bgemm_split_count(0, 0, M, N, K, 1, 0) > 1
@@ -211,7 +212,7 @@ def test_bgemm_deep_k_keeps_the_wide_splits_under_capture(hk, orc):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
         call(torch.cuda.current_stream().cuda_stream)
-    call(torch.cuda.current_stream().cuda_stream, 8)
+    call(torch.cuda.current_stream().cuda_stream, splits)
     wide = to_host_bits(dC)
     for _ in range(3):
         dC.zero_()
