@@ -181,14 +181,14 @@ struct QPlanes {
   const float* d;
 };
 
-// How the (key tile, query tile) pairs of a head are dealt to workgroups. A workgroup owns a key tile
-// and at most `chunk` of its query tiles; a key tile of several workgroups has its dK / dV summed
-// from partials ([item][b, h][dK, dV][128 keys][64], fp32) in item order by attn_bwd_sum. A head's
-// items are numbered key tile by key tile.
-struct Deal {
-  int chunk;    // query tiles per workgroup
+// How the (key tile, query tile) pairs of a head are dealt to workgroups (Deal): a workgroup owns a key
+// tile and at most `chunk` of its query tiles; a key tile of several workgroups has its dK / dV summed
+// from partials ([item][b, h][dK, dV][128 keys][64], fp32) in item order by attn_bwd_sum.
+struct Shares {
+  Deal deal;
   float* part;  // NULL when every key tile has one workgroup
 };
+
 // Vector memory operations each lane issues after a tile's copies: the dQ atomics. A wave
 // waits with vmcnt(kAtomicsPerTile) for its copies of the next tile (vector memory operations
 // complete in issue order), so the atomics themselves are never waited for.
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void attn_bwd_prepare(hk_attn_bwd_params p, ch
 // share a key tile (deal.part). Both off, the loop tests nothing per tile.
 template <bool RAGGED, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_params p, int nbh,
-                                                                QPlanes qp, Deal deal) {
+                                                                QPlanes qp, Shares sh) {
   extern __shared__ __attribute__((aligned(16))) char lds_generic[];
   char HK_LDS* lds = (char HK_LDS*)lds_generic;
   char HK_LDS* sKh = lds + kOffKh;
@@ -263,10 +263,9 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   const int bh = static_cast<int>(blockIdx.x) - item * nbh;
   int kt = item, piece = 0, pieces = 1;
   if (SPLIT) {
-    const int nkt = static_cast<int>((T + kBKV - 1) / kBKV);
-    kt = item_key_tile(T, p.is_causal, nkt, item, deal.chunk);
-    piece = item - first_item(T, p.is_causal, nkt, kt, deal.chunk);
-    pieces = key_items(T, p.is_causal, kt, deal.chunk);
+    kt = sh.deal.key_tile(item);
+    piece = item - sh.deal.first_item(kt);
+    pieces = sh.deal.key_items(kt);
   }
   const int b = bh / p.nh, h = bh - b * p.nh;
   const int64_t k0 = static_cast<int64_t>(kt) * kBKV;
@@ -619,7 +618,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
   }
   __syncthreads();
   if (SPLIT && qh == 0 && pieces > 1) {
-    float* dkp = deal.part + (static_cast<int64_t>(item) * nbh + bh) * (2 * kBKV * kHD) +
+    float* dkp = sh.part + (static_cast<int64_t>(item) * nbh + bh) * (2 * kBKV * kHD) +
                  (32 * kg + 4 * hh) * kHD + c;
     float* dvp = dkp + kBKV * kHD;
 #pragma unroll
@@ -657,11 +656,11 @@ __global__ __launch_bounds__(kThreads, 1) void attn_bwd_kernel(hk_attn_bwd_param
 constexpr int kSumThreads = 256;
 constexpr int kSumBlocks = 2 * kBKV * kHD / 4 / kSumThreads;
 __global__ __launch_bounds__(kSumThreads) void attn_bwd_sum(hk_attn_bwd_params p, int nbh,
-                                                            Deal deal) {
+                                                            Shares sh) {
   const int kt = blockIdx.x / kSumBlocks, bh = blockIdx.y;
-  const int pieces = key_items(p.T, p.is_causal, kt, deal.chunk);
+  const int pieces = sh.deal.key_items(kt);
   if (pieces == 1) return;
-  const int item = first_item(p.T, p.is_causal, static_cast<int>((p.T + kBKV - 1) / kBKV), kt, deal.chunk);
+  const int item = sh.deal.first_item(kt);
   const int idx = (blockIdx.x % kSumBlocks) * kSumThreads + threadIdx.x;
   const bool is_dv = idx >= kBKV * kHD / 4;
   const int i = idx - (is_dv ? kBKV * kHD / 4 : 0);
@@ -670,7 +669,7 @@ __global__ __launch_bounds__(kSumThreads) void attn_bwd_sum(hk_attn_bwd_params p
   const int b = bh / p.nh, h = bh - b * p.nh;
   const int64_t step = static_cast<int64_t>(nbh) * (2 * kBKV * kHD);
   const float* s =
-      deal.part + (static_cast<int64_t>(item) * nbh + bh) * (2 * kBKV * kHD) + 4 * idx;
+      sh.part + (static_cast<int64_t>(item) * nbh + bh) * (2 * kBKV * kHD) + 4 * idx;
   f32x4_t v = *reinterpret_cast<const f32x4_t*>(s);
   for (int j = 1; j < pieces; ++j) v += *reinterpret_cast<const f32x4_t*>(s + j * step);
   const float scale = is_dv ? 1.0f : p.scale;
@@ -721,10 +720,9 @@ hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool ze
   const int64_t rows = bh * p.T;
   const size_t plane = static_cast<size_t>(rows) * kRowBytes;
   const size_t planes = (4 * plane + 2 * static_cast<size_t>(rows) * 4 + 255) & ~size_t{255};
-  Deal deal{pick_chunk(p.T, p.is_causal, static_cast<int>(nkt), bh, hk::device_cu_count()), nullptr};
-  int64_t items = nkt;
-  if (deal.chunk < query_tiles(p.T, p.is_causal, 0))
-    items = first_item(p.T, p.is_causal, static_cast<int>(nkt), static_cast<int>(nkt), deal.chunk);
+  const int T = static_cast<int>(p.T);
+  Shares sh{make_deal(T, p.is_causal, pick_chunk(T, p.is_causal, bh, hk::device_cu_count())), nullptr};
+  int64_t items = sh.deal.items;
   bool split = items > nkt;
   const size_t part_bytes =
       split ? static_cast<size_t>(items * bh) * 2 * kBKV * kHD * sizeof(float) : 0;
@@ -743,7 +741,6 @@ hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool ze
     HK_RETURN_IF_ERROR(hk::device_workspace(planes, stream, &ws));
     split = false;
     items = nkt;
-    deal.chunk = query_tiles(p.T, p.is_causal, 0);
   }
   char* wsb = static_cast<char*>(ws);
   float* l2 = reinterpret_cast<float*>(wsb + 4 * plane);
@@ -754,17 +751,17 @@ hipError_t attn_backward(const hk_attn_bwd_params* params, int head_dim, bool ze
                      l2 + rows, zero_dq);
   HK_RETURN_IF_ERROR(hk::launch_status());
   const QPlanes qp{wsb, wsb + plane, wsb + 2 * plane, wsb + 3 * plane, l2, l2 + rows};
-  if (split) deal.part = reinterpret_cast<float*>(wsb + planes);
+  if (split) sh.part = reinterpret_cast<float*>(wsb + planes);
   const bool ragged = p.T % kBQ != 0;
   auto* kernel = split ? (ragged ? attn_bwd_kernel<true, true> : attn_bwd_kernel<false, true>)
                        : (ragged ? attn_bwd_kernel<true, false> : attn_bwd_kernel<false, false>);
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(items * bh)), dim3(kThreads), kLdsBytes,
-                     stream, p, static_cast<int>(bh), qp, deal);
+                     stream, p, static_cast<int>(bh), qp, sh);
   HK_RETURN_IF_ERROR(hk::launch_status());
   if (!split) return hipSuccess;
   hipLaunchKernelGGL(attn_bwd_sum,
                      dim3(static_cast<unsigned>(nkt * kSumBlocks), static_cast<unsigned>(bh)),
-                     dim3(kSumThreads), 0, stream, p, static_cast<int>(bh), deal);
+                     dim3(kSumThreads), 0, stream, p, static_cast<int>(bh), sh);
   return hk::launch_status();
 }
 

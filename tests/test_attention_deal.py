@@ -12,7 +12,7 @@ DRIVER = r"""
 #include "attention_deal.h"
 using namespace hk::attn;
 
-static int pick_by_walk(int64_t T, bool causal, int nkt, int64_t nbh, int cus) {
+static int pick_by_walk(int T, bool causal, int nkt, int64_t nbh, int cus) {
   const int most = query_tiles(T, causal, 0);
   if (nkt * nbh >= int64_t{4} * cus) return most;
   double best = 0.0;
@@ -20,7 +20,7 @@ static int pick_by_walk(int64_t T, bool causal, int nkt, int64_t nbh, int cus) {
   for (int chunk = most; chunk >= 1; --chunk) {
     int64_t wgs = 0, tiles = 0;
     for (int kt = 0; kt < nkt; ++kt) {
-      wgs += key_items(T, causal, kt, chunk);
+      wgs += (query_tiles(T, causal, kt) + chunk - 1) / chunk;
       tiles += query_tiles(T, causal, kt);
     }
     if (wgs * nbh > int64_t{8} * cus) break;
@@ -34,25 +34,26 @@ static int pick_by_walk(int64_t T, bool causal, int nkt, int64_t nbh, int cus) {
 }
 
 int main() {
-  for (int64_t T : {1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 333, 520, 1000, 1024, 1025, 2031, 4097,
-                    8192, 16383, 65536})
+  for (int T : {1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 333, 520, 1000, 1024, 1025, 2031, 4097, 8192,
+                16383, 65536, 130000})
     for (int causal = 0; causal < 2; ++causal) {
-      const int nkt = static_cast<int>((T + kBKV - 1) / kBKV), most = query_tiles(T, causal, 0);
+      const int nkt = (T + kBKV - 1) / kBKV, most = query_tiles(T, causal, 0);
       for (int chunk = 1; chunk <= most; chunk += most > 600 && chunk > 40 ? 37 : 1) {
+        const Deal d = make_deal(T, causal, chunk);
         int sum = 0;
-        for (int kt = 0; kt <= nkt; ++kt) {
-          if (first_item(T, causal, nkt, kt, chunk) != sum) return printf("first item\n"), 1;
-          if (kt == nkt) break;
-          const int n = key_items(T, causal, kt, chunk);
+        for (int kt = 0; kt < nkt; ++kt) {
+          const int n = (query_tiles(T, causal, kt) + chunk - 1) / chunk;
+          if (d.key_items(kt) != n || d.first_item(kt) != sum) return printf("items\n"), 1;
           for (int i : {sum, sum + n / 2, sum + n - 1})
-            if (item_key_tile(T, causal, nkt, i, chunk) != kt) return printf("key tile\n"), 1;
+            if (d.key_tile(i) != kt) return printf("key tile\n"), 1;
           sum += n;
         }
+        if (d.items != sum || d.nkt != nkt) return printf("all items\n"), 1;
       }
       for (int nbh : {1, 2, 4, 12, 24, 96, 400})
         for (int cus : {64, 256})
-          if (pick_chunk(T, causal, nkt, nbh, cus) != pick_by_walk(T, causal, nkt, nbh, cus))
-            return printf("pick T %d causal %d heads %d\n", int(T), causal, nbh), 1;
+          if (pick_chunk(T, causal, nbh, cus) != pick_by_walk(T, causal, nkt, nbh, cus))
+            return printf("pick T %d causal %d heads %d\n", T, causal, nbh), 1;
     }
   printf("ok\n");
   return 0;
